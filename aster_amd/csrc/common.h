@@ -118,15 +118,18 @@ __device__ __forceinline__ float strided_max(float x) {
   return x;
 }
 
-__device__ __forceinline__ float wave_max(float x) {
+// Maximum over aligned groups of N consecutive lanes (N in 8,16,32,64), in every lane.
+template <int N>
+__device__ __forceinline__ float group_max(float x) {
   x = fmaxf(x, dpp<kDppXor1>(x));
   x = fmaxf(x, dpp<kDppXor2>(x));
   x = fmaxf(x, dpp<kDppHalfMirror>(x));
-  x = fmaxf(x, dpp<kDppMirror>(x));
-  x = fmaxf(x, shfl_xor(x, 16));
-  x = fmaxf(x, shfl_xor(x, 32));
+  if constexpr (N >= 16) x = fmaxf(x, dpp<kDppMirror>(x));
+  if constexpr (N >= 32) x = fmaxf(x, shfl_xor(x, 16));
+  if constexpr (N >= 64) x = fmaxf(x, shfl_xor(x, 32));
   return x;
 }
+__device__ __forceinline__ float wave_max(float x) { return group_max<kWave>(x); }
 
 // Sum over the 64 lanes (every lane gets it): after the xor-1/xor-2 butterflies a
 // lane holds its quad's sum, and each mirror step adds the mirrored (disjoint)
@@ -152,28 +155,15 @@ __device__ __forceinline__ constexpr float format_max() {
   return KF == kInt8 ? 127.f : KF == kE4M3 ? 448.f : 57344.f;
 }
 
-// Finite c with |c| <= format_max -> FP8 bits, round to nearest even. With M mantissa
-// bits and exponent bias B: below the smallest normal 2^(1-B) the value counts
-// subnormal steps of 2^(1-B-M), rint(|c| * 2^(B-1+M)) in 0..2^M (scaling by a power of
-// two is exact; 2^M is the smallest normal's code); above it the fp32 mantissa is
-// rounded to M bits at bit 23-M (half to even, a carry steps the exponent) and the
-// exponent rebiased from 127 to B. The sign is kept (-0 for a negative underflow).
+// Finite c with |c| <= format_max -> FP8 bits, round to nearest even with subnormals and
+// the sign of zero kept: the OCP conversions of gfx950, equal to the float32 -> float8
+// conversion for every such float.
 template <int KF>
-__device__ __forceinline__ uint8_t fp8_round(float c) {
-  constexpr int M = KF == kE4M3 ? 3 : 2;
-  constexpr int B = KF == kE4M3 ? 7 : 15;
-  const uint32_t bits = __builtin_bit_cast(uint32_t, c);
-  const uint32_t sign = (bits >> 24) & 0x80u;
-  const uint32_t mag = bits & 0x7fffffffu;
-  uint32_t code;
-  if (mag < ((uint32_t)(128 - B) << 23)) {
-    code = (uint32_t)__builtin_rintf(__builtin_bit_cast(float, mag) * (float)(1 << (B - 1 + M)));
-  } else {
-    const uint32_t r = mag + ((1u << (22 - M)) - 1u) + ((mag >> (23 - M)) & 1u);
-    code = (r >> (23 - M)) - ((uint32_t)(127 - B) << M);
-  }
-  return (uint8_t)(code | sign);
+__device__ __forceinline__ uint32_t fp8_pair(float lo, float hi) {
+  if constexpr (KF == kE4M3) return __builtin_amdgcn_cvt_pk_fp8_f32(lo, hi, 0, false);
+  else return __builtin_amdgcn_cvt_pk_bf8_f32(lo, hi, 0, false);
 }
+
 // The row's scale from its largest magnitude (kv_quantization.py:86-90): true
 // division, then the FLT_MIN clamp; an all-zero row gets scale 1.
 template <int KF>
@@ -188,7 +178,37 @@ __device__ __forceinline__ int8_t quant_code(float x, float scale) {
   constexpr float kMax = format_max<KF>();
   const float n = fminf(fmaxf(x / scale, -kMax), kMax);
   if constexpr (KF == kInt8) return (int8_t)__builtin_rintf(n);
-  else return (int8_t)fp8_round<KF>(n);
+  else return (int8_t)fp8_pair<KF>(n, 0.f);
+}
+
+// x / scale clamped to the format's range, correctly rounded as the division, from inv =
+// 1 / scale (correctly rounded): the product's residual, exact in one fma, corrects it
+// (Markstein's division step). Equal to the division for every 16-bit x and row maximum,
+// and for 4e8 float32 pairs drawn around the codes' ties, where scale >= kMinFastScale
+// keeps the residual of every quotient that can round to a code above the denormals.
+constexpr float kMinFastScale = 0x1p-64f;
+template <int KF>
+__device__ __forceinline__ float quant_unit(float x, float scale, float inv) {
+  constexpr float kMax = format_max<KF>();
+  const float q = x * inv;
+  float n = __builtin_fmaf(__builtin_fmaf(-q, scale, x), inv, q);
+  if constexpr (KF != kInt8) n = __builtin_copysignf(n, x);  // x = -0 gives +0 above
+  return fminf(fmaxf(n, -kMax), kMax);
+}
+
+// Four quotients of quant_unit as a word of codes. int8: adding 1.5 2^23 rounds half to
+// even and leaves the integer in the low byte.
+template <int KF>
+__device__ __forceinline__ uint32_t quant_pack(const float (&n)[4]) {
+  if constexpr (KF == kInt8) {
+    uint32_t b[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) b[i] = __builtin_bit_cast(uint32_t, n[i] + 12582912.f);
+    return __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u) |
+           __builtin_amdgcn_perm(b[3], b[2], 0x04000c0cu);
+  } else {
+    return (fp8_pair<KF>(n[0], n[1]) & 0xffffu) | fp8_pair<KF>(n[2], n[3]) << 16;
+  }
 }
 
 // The f16 conversions below give a code's value times 2^-8 for E4M3FN (its bits
