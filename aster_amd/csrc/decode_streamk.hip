@@ -68,6 +68,12 @@ constexpr int kMaxPackSeqsSK = 256;
 constexpr int kMaxPacksSK = 128;
 constexpr int kMaxRowsSK = kMaxSeqsSK + 1;  // block prefix entries over work rows (+ 1)
 constexpr int kFastPieces = 16;   // merge: sequences in at most this many pieces load at once
+// Waves that merge a row where the rows average kWideMergePieces pieces or more; below, one
+// round of one wave holds a row. Rows of 100 to 4096 tokens, head dim 128, one wave against
+// eight: 8 rows x 8 kv heads (32 pieces a row) 26.1 -> 20.1 us a call, 16 x 8 (16 pieces)
+// 26.3 -> 24.3, 16 x 4 27.5 -> 21.5, 32 x 4 27.5 -> 25.6.
+constexpr int kMergeWaves = 8;
+constexpr int kWideMergePieces = 16;
 
 
 // Work rows of one kv head: packs 0 .. npk-1, then sequence s as row npk + s.
@@ -752,8 +758,14 @@ constexpr int merge_heads() { return G < 4 ? G : 4; }
 // round of R = min(64 / GS, kFast) pieces, lane u GS + h holds (m, l) of piece u, head
 // h0 + h, and the maxima and weight sums reduce over the lanes of one head. The
 // merge_softmax rule (online_attention.py:42-63) and SoftmaxState.output (:35-39).
-template <typename QT, int D, int G, int GS>
-__global__ __launch_bounds__(kWave) void merge_streamk_kernel(AttnArgs a) {
+//
+// Bound by the chain of round trips: a round of R pieces costs two (statistics, rows).
+// With NW > 1, a workgroup takes the row: wave w merges rounds w, w + NW, ..., and the
+// waves' states combine through LDS. One row of 8192 tokens, cut over 256 waves, is 16
+// rounds for one wave (36.5 us, three times the streaming) and 2 for each of 8; the call goes
+// 47.6 -> 21.3 us (8 kv heads x 4 query heads, head dim 128).
+template <typename QT, int D, int G, int GS, int NW>
+__global__ __launch_bounds__(NW * kWave) void merge_streamk_kernel(AttnArgs a) {
   constexpr int E = GS * D / kWave;  // floats per lane
   static_assert(G % GS == 0 && E >= 1 && GS * D % kWave == 0, "lanes cover the heads' rows");
   constexpr int HS = G / GS;  // waves per (sequence, kv head)
@@ -762,7 +774,8 @@ __global__ __launch_bounds__(kWave) void merge_streamk_kernel(AttnArgs a) {
   constexpr int R0 = kWave / GS < kFastPieces ? kWave / GS : kFastPieces;
   constexpr int R = R0 < kRegs ? R0 : kRegs;  // pieces per round
   typedef float vec_t __attribute__((ext_vector_type(V)));
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x % kWave;
+  const int wave = NW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) : 0;
   const int hkv = a.cache.num_kv_heads;
   const int seq = blockIdx.x / (hkv * HS), kvh = blockIdx.x / HS % hkv;
   const int h0 = blockIdx.x % HS * GS;  // first head of the group this wave takes
@@ -819,8 +832,9 @@ __global__ __launch_bounds__(kWave) void merge_streamk_kernel(AttnArgs a) {
     lp = live ? a.ws_ml[(sl + h0 + sh) * 2 + 1] : 0.f;
   };
   float M = -INFINITY;  // of head sh (lane-parallel layout)
-  if (pieces > R) {     // several rounds: the maxima first
-    for (int p0 = 0; p0 < pieces; p0 += R) {
+  const bool rounds = pieces > NW * R;
+  if (rounds) {  // several rounds: the maxima first
+    for (int p0 = wave * R; p0 < pieces; p0 += NW * R) {
       int64_t sl;
       float mp, lp;
       stats(p0, sl, mp, lp);
@@ -830,7 +844,7 @@ __global__ __launch_bounds__(kWave) void merge_streamk_kernel(AttnArgs a) {
   float L = 0.f, O[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) O[e] = 0.f;
-  for (int p0 = 0; p0 < pieces; p0 += R) {
+  for (int p0 = wave * R; p0 < pieces; p0 += NW * R) {
     int64_t sl;
     float mp, lp;
     stats(p0, sl, mp, lp);
@@ -848,7 +862,8 @@ __global__ __launch_bounds__(kWave) void merge_streamk_kernel(AttnArgs a) {
         for (int c = 0; c < V; ++c) v[u][e + c] = x[c];
       }
     }
-    const float mx = pieces > R ? M : head_max(mp);
+    if (!rounds) M = head_max(mp);
+    const float mx = M;
     const float w = mp == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mp - mx);
     L += head_sum(lp * w);
 #pragma unroll
@@ -858,7 +873,45 @@ __global__ __launch_bounds__(kWave) void merge_streamk_kernel(AttnArgs a) {
       for (int e = 0; e < E; ++e) O[e] = fmaf(v[u][e], wu, O[e]);
     }
   }
-  const float inv_l = 1.f / fmaxf(__shfl(L, hl, kWave), FLT_MIN);
+  if constexpr (NW > 1) {
+    // the waves' states (M, L of head sh in lane sh, O in units of 2^M), combined by wave 0
+    // (a wave without pieces holds M = -inf and weighs 0)
+    __shared__ float s_m[NW][GS], s_l[NW][GS];
+    __shared__ __attribute__((aligned(16))) float s_o[NW][E * kWave];
+    if (lane < GS) {
+      s_m[wave][lane] = M;
+      s_l[wave][lane] = L;
+    }
+#pragma unroll
+    for (int e = 0; e < E; e += V) {
+      vec_t x;
+#pragma unroll
+      for (int c = 0; c < V; ++c) x[c] = O[e + c];
+      *reinterpret_cast<vec_t*>(&s_o[wave][(e / V * kWave + lane) * V]) = x;
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) mx = fmaxf(mx, s_m[w][hl]);
+    float l = 0.f;
+#pragma unroll
+    for (int e = 0; e < E; ++e) O[e] = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float mw = s_m[w][hl];
+      const float ww = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - mx);
+      l += s_l[w][hl] * ww;
+#pragma unroll
+      for (int e = 0; e < E; e += V) {
+        const vec_t x = *reinterpret_cast<const vec_t*>(&s_o[w][(e / V * kWave + lane) * V]);
+#pragma unroll
+        for (int c = 0; c < V; ++c) O[e + c] = fmaf(x[c], ww, O[e + c]);
+      }
+    }
+    L = l;
+  }
+  const float inv_l = 1.f / fmaxf(NW > 1 ? L : __shfl(L, hl, kWave), FLT_MIN);
   QT* out = static_cast<QT*>(a.out) + (int64_t)decode_token(a, seq) * a.o_tok +
             (int64_t)(kvh * G + h0 + hl) * a.o_head + lane * E % D;
   QT r[E];
@@ -912,8 +965,12 @@ int launch(AttnArgs a, hipStream_t stream) {
   const int wgs = (int)(waves / NW);
   hipLaunchKernelGGL(kernel, dim3(wgs), dim3(NW * kWave), 0, stream, a);
   constexpr int GS = merge_heads<G>();
-  hipLaunchKernelGGL((merge_streamk_kernel<QT, D, G, GS>),
-                     dim3(a.num_seqs * a.cache.num_kv_heads * (G / GS)), dim3(kWave), 0, stream, a);
+  const dim3 grid(a.num_seqs * a.cache.num_kv_heads * (G / GS));
+  if (a.num_seqs * a.cache.num_kv_heads * kWideMergePieces <= a.pref_waves)
+    hipLaunchKernelGGL((merge_streamk_kernel<QT, D, G, GS, kMergeWaves>), grid,
+                       dim3(kMergeWaves * kWave), 0, stream, a);
+  else
+    hipLaunchKernelGGL((merge_streamk_kernel<QT, D, G, GS, 1>), grid, dim3(kWave), 0, stream, a);
   const hipError_t err = hipGetLastError();
   return err == hipSuccess ? 0 : hip_fail(err, "paged_attention (stream-K) launch");
 }
