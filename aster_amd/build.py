@@ -79,8 +79,12 @@ def hipcc():
 # MFMA accumulators live in VGPRs (-amdgpu-mfma-vgpr-form), so AGPRs only appear as
 # spill space beyond 256 VGPRs, and they cost occupancy (a kernel that needed 217
 # registers ran at 313 and one wave per SIMD after a change that went unnoticed).
-# The exact fp32 VALU decode kernels (fp32 queries) are known to spill this way.
-AGPR_SPILL_ALLOWED = ("decode_valu_kernel",)
+# The exact fp32 VALU decode kernels (fp32 queries) are known to spill this way. The
+# prefill kernels at head dim 256 run one wave per SIMD by design (their operand buffers
+# fill the LDS), so the second half of the register file is theirs.
+AGPR_SPILL_ALLOWED = ("decode_valu_kernel", "prefill_mfma_kernelIfLi256", "prefill_mfma_kernelIDF16_Li256",
+                      "prefill_mfma_kernelINS_6bf16_tELi256", "prefix_tiles_kernelIfLi256",
+                      "prefix_tiles_kernelIDF16_Li256", "prefix_tiles_kernelINS_6bf16_tELi256")
 
 
 def _scratch_kernels(remarks):

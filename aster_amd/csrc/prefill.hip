@@ -25,6 +25,7 @@
 // to the 8 XCDs round robin) runs one contiguous range of units: the tiles
 // sharing a sequence's K/V then share that XCD's L2.
 #include <climits>
+#include <cstddef>
 #include <type_traits>
 
 #include "attention_common.h"
@@ -39,7 +40,6 @@ namespace {
 constexpr int KF = ASTR_KF;  // this translation unit's code format
 
 constexpr int kXcds = 8;
-constexpr int kPrefillBuffers = 3;
 
 // Per-wave timeline of the prefix-tile kernel (trace builds only, -DASTR_TRACE=1, built
 // apart from the product library by `python -m aster_amd.build --trace`): wall-clock
@@ -59,8 +59,9 @@ static __device__ int g_ttrace_info[kTileTraceWaves][4];
 
 template <int D>
 struct PrefillShape {
-  static constexpr int NT = D == 256 ? 1 : 2;     // 16-column MFMA tiles per wave
-  static constexpr int kCols = kWaves * 16 * NT;  // (token, head) columns per workgroup
+  static constexpr int NT = 1;                    // 32-column MFMA tiles per wave
+  static constexpr int kCols = kWaves * 32 * NT;  // (token, head) columns per workgroup
+  static constexpr int kOccupancy = D == 256 ? 1 : 2;  // workgroups per CU (LDS: 130 KB at 256)
 };
 
 // Keys visible to query tile `tile` (tokens [t0, t1) of the sequence's n query tokens,
@@ -200,511 +201,268 @@ __device__ int scan_tiles(const AttnArgs& a, int tq, int unit, int* s_wsum, int*
   return base;
 }
 
-// |S_int| <= 127 * kQRange * 256; a score factor below this keeps every score finite
-constexpr float kSafeFactor = 1.0e29f;
-// INT8 codes: the two-term query Q is within 1/2 of x = q * kQRange / max|q| per
-// element, so a key with scale ks carries at most 1/2 * 127 D * ks * cf of score error
-// (base 2; cf the column's score factor). A step in which any key scale times a
-// column's cf exceeds kFineScoreError / (63.5 D) adds the third term, K.lo2 / 128 (lo2 =
-// rint(128 (x - Q))), which divides that bound by 128. The worst case aligns every code
-// at 127 with every rounding; the typical error is ~50 times smaller (the rounding
-// errors are independent and codes average ~1/4 of 127), so steps without the term
-// carry ~2e-4 nats of score error at most, well inside what moves an output by the
-// north_star's 2e-3. Seeded N(0,1) queries and keys stay ~4x below the threshold.
-constexpr float kFineScoreError = 1.f / 64.f;
-// FP8 codes take the f16 QK path: |S| <= D * 2^15 * max|code as f16| (448 * 2^-8 for
-// E4M3FN, 57344 for E5M2) with D <= 256, times a factor below these stays finite.
-constexpr float kSafeFactorE4M3 = 1.0e31f;
-constexpr float kSafeFactorE5M2 = 5.0e26f;
-constexpr float safe_factor() {
-  return KF == kInt8 ? kSafeFactor : KF == kE4M3 ? kSafeFactorE4M3 : kSafeFactorE5M2;
+// |s| <= D 2^15 max|code as f16| for a column whose largest |q| is below 2^15; a key
+// factor below this keeps every score finite (max code 127; 448 2^-8 for E4M3FN; 57344).
+constexpr float safe_factor() { return KF == kInt8 ? 1.0e29f : KF == kE4M3 ? 1.0e31f : 5.0e26f; }
+
+typedef float float16v_t __attribute__((ext_vector_type(16)));
+
+// Maximum and sum over a lane and the one 32 away (v_permlane32_swap_b32: the pair of
+// results holds the low half's and the high half's value in every lane).
+__device__ __forceinline__ float max32(float x) {
+  const uint32_t b = __builtin_bit_cast(uint32_t, x);
+  const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+}
+__device__ __forceinline__ float sum32(float x) {
+  const uint32_t b = __builtin_bit_cast(uint32_t, x);
+  const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
 }
 
-// Query operands of one column tile: two int8 terms per 64-wide d chunk for int8 codes
-// (the int8 QK MFMA), f16 halves per 32-wide chunk for FP8 codes (the f16 QK MFMA).
-template <int D>
-struct QOpI8 {
-  int4_t hi[D / 64], lo[D / 64];
-};
-template <int D>
-struct QOpF16 {
-  half8_t op[D / 32];
-};
-template <int D>
-using QOp = typename std::conditional<KF == kInt8, QOpI8<D>, QOpF16<D>>::type;
+// The lane's index, from the lane mask: no register holds it through the key steps.
+__device__ __forceinline__ int lane_id() {
+  return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+}
 
-// f16 B-operands of one query column for the f16 QK MFMAs (the FP8 path): chunk
-// kk = 2h + sub holds d = 16 qg + 64 h + 8 sub + [0, 8), like the K operands. The
-// column is scaled by an exact power of two 2^-ex that keeps max|q| < 2^15 before
-// rounding to f16; returns qk_scale_log2 * 2^ex * code_scale (NaN for a non-finite
-// query, which makes every score of the column non-finite as in fp32 arithmetic).
-// Cross-lane: uniform control flow.
+// Query operands of one 32-column tile: B operands of the 16-wide d chunks (lane (c, h):
+// column c, d = 16 cc + 8 h + [0, 8)). A 16-bit query is exact in f16 and takes one term;
+// an fp32 query takes hi = f16(q) and lo = f16(q - hi), 22 bits.
 template <typename QT, int D>
-__device__ __forceinline__ float query_column_f16(const QueryColumn<QT, D>& raw, bool valid,
-                                                  float qk_scale_log2, half8_t (&qop)[D / 32]) {
-  constexpr int kVec = 16 / (int)sizeof(QT);
+struct QOp {
+  static constexpr int kTerms = sizeof(QT) == 4 ? 2 : 1;
+  // whether the registers hold key-step operands ahead of their use beside the query's (two
+  // terms at head dim 128 and 256 leave none)
+  static constexpr bool kAhead = !(kTerms == 2 && D >= 128);
+  half8_t op[kTerms][D / 16];
+};
+
+// The lane's elements of one query column as loaded.
+template <typename QT, int D>
+struct QueryTile {
+  static constexpr int kWords = 8 * (int)sizeof(QT) / 16;  // 16-byte words per chunk
+  uint4 w[D / 16][kWords];
+};
+template <typename QT, int D>
+__device__ __forceinline__ void load_query_tile(const QT* qp, QueryTile<QT, D>& raw) {
+#pragma unroll
+  for (int cc = 0; cc < D / 16; ++cc)
+#pragma unroll
+    for (int i = 0; i < QueryTile<QT, D>::kWords; ++i)
+      raw.w[cc][i] = reinterpret_cast<const uint4*>(qp + 16 * cc)[i];
+}
+
+// The column's f16 operands. A column whose largest |q| lies in [2^-10, 2^15) (fp32:
+// [2^-3, 2^15)) or is 0 enters as it is: f16 then holds a 16-bit element exactly down to
+// 2^-17, and its own step of 2^-24 is at most 2^-14 of the column's maximum anywhere
+// (fp32: both terms together 2^-21). Any other column is scaled by the exact 2^-ex that
+// brings its maximum into [2^14, 2^15); the return value 2^ex (1 when unscaled, NaN for a
+// non-finite column, which makes each of its scores non-finite as in fp32 arithmetic) goes
+// back onto its scores in the steps' edge path. Cross-lane: uniform control flow.
+template <typename QT, int D>
+__device__ __forceinline__ float query_operand(const QueryTile<QT, D>& raw, bool valid,
+                                               QOp<QT, D>& q) {
+  float x[D / 16][8];
   float mx = 0.f;
-  bool finite = true;
 #pragma unroll
-  for (int h = 0; h < D / 64; ++h)
-#pragma unroll
-    for (int c = 0; c < 16 / kVec; ++c) {
-      const QT* e = reinterpret_cast<const QT*>(&raw.w[h][c]);
-#pragma unroll
-      for (int i = 0; i < kVec; ++i) {
-        const float x = to_float<QT>(e[i]);
-        mx = fmaxf(mx, fabsf(x));
-        finite = finite && __builtin_isfinite(x);
-      }
-    }
-  mx = valid ? mx : 0.f;
-  mx = fmaxf(mx, shfl_xor(mx, 16));
-  mx = fmaxf(mx, shfl_xor(mx, 32));
-  const uint64_t nonfinite_lanes = __ballot(valid && !finite);
-  finite = ((nonfinite_lanes >> (threadIdx.x % 16)) & 0x0001000100010001ull) == 0;
-  int ex = 0;
-  if (finite && mx >= 32768.f) {
-    frexpf(mx, &ex);
-    ex -= 15;  // mx * 2^-ex < 2^15
-  }
-  const float down = ldexpf(1.f, -ex);
-#pragma unroll
-  for (int kk = 0; kk < D / 32; ++kk) {
-    const int h = kk / 2, sub = kk % 2;
+  for (int cc = 0; cc < D / 16; ++cc) {
+    const QT* e = reinterpret_cast<const QT*>(raw.w[cc]);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const int el = 8 * sub + i;  // element of the lane's 16 in chunk h
-      const QT* e = reinterpret_cast<const QT*>(&raw.w[h][el / kVec]);
-      qop[kk][i] = valid ? (_Float16)(to_float<QT>(e[el % kVec]) * down) : (_Float16)0.f;
+      x[cc][i] = valid ? to_float<QT>(e[i]) : 0.f;
+      mx = vmax(mx, fabsf(x[cc][i]));  // NaN-propagating
     }
   }
-  if (!finite) return __builtin_nanf("");
-  return qk_scale_log2 * ldexpf(1.f, ex) * code_scale<KF>();
+  mx = vmax(mx, shfl_xor(mx, 32));
+  constexpr float kLeast = sizeof(QT) == 4 ? 0x1p-3f : 0x1p-10f;
+  float back = 1.f;
+  const bool plain = mx == 0.f || (mx >= kLeast && mx < 32768.f);
+  if (__ballot(!plain) != 0) {
+    int ex = 0;
+    const bool finite = __builtin_isfinite(mx);
+    if (!plain && finite) {
+      frexpf(mx, &ex);
+      ex = max(ex - 15, -126);
+    }
+#pragma unroll
+    for (int cc = 0; cc < D / 16; ++cc)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[cc][i] = ldexpf(x[cc][i], -ex);
+    back = finite ? ldexpf(1.f, ex) : __builtin_nanf("");
+  }
+#pragma unroll
+  for (int cc = 0; cc < D / 16; ++cc)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const _Float16 hi = (_Float16)x[cc][i];
+      q.op[0][cc][i] = hi;
+      if constexpr (QOp<QT, D>::kTerms == 2) q.op[1][cc][i] = (_Float16)(x[cc][i] - (float)hi);
+    }
+  return back;
 }
 
-// Dequantized V of one staged block as the f16 A-operands of the PV MFMAs, written
-// once by the wave that loaded the block into the slab of its block pair: half `half`
-// of entry n * 64 + lane holds, for that lane (qg, r) of every wave,
-// V[4 qg + j][r * VB + n] * v_scale[4 qg + j] * 2^-e, j = 0..3, so that one 16-byte read
-// at the reader's own lane index gives the pair's whole operand (conflict-free). The
-// code is exact in f16 (FP8 codes times 2^-8) and multiplied by the f16-rounded scale
-// times 2^8 (times 2^-e). A slab value is at most v_scale * format_max in magnitude; the
-// block's exponent e (returned, wave-uniform) is the unit's current exponent `ve`, or
-// more when a scale exceeds `vlim` = 2^(15 + ve) / format_max, so every value stays
-// below 2^15. A block that was not loaded this step leaves stale codes and finite (or
-// zeroed) scales: finite values, which meet p = 0 for its keys.
+// The LDS of one workgroup: the f16 operands of two key steps (the one computed and the
+// one being converted), each of four 16-token blocks in two 32-key tiles.
+//   k  A operands of S^T = K Q^T: entry (tile, chunk cc, lane (key, h)) holds
+//      K[key][16 cc + 8 h + [0, 8)], the codes as f16 (exact)
+//   v  A operands of O^T += V^T P^T: entry (block, n, lane (r, h)) holds, of dimension
+//      d = (D / 32) r + n, the block's tokens 4 h + [0, 4) and 8 + 4 h + [0, 4), the rows
+//      of S^T that lane half h holds, times the token's V scale and 2^-e of the block
+//   ks the keys' score factors k_scale * qk_scale_log2 (* code_scale)
+//   pad the blocks' padding bytes; flags: the block's V exponent e, plus kLargeFlag where
+//   a key factor exceeds safe_factor()
+constexpr int kLargeFlag = 1 << 16;
 template <int D>
-__device__ __forceinline__ int convert_v(const char* st, int lane, int half, uint2* vt, int ve,
-                                         float vlim) {
-  using S = Stage<D>;
-  constexpr int VB = D / 16;
-  const int r = lane & 15, qg = lane >> 4;
-  const float4_t vsf = *reinterpret_cast<const float4_t*>(st + S::kS + 64 + 16 * qg);
-  constexpr float cs = v_weight_scale<KF>();
-  // the V code words go out with the scales, so that both LDS latencies overlap
-  uint32_t vw[4][VB / 4];
+struct PrefillLds {
+  static constexpr int kChunks = D / 16, kRowsN = D / 32;
+  uint4 k[2][2 * kChunks * kWave];
+  uint4 v[2][kWaves * kRowsN * kWave];
+  __attribute__((aligned(16))) float ks[2][kWaves * kBlockTokens];
+  __attribute__((aligned(16))) uint32_t pad[2][kWaves * 4];
+  __attribute__((aligned(16))) int flags[2][kWaves];
+};
+
+// One block of the wave's own as loaded from the arena, on its way to the operands. K:
+// lane (key = lane % 16, lane / 16) takes 16 consecutive d per 64. V: D / 4 lanes take the
+// dwords of a token row, for the lane's quads of four tokens (quad q: tokens 4 q + [0, 4)).
+template <int D>
+struct RawBlock {
+  static constexpr int kRowLanes = D / 4;             // lanes across a token row
+  static constexpr int kGroups = kWave / kRowLanes;   // 4, 2, 1
+  static constexpr int kQuads = 4 / kGroups;          // quads per lane: g, g + kGroups, ...
+  uint4 k[D / 64];
+  uint32_t v[kQuads][4];
+  float4_t vs[kQuads];
+  float ks;
+  uint32_t pad;
+  int id;
+};
+
+template <int D>
+__device__ __forceinline__ uint32_t load_pad(const AttnArgs& a, int id, int lane) {
+  return *reinterpret_cast<const uint32_t*>(a.cache.key_valid + (int64_t)id * kBlockTokens +
+                                            4 * (lane & 3));
+}
+
+// kPad: the padding bytes too (else convert_raw reads them)
+template <int D, bool kPad>
+__device__ __forceinline__ void load_raw(const AttnArgs& a, int id, int kvh, int lane, bool masks,
+                                         RawBlock<D>& b) {
+  using R = RawBlock<D>;
+  const int8_t* kp = a.cache.k_codes + id * a.cache.code_block_stride + kvh * a.cache.code_head_stride;
+  const int8_t* vp = a.cache.v_codes + id * a.cache.code_block_stride + kvh * a.cache.code_head_stride;
+  const float* ksp = a.cache.k_scales + id * a.cache.scale_block_stride + kvh * a.cache.scale_head_stride;
+  const float* vsp = a.cache.v_scales + id * a.cache.scale_block_stride + kvh * a.cache.scale_head_stride;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const char* rowp = st + S::kV + (4 * qg + j) * D + r * VB;
-    if constexpr (VB == 4) {
-      vw[j][0] = *reinterpret_cast<const uint32_t*>(rowp);
-    } else if constexpr (VB == 8) {
-      const uint2 w = *reinterpret_cast<const uint2*>(rowp);
-      vw[j][0] = w.x;
-      vw[j][1] = w.y;
-    } else {
-      const uint4 w = *reinterpret_cast<const uint4*>(rowp);
-      vw[j][0] = w.x;
-      vw[j][1] = w.y;
-      vw[j][2] = w.z;
-      vw[j][3] = w.w;
-    }
+  for (int i = 0; i < D / 64; ++i)
+    b.k[i] = *reinterpret_cast<const uint4*>(kp + (lane & 15) * D + (lane >> 4) * 16 + 64 * i);
+  const int g = lane / R::kRowLanes, dg = lane % R::kRowLanes;
+#pragma unroll
+  for (int q = 0; q < R::kQuads; ++q) {
+    const int quad = g + q * R::kGroups;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      b.v[q][t] = *reinterpret_cast<const uint32_t*>(vp + (4 * quad + t) * D + 4 * dg);
+    b.vs[q] = *reinterpret_cast<const float4_t*>(vsp + 4 * quad);
   }
-  half4_t vsh;
+  b.ks = ksp[lane & 15];
+  b.id = id;
+  if constexpr (kPad) b.pad = masks ? load_pad<D>(a, id, lane) : 0x01010101u;
+}
+
+// The wave's block into the operands of buffer `buf`, as block `w` of its step. The V
+// exponent e is the unit's current `ve`, or more where a scale exceeds `vlim` = 2^(15 + ve)
+// / format_max, so that every f16 product stays below 2^15.
+template <int D, bool kPad>
+__device__ __forceinline__ void convert_raw(const AttnArgs& a, const RawBlock<D>& b,
+                                            PrefillLds<D>& L, int buf, int w, int lane, bool masks,
+                                            int ve, float vlim) {
+  using R = RawBlock<D>;
+  using Lds = PrefillLds<D>;
+  // K: 16 codes -> the two lane halves' entries of one chunk
+  uint4* kd = L.k[buf] + (w / 2) * Lds::kChunks * kWave + 16 * (w % 2) + (lane & 15);
+#pragma unroll
+  for (int i = 0; i < D / 64; ++i) {
+    uint4* e = kd + (4 * i + (lane >> 4)) * kWave;
+    half2_t p[8];
+    codes_to_f16<KF>(b.k[i].x, p[0], p[1]);
+    codes_to_f16<KF>(b.k[i].y, p[2], p[3]);
+    codes_to_f16<KF>(b.k[i].z, p[4], p[5]);
+    codes_to_f16<KF>(b.k[i].w, p[6], p[7]);
+    auto word = [&](int j) { return __builtin_bit_cast(uint32_t, p[j]); };
+    e[0] = uint4{word(0), word(1), word(2), word(3)};
+    e[32] = uint4{word(4), word(5), word(6), word(7)};
+  }
+  // V
+  float vsm = 0.f;
+#pragma unroll
+  for (int q = 0; q < R::kQuads; ++q)
+    vsm = fmaxf(vsm, fmaxf(fmaxf(b.vs[q][0], b.vs[q][1]), fmaxf(b.vs[q][2], b.vs[q][3])));
+  constexpr float cs = v_weight_scale<KF>();
   int e = ve;
-  const float vsm = fmaxf(fmaxf(vsf[0], vsf[1]), fmaxf(vsf[2], vsf[3]));
+  float c = cs;
   if (__ballot(vsm > vlim) != 0 || ve != 0) {
     if (__ballot(vsm > vlim) != 0) {
-      float wm = fmaxf(vsm, shfl_xor(vsm, 16));
-      wm = fmaxf(wm, shfl_xor(wm, 32));
+      float wm = 0.f;  // a group of lanes holds the same scales: 16 lanes or more
+#pragma unroll
+      for (int i = 0; i < kWave; i += 16)
+        wm = fmaxf(wm, __builtin_bit_cast(float, __builtin_amdgcn_readlane(
+                                                     __builtin_bit_cast(int, vsm), i)));
       int x;
       frexpf(wm * (format_max<KF>() / 32768.f), &x);  // wm * M / 2^15 in [2^(x-1), 2^x)
       e = max(ve, __builtin_amdgcn_readfirstlane(x));
     }
-    const float c = ldexpf(cs, -e);
-    vsh = half4_t{(_Float16)(vsf[0] * c), (_Float16)(vsf[1] * c), (_Float16)(vsf[2] * c),
-                  (_Float16)(vsf[3] * c)};
-  } else {
-    vsh = half4_t{(_Float16)(vsf[0] * cs), (_Float16)(vsf[1] * cs), (_Float16)(vsf[2] * cs),
-                  (_Float16)(vsf[3] * cs)};
+    c = ldexpf(cs, -e);
   }
+  const int g = lane / R::kRowLanes, dg = lane % R::kRowLanes;
+  half4_t vop[4][R::kQuads];
 #pragma unroll
-  for (int n = 0; n < VB; ++n) {
-    const uint32_t col[4] = {vw[0][n / 4], vw[1][n / 4], vw[2][n / 4], vw[3][n / 4]};
-    half4_t v;
-    switch (n % 4) {
-      case 0: v = v_operand<0, KF>(col); break;
-      case 1: v = v_operand<1, KF>(col); break;
-      case 2: v = v_operand<2, KF>(col); break;
-      default: v = v_operand<3, KF>(col); break;
-    }
-    if constexpr (KF == kE5M2) {
-      constexpr _Float16 down = (_Float16)(1.f / 256.f);
-      v = v * half4_t{down, down, down, down};  // exact: E5M2 values times 2^-8 fit f16
-    }
-    vt[2 * (n * kWave + lane) + half] = __builtin_bit_cast(uint2, v * vsh);
-  }
-  return e;
-}
-
-// The PV MFMAs of one step: weights p = exp2(u * cfe - m) rounded to f16 for the 32 keys
-// of each block pair, against the slab of that pair, and the row sums from the same
-// rounded weights. The weights of block b carry 2^(e_b - ve) (vf[b], at most 1, exact
-// on f16; 1 unless the step's blocks were converted with different exponents) for the
-// numerator only (scaled in place after the row sums), so that every block's products
-// are in units of 2^-ve.
-template <int D, int NT>
-__device__ __forceinline__ void prefill_pv(const uint4* vt, const float (&u)[NT][16],
-                                           const float (&cfe)[NT], const float (&m)[NT],
-                                           int lane, const half8_t& ones, const half4_t& vf,
-                                           float4_t (&acc)[NT][D / 16 + 1]) {
-  constexpr int NPV = D / 16;
+  for (int q = 0; q < R::kQuads; ++q) {
+    const half4_t vsh = {(_Float16)(b.vs[q][0] * c), (_Float16)(b.vs[q][1] * c),
+                         (_Float16)(b.vs[q][2] * c), (_Float16)(b.vs[q][3] * c)};
+    vop[0][q] = v_operand<0, KF>(b.v[q]);
+    vop[1][q] = v_operand<1, KF>(b.v[q]);
+    vop[2][q] = v_operand<2, KF>(b.v[q]);
+    vop[3][q] = v_operand<3, KF>(b.v[q]);
 #pragma unroll
-  for (int pp = 0; pp < 2; ++pp) {
-    half8_t pop[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        pop[t][i] = (_Float16)__builtin_amdgcn_exp2f(fmaf(u[t][8 * pp + i], cfe[t], -m[t]));
-    // row sums: a V^T row of ones (row 0 of the extra tile) gives sum_k f16(p_k), the
-    // same rounded weights the numerator uses
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-      acc[t][NPV] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pop[t], acc[t][NPV], 0, 0, 0);
-    // (branch-free: vf is 1 but where the step mixes exponents, and a branch here would
-    // split the exponentials from the PV MFMAs they overlap with)
-    {
-      const _Float16 f0 = vf[2 * pp], f1 = vf[2 * pp + 1];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) pop[t] = pop[t] * half8_t{f0, f0, f0, f0, f1, f1, f1, f1};
-    }
-#pragma unroll
-    for (int n = 0; n < NPV; ++n) {
-      const half8_t vop = __builtin_bit_cast(half8_t, vt[pp * (NPV * kWave) + n * kWave + lane]);
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        acc[t][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop, pop[t], acc[t][n], 0, 0, 0);
-    }
-  }
-}
-
-// One key step: the four staged 16-token blocks w = 0..3 (first key position
-// kb0 + 16 w) through the MFMAs for the wave's NT column tiles:
-//   S^T = K . Q^T      v_mfma_i32_16x16x64_i8 twice per 64-wide d chunk (hi, then lo
-//                      on the hi result shifted by 7): exact int32 dot products
-//   O^T += V^T . P^T   v_mfma_f32_16x16x32_f16 over the 32 keys of block pair
-//                      (0, 1) and (2, 3); V^T carries the V scales, one more tile
-//                      with a row of ones accumulates the softmax row sums
-// Score slot j = 4 w + i of lane group qg is key 4 qg + i of block w; in the PV
-// operands, slots 8 p + [0, 8) of pair p match the interleaved V slab. The base-2
-// score of a key is u * cf with u = S_int * k_scale, folded into the exponent as
-// fma(u, cfe, -m) (cfe = cf, or FLT_MIN where cf = 0, so that a masked u = -inf stays
-// -inf). Bit w of `use` (wave-uniform): block w holds keys some column of the wave
-// sees; of `bounded`: the column bounds [lo, hi] cut into block w. `masks`: the
-// stages carry the blocks' padding bytes (0 = padding key), and a step holding one
-// takes the edge path.
-// With every block used, none bounded and every key scale times query factor below
-// kSafeFactor (no score can overflow) the step takes no per-score condition; otherwise
-// the scores are masked to -inf outside the bounds, for padding keys and for unused
-// blocks (whose stages hold stale but finite codes and scales) and checked for
-// non-finite values.
-// The query columns of a wave's NT tiles, for the third query term: column t of lane
-// (qg, r) is head chead[t] of token row q0 + ctok[t] (token row q0 + t0 when it is not
-// valid, as loaded for the first two terms).
-template <int NT>
-struct ColumnRefs {
-  int q0, t0;
-  const int (&ctok)[NT];
-  const int (&chead)[NT];
-  const bool (&cvalid)[NT];
-};
-
-// The third query term of a step (INT8 codes, every tile of the wave): per 64-wide d
-// chunk, lo2 rebuilt from the query elements by the column's own quantization (the terms
-// query_column_i8 gives for three terms), that chunk's K.lo2 exact in int32 on the
-// staged codes, added to the dequantized scores as (K.lo2 / 128) * ks. One chunk of one
-// tile is live at a time and the key scales are read again from LDS, so the path fits
-// beside the step's accumulators.
-template <typename QT, int D, int NT>
-__device__ __forceinline__ void prefill_third_term(const char* cur, const AttnArgs& a,
-                                                   const ColumnRefs<NT>& col, int r, int qg,
-                                                   float (&u)[NT][4 * kWaves]) {
-  using S = Stage<D>;
-  constexpr int KCH = D / 64;
-  constexpr int kVec = 16 / (int)sizeof(QT);
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const QT* qp = static_cast<const QT*>(a.q) +
-                   (int64_t)(col.q0 + (col.cvalid[t] ? col.ctok[t] : col.t0)) * a.q_tok +
-                   (int64_t)col.chead[t] * a.q_head + 16 * qg;
-    // the column's quantization as query_column_i8 sets it: the NaN-propagating maximum
-    // of |q| over the column (lanes r, r + 16, r + 32, r + 48), the exact lift of columns
-    // below 2^-64 and inv = kQRange / max (a maximum does not depend on its order)
-    float mx = 0.f;
-#pragma nounroll
-    for (int h = 0; h < KCH; ++h) {
-      uint4 w[16 / kVec];
-#pragma unroll
-      for (int c = 0; c < 16 / kVec; ++c) w[c] = reinterpret_cast<const uint4*>(qp + 64 * h)[c];
-      const QT* e = reinterpret_cast<const QT*>(w);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) mx = vmax(mx, fabsf(to_float<QT>(e[i])));
-    }
-    mx = vmax(mx, shfl_xor(mx, 16));
-    mx = vmax(mx, shfl_xor(mx, 32));
-    mx = col.cvalid[t] ? mx : 0.f;
-    const bool finite = __builtin_isfinite(mx);
-    const float up = mx > 0.f && mx < 0x1p-64f ? 0x1p64f : 1.f;
-    mx *= up;
-    const float inv = (finite && mx > 0.f) ? (float)kQRange / mx : 0.f;
-#pragma nounroll
-    for (int h = 0; h < KCH; ++h) {
-      uint4 w[16 / kVec];
-#pragma unroll
-      for (int c = 0; c < 16 / kVec; ++c) w[c] = reinterpret_cast<const uint4*>(qp + 64 * h)[c];
-      const QT* e = reinterpret_cast<const QT*>(w);
-      int4_t lo2;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        uint32_t fb[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          fb[i] = __builtin_bit_cast(
-              uint32_t,
-              query_terms<3>(to_float<QT>(e[4 * k + i]) * up, inv).lo2);
-        lo2[k] = (int)low_bytes(fb);
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (KF == kE5M2) {
+        constexpr _Float16 down = (_Float16)(1.f / 256.f);
+        vop[i][q] = vop[i][q] * half4_t{down, down, down, down};  // exact: E5M2 times 2^-8 fits f16
       }
-      // chunk h's share of K.lo2 (exact), added to each score on its own
-#pragma unroll
-      for (int b = 0; b < kWaves; ++b) {
-        const char* st = cur + b * S::kBytes;
-        const int4_t sf = __builtin_amdgcn_mfma_i32_16x16x64_i8(
-            *reinterpret_cast<const int4_t*>(st + S::kK + k_chunk<D>(r, qg + 4 * h)), lo2,
-            int4_t{0, 0, 0, 0}, 0, 0, 0);
-        const float4_t ks = *reinterpret_cast<const float4_t*>(st + S::kS + 16 * qg);
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          u[t][4 * b + k] = __builtin_fmaf((float)sf[k], ks[k] * (1.f / 128.f), u[t][4 * b + k]);
-      }
+      vop[i][q] = vop[i][q] * vsh;
     }
   }
-}
-
-template <typename QT, int D, int NT>
-__device__ __forceinline__ void prefill_step(const char* cur, const uint4* vt, uint32_t use,
-                                             uint32_t bounded, bool masks, int kb0,
-                                             const QOp<D> (&qop)[NT],
-                                             const float (&cf)[NT], const float (&cfe)[NT],
-                                             const int (&lo)[NT], const int (&hi)[NT], int r,
-                                             int qg, const half8_t& ones,
-                                             const half4_t& vf,
-                                             float4_t (&acc)[NT][D / 16 + 1], float (&m)[NT],
-                                             bool& bad_score, const AttnArgs& a,
-                                             const ColumnRefs<NT>& cols) {
-  using S = Stage<D>;
-  constexpr int KCH = D / 64;
-  constexpr int NPV = D / 16;
-  constexpr int NBK = kWaves;  // blocks per step
-  // a step holding a padding key takes the edge path (read ahead of the QK block)
-  bool padded = false;
-  if (masks) {
-    uint32_t bad = 0;
+  // dimension d = 4 dg + i is row r = d / (D / 32) of operand n = d % (D / 32); quad
+  // 2 a' + h is half a' of lane half h's entry
+  uint4* vd = L.v[buf] + w * Lds::kRowsN * kWave;
 #pragma unroll
-    for (int b = 0; b < NBK; ++b)
-      bad |= *reinterpret_cast<const uint32_t*>(cur + b * S::kBytes + S::kF + 4 * qg) ^ 0x01010101u;
-    padded = __ballot(bad != 0) != 0;
-  }
-  // raw scores of key 4 qg + i of block b, column tile t: exact int32 (int8 codes) or
-  // f32 (FP8 codes as f16 against the f16 query)
-  using Acc = typename std::conditional<KF == kInt8, int4_t, float4_t>::type;
-  Acc sacc[NBK][NT];
-#pragma unroll
-  for (int b = 0; b < NBK; ++b) {
-    const char* st = cur + b * S::kBytes;
-    if constexpr (KF == kInt8) {
-      int4_t kop[KCH];
-#pragma unroll
-      for (int h = 0; h < KCH; ++h)
-        kop[h] = *reinterpret_cast<const int4_t*>(st + S::kK + k_chunk<D>(r, qg + 4 * h));
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        sacc[b][t] = int4_t{0, 0, 0, 0};
-#pragma unroll
-        for (int h = 0; h < KCH; ++h)
-          sacc[b][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop[h], qop[t].hi[h], sacc[b][t], 0, 0, 0);
-        sacc[b][t] = sacc[b][t] << 7;
-#pragma unroll
-        for (int h = 0; h < KCH; ++h)
-          sacc[b][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop[h], qop[t].lo[h], sacc[b][t], 0, 0, 0);
-      }
+  for (int i = 0; i < 4; ++i) {
+    const int d = 4 * dg + i, r = d / Lds::kRowsN, n = d % Lds::kRowsN;
+    if constexpr (R::kGroups == 4) {
+      reinterpret_cast<uint2*>(vd + n * kWave + 32 * (g & 1) + r)[g >> 1] =
+          __builtin_bit_cast(uint2, vop[i][0]);
+    } else if constexpr (R::kGroups == 2) {
+      const uint2 lo = __builtin_bit_cast(uint2, vop[i][0]), hi = __builtin_bit_cast(uint2, vop[i][1]);
+      vd[n * kWave + 32 * g + r] = uint4{lo.x, lo.y, hi.x, hi.y};
     } else {
 #pragma unroll
-      for (int t = 0; t < NT; ++t) sacc[b][t] = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int h = 0; h < KCH; ++h) {
-        const uint4 c = *reinterpret_cast<const uint4*>(st + S::kK + k_chunk<D>(r, qg + 4 * h));
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub) {
-          half2_t p0, p1, p2, p3;
-          codes_to_f16<KF>(sub ? c.z : c.x, p0, p1);
-          codes_to_f16<KF>(sub ? c.w : c.y, p2, p3);
-          const half8_t kop = {p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-#pragma unroll
-          for (int t = 0; t < NT; ++t)
-            sacc[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop, qop[t].op[2 * h + sub],
-                                                                 sacc[b][t], 0, 0, 0);
-        }
+      for (int h = 0; h < 2; ++h) {
+        const uint2 lo = __builtin_bit_cast(uint2, vop[i][h]);
+        const uint2 hi = __builtin_bit_cast(uint2, vop[i][2 + h]);
+        vd[n * kWave + 32 * h + r] = uint4{lo.x, lo.y, hi.x, hi.y};
       }
     }
   }
-  float4_t ks[NBK];
-#pragma unroll
-  for (int b = 0; b < NBK; ++b)
-    ks[b] = *reinterpret_cast<const float4_t*>(cur + b * S::kBytes + S::kS + 16 * qg);
-  // computed without a branch, so that the QK MFMAs and the conversions below share
-  // one block: scales are finite and >= 0, their order is that of their bit patterns
-  int kx = 0;
-#pragma unroll
-  for (int b = 0; b < NBK; ++b) {
-    const int4_t kb = __builtin_bit_cast(int4_t, ks[b]);
-    kx = max(kx, max(max(kb[0], kb[1]), max(kb[2], kb[3])));
-  }
-  const float kmax = __builtin_bit_cast(float, kx);
-  bool ok = true, fine = false;
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const float x = kmax * cf[t];
-    ok = ok && x <= safe_factor();  // false for NaN
-    if constexpr (KF == kInt8) fine = fine || x > kFineScoreError / (63.5f * D);
-  }
-  const bool unsafe = __ballot(!ok) != 0;
-  float u[NT][4 * NBK];
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int j = 0; j < 4 * NBK; ++j) u[t][j] = (float)sacc[j / 4][t][j % 4] * ks[j / 4][j % 4];
-  if constexpr (KF == kInt8) {
-    // steps whose key scales make the two-term query's error bound pass the budget
-    if (__builtin_expect(__ballot(fine) != 0, 0)) prefill_third_term<QT, D, NT>(cur, a, cols, r, qg, u);
-  }
-  const bool edge = (use != (1u << NBK) - 1) | (bounded != 0) | unsafe | padded;
-  if (edge) {
-    asm volatile("");  // keeps this a branch: if-converted, the interior steps would pay for it
-    // Per-score masks as all-ones/zero words in VGPRs (sign bits of differences, bit
-    // selects), not as compare results: lane masks from 32 unrolled compares per tile
-    // would stay live in SGPRs and push the loop's uniform values into spills.
-    uint32_t nonfinite = 0;
-#pragma unroll
-    for (int b = 0; b < NBK; ++b) {
-      // the padding bytes of this lane's four keys of block b (1 = real, 0 = padding)
-      const uint32_t pad = masks ? *reinterpret_cast<const uint32_t*>(cur + b * S::kBytes + S::kF +
-                                                                      4 * qg)
-                                 : 0x01010101u;
-      const bool used = (use >> b) & 1u, bnd = (bounded >> b) & 1u;  // wave-uniform
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int j = 4 * b + k;
-        const int key = kb0 + 16 * b + 4 * qg + k;
-        const int32_t padding = (int32_t)(((pad >> (8 * k)) & 0xffu) - 1u) >> 31;  // -1: padding
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          // -1 when key < lo or key > hi (either difference negative), else 0
-          const int32_t outside = bnd ? ((key - lo[t]) | (hi[t] - key)) >> 31 : 0;
-          const uint32_t hide = used ? (uint32_t)(outside | padding) : 0xffffffffu;
-          const uint32_t ub = __builtin_bit_cast(uint32_t, u[t][j]);
-          const uint32_t xb = __builtin_bit_cast(uint32_t, u[t][j] * cf[t]);
-          // exponent field all ones (inf or NaN) -> bit 31 after the carry
-          nonfinite |= ((xb & 0x7f800000u) + 0x00800000u) & ~hide;
-          u[t][j] = __builtin_bit_cast(float, (ub & ~hide) | (0xff800000u & hide));  // -inf
-        }
-      }
-    }
-    if (__ballot((nonfinite >> 31) != 0) != 0) bad_score = true;
-  }
-  float tmax[NT];
-  bool need = false;
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    // NaN-propagating maximum (v_maximum3_f32: no operand canonicalization)
-    float mu = u[t][0];
-#pragma unroll
-    for (int j = 1; j < 4 * NBK; ++j) mu = vmax(mu, u[t][j]);
-    tmax[t] = mu * cfe[t];  // cfe > 0: the maximum of the scaled scores
-    need |= tmax[t] > m[t] + kRescaleSlack;
-  }
-  if (__ballot(need) != 0) {
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      float x = fmaxf(tmax[t], shfl_xor(tmax[t], 16));
-      x = fmaxf(x, shfl_xor(x, 32));
-      const float mn = fmaxf(m[t], x);
-      const float alpha = __builtin_amdgcn_exp2f(m[t] - mn);
-#pragma unroll
-      for (int n = 0; n <= NPV; ++n) acc[t][n] *= alpha;
-      m[t] = mn;
-    }
-  }
-  static_assert(NBK == 4, "two block pairs per step");
-  const int lane = qg * 16 + r;
-  prefill_pv<D, NT>(vt, u, cfe, m, lane, ones, vf, acc);
+  // key factors: at least FLT_MIN, so that a masked score's -inf stays -inf
+  const float ksf = fmaxf(b.ks * (a.qk_scale_log2 * code_scale<KF>()), FLT_MIN);
+  const bool large = __ballot(!(ksf <= safe_factor())) != 0;
+  if (lane < 16) L.ks[buf][16 * w + lane] = ksf;
+  if (masks && lane < 4) L.pad[buf][4 * w + lane] = kPad ? b.pad : load_pad<D>(a, b.id, lane);
+  if (lane == 0) L.flags[buf][w] = e | (large ? kLargeFlag : 0);
 }
 
-// N consecutive outputs from fp32, with 16-byte (or 8-byte) stores.
-template <typename QT, int N>
-__device__ __forceinline__ void store_run(QT* dst, const float (&v)[N]) {
-  constexpr int kVec = 16 / (int)sizeof(QT);
-  if constexpr (sizeof(QT) == 2 && N % 8 == 0) {
-#pragma unroll
-    for (int c = 0; c < N / 8; ++c) {
-      const uint4 w = {pack2<QT>(v[8 * c], v[8 * c + 1]), pack2<QT>(v[8 * c + 2], v[8 * c + 3]),
-                       pack2<QT>(v[8 * c + 4], v[8 * c + 5]), pack2<QT>(v[8 * c + 6], v[8 * c + 7])};
-      reinterpret_cast<uint4*>(dst)[c] = w;
-    }
-  } else if constexpr (sizeof(QT) == 2 && N == 4) {
-    *reinterpret_cast<uint2*>(dst) = uint2{pack2<QT>(v[0], v[1]), pack2<QT>(v[2], v[3])};
-  } else if constexpr (N % kVec == 0) {
-#pragma unroll
-    for (int c = 0; c < N / kVec; ++c) {
-      uint4 w;
-      QT* e = reinterpret_cast<QT*>(&w);
-#pragma unroll
-      for (int i = 0; i < kVec; ++i) e[i] = from_float<QT>(v[c * kVec + i]);
-      reinterpret_cast<uint4*>(dst)[c] = w;
-    }
-  } else if constexpr (N * (int)sizeof(QT) == 8) {
-    uint2 w;
-    QT* e = reinterpret_cast<QT*>(&w);
-#pragma unroll
-    for (int i = 0; i < N; ++i) e[i] = from_float<QT>(v[i]);
-    *reinterpret_cast<uint2*>(dst) = w;
-  } else {
-#pragma unroll
-    for (int i = 0; i < N; ++i) dst[i] = from_float<QT>(v[i]);
-  }
-}
-
-// The LDS of one prefill workgroup: the key-step stages, the V operand slabs of the
-// current step and the step's block exponents.
-template <int D>
-struct PrefillLds {
-  static constexpr int NB = kPrefillBuffers;  // key steps in flight: NB - 1 ahead of the one computed
-  __attribute__((aligned(16))) char stages[NB * kWaves * Stage<D>::kBytes];  // [step % NB][wave]
-  uint4 vt[kWaves / 2][(D / 16) * kWave];  // the current step's V operands, one slab per pair
-  __attribute__((aligned(16))) int vexp[kWaves];  // the step's block exponents
-};
-
-// A workgroup's columns: flat column f = (wave * NT + t) * 16 + r. The unit's columns
+// A workgroup's columns: flat column f = (wave * NT + t) * 32 + c. The unit's columns
 // read query token rows q0 + tok (an invalid column reads row q0 + t0 and is zeroed)
 // and see keys [lo, hi]; per wave, the bounds of its columns' key ranges (lo_min ..
 // hi_max: keys some column sees; lo_max .. hi_min: keys every valid column sees) and
@@ -718,193 +476,353 @@ struct WaveBounds {
   bool any;
 };
 
+// Half a key step: the 32 keys from position kb0 on (blocks w = 0, 1 of tile kt of the
+// step's operands) through the MFMAs for the wave's NT column tiles:
+//   S^T = K Q^T       v_mfma_f32_32x32x16_f16 over the 16-wide d chunks
+//   O^T += V^T P^T    v_mfma_f32_32x32x16_f16 over each block's 16 keys
+// Lane (c, h) holds column c's scores of keys 8 a + 4 h + b (element 4 a + b), which is
+// the layout that P^T enters the second product in. t = s * ks - m is the base-2 score
+// over the running maximum, p = exp2(t). Bit w of `use` (wave-uniform): block w holds keys
+// some column of the wave sees; of `bounded`: the column bounds [lo, hi] cut into block w.
+// `slow`: a column is scaled or a key factor large. Keys that are all used, not bounded,
+// not padded and not slow take no per-score condition (no score can overflow); otherwise
+// scores are masked to -inf outside the bounds, for padding keys and for unused blocks
+// (whose operands are stale but finite) and checked for non-finite values. vf: the blocks'
+// exponent factors 2^(e_w - ve) on the weights of the numerator only, where `vmix`.
+//
+// The operands come from LDS well ahead of their MFMAs (a read takes over 100 cycles, and a
+// wave that waits for each pair of them spends more time there than on the arithmetic): the
+// caller passes this half's K operands, and the V operands go out before the scores.
+// `between` runs ahead of the output MFMAs (it loads the next half's K operands).
+template <int D>
+__device__ __forceinline__ void load_k_operands(const PrefillLds<D>& L, int buf, int kt, int lane,
+                                                half8_t (&kop)[D / 16]) {
+  const uint4* kp = L.k[buf] + kt * PrefillLds<D>::kChunks * kWave + lane;
+#pragma unroll
+  for (int cc = 0; cc < D / 16; ++cc) kop[cc] = __builtin_bit_cast(half8_t, kp[cc * kWave]);
+}
+
+template <typename QT, int D, int NT, typename Between>
+__device__ __forceinline__ void prefill_half(const PrefillLds<D>& L, int buf, int kt, uint32_t use,
+                                             uint32_t bounded, bool masks, bool slow, int kb0,
+                                             half8_t (&kop)[D / 16], Between between,
+                                             const QOp<QT, D> (&qop)[NT], const float (&back)[NT],
+                                             const int (&lo)[NT], const int (&hi)[NT], int lane,
+                                             bool vmix, half2_t vf,
+                                             float16v_t (&acc)[NT][D / 32], float (&m)[NT],
+                                             float (&l)[NT], bool& bad_score) {
+  using Lds = PrefillLds<D>;
+  const int h = lane >> 5;
+  bool padded = false;
+  if (masks) {
+    const uint4 pw = *reinterpret_cast<const uint4*>(&L.pad[buf][8 * kt + 4 * (lane & 1)]);
+    padded = __ballot(pw.x != 0x01010101u || pw.y != 0x01010101u || pw.z != 0x01010101u ||
+                      pw.w != 0x01010101u) != 0;
+  }
+  constexpr int kAhead = QOp<QT, D>::kAhead ? D == 128 ? 6 : 2 * Lds::kRowsN : 0;
+  half8_t vop[2 * Lds::kRowsN];
+  auto load_v = [&](int n0, int n1) __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = n0; n < n1; ++n)
+      vop[n] = __builtin_bit_cast(half8_t, L.v[buf][(2 * kt * Lds::kRowsN + n) * kWave + lane]);
+  };
+  if constexpr (QOp<QT, D>::kAhead) {
+    load_v(0, kAhead);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  float16v_t s[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) s[t][j] = 0.f;
+#pragma unroll
+  for (int cc = 0; cc < Lds::kChunks; ++cc) {
+    if constexpr (!QOp<QT, D>::kAhead)
+      kop[cc] = __builtin_bit_cast(half8_t, L.k[buf][(kt * Lds::kChunks + cc) * kWave + lane]);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int x = 0; x < QOp<QT, D>::kTerms; ++x)
+        s[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kop[cc], qop[t].op[x][cc], s[t], 0, 0, 0);
+  }
+  float4_t ks[4];  // factors of keys 8 x + 4 h + [0, 4)
+#pragma unroll
+  for (int x = 0; x < 4; ++x)
+    ks[x] = *reinterpret_cast<const float4_t*>(&L.ks[buf][32 * kt + 8 * x + 4 * h]);
+  if constexpr (QOp<QT, D>::kAhead) __builtin_amdgcn_sched_barrier(0);
+  if (use != 3u || bounded != 0 || slow || padded) {
+    asm volatile("");  // keeps this a branch: if-converted, the interior steps would pay for it
+    // Per-score masks as all-ones/zero words in VGPRs (sign bits of differences, bit
+    // selects): lane masks of unrolled compares would stay live in SGPRs and spill.
+    uint32_t nonfinite = 0;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const int w = x / 2;
+      const uint32_t pad = masks ? L.pad[buf][8 * kt + 2 * x + h] : 0x01010101u;
+      const bool used = (use >> w) & 1u, bnd = (bounded >> w) & 1u;  // wave-uniform
+#pragma unroll
+      for (int y = 0; y < 4; ++y) {
+        const int j = 4 * x + y;
+        const int key = kb0 + 8 * x + 4 * h + y;
+        const int32_t padding = (int32_t)(((pad >> (8 * y)) & 0xffu) - 1u) >> 31;  // -1: padding
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          // -1 when key < lo or key > hi (either difference negative), else 0
+          const int32_t outside = bnd ? ((key - lo[t]) | (hi[t] - key)) >> 31 : 0;
+          const uint32_t hide = used ? (uint32_t)(outside | padding) : 0xffffffffu;
+          const float sv = s[t][j] * back[t];
+          const uint32_t xb = __builtin_bit_cast(uint32_t, sv * ks[x][y]);
+          // exponent field all ones (inf or NaN) -> bit 31 after the carry
+          nonfinite |= ((xb & 0x7f800000u) + 0x00800000u) & ~hide;
+          s[t][j] = __builtin_bit_cast(
+              float, (__builtin_bit_cast(uint32_t, sv) & ~hide) | (0xff800000u & hide));  // -inf
+        }
+      }
+    }
+    if (__ballot((nonfinite >> 31) != 0) != 0) bad_score = true;
+  }
+  bool need = false;
+  float me[NT], tmax[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    me[t] = m[t] > -FLT_MAX ? m[t] : 0.f;  // a column without a key so far: scores as they are
+    float mu = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      s[t][j] = __builtin_fmaf(s[t][j], ks[j / 4][j % 4], -me[t]);
+      mu = vmax(mu, s[t][j]);  // NaN-propagating
+    }
+    tmax[t] = mu;
+    need |= !(mu <= kRescaleSlack) || m[t] == -FLT_MAX;
+  }
+  if (__ballot(need) != 0) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const float x = max32(tmax[t]) + me[t];
+      const float mn = fmaxf(m[t], x);
+      const float alpha = __builtin_amdgcn_exp2f(m[t] - mn);
+      const float shift = (mn > -FLT_MAX ? mn : 0.f) - me[t];
+#pragma unroll
+      for (int n = 0; n < Lds::kRowsN; ++n) acc[t][n] *= alpha;
+      l[t] *= alpha;
+      m[t] = mn;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) s[t][j] -= shift;
+    }
+  }
+  // weights rounded to f16; the sums take the same rounded weights as the numerator
+  typedef uint32_t word4_t __attribute__((ext_vector_type(4)));
+  word4_t pop[NT][2];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i0 = 8 * w + 2 * j;
+        const uint32_t pair = pack2<_Float16>(__builtin_amdgcn_exp2f(s[t][i0]),
+                                              __builtin_amdgcn_exp2f(s[t][i0 + 1]));
+        l[t] = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, pair),
+                                      half2_t{(_Float16)1.f, (_Float16)1.f}, l[t], false);
+        pop[t][w][j] = pair;
+      }
+  if constexpr (QOp<QT, D>::kAhead) {
+    load_v(kAhead, 2 * Lds::kRowsN);
+    between();
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // (the sums are done here: sunk past the branch, they would keep a second copy of the weights)
+#pragma unroll
+  for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(l[t]));
+  if (__builtin_expect(vmix, 0)) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        const _Float16 f = vf[w];
+        pop[t][w] = __builtin_bit_cast(word4_t, __builtin_bit_cast(half8_t, pop[t][w]) *
+                                                    half8_t{f, f, f, f, f, f, f, f});
+      }
+  }
+#pragma unroll
+  for (int w = 0; w < 2; ++w)
+#pragma unroll
+    for (int n = 0; n < Lds::kRowsN; ++n) {
+      const int x = w * Lds::kRowsN + n;
+      if constexpr (!QOp<QT, D>::kAhead) load_v(x, x + 1);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        acc[t][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+            vop[x], __builtin_bit_cast(half8_t, pop[t][w]), acc[t][n], 0, 0, 0);
+    }
+}
+
+// N consecutive outputs from fp32, with 16-byte stores.
+template <typename QT, int N>
+__device__ __forceinline__ void store_run(QT* dst, const float (&v)[N]) {
+  constexpr int kVec = 16 / (int)sizeof(QT);
+  static_assert(N % kVec == 0, "whole 16-byte stores");
+#pragma unroll
+  for (int c = 0; c < N / kVec; ++c) {
+    uint4 w;
+    if constexpr (sizeof(QT) == 2) {
+      w = uint4{pack2<QT>(v[8 * c], v[8 * c + 1]), pack2<QT>(v[8 * c + 2], v[8 * c + 3]),
+                pack2<QT>(v[8 * c + 4], v[8 * c + 5]), pack2<QT>(v[8 * c + 6], v[8 * c + 7])};
+    } else {
+      QT* e = reinterpret_cast<QT*>(&w);
+#pragma unroll
+      for (int i = 0; i < kVec; ++i) e[i] = from_float<QT>(v[c * kVec + i]);
+    }
+    reinterpret_cast<uint4*>(dst)[c] = w;
+  }
+}
+
+// The D / 8 consecutive outputs that lane half h holds of its column in accumulator rows
+// 8 x + 4 h + [0, 4): elements D / 4 x + D / 8 h + [0, D / 8).
+template <int D>
+__device__ __forceinline__ void acc_run(const float16v_t (&acc)[D / 32], int x, float scale,
+                                        float (&v)[D / 8]) {
+#pragma unroll
+  for (int y = 0; y < 4; ++y)
+#pragma unroll
+    for (int n = 0; n < D / 32; ++n) v[y * (D / 32) + n] = acc[n][4 * x + y] * scale;
+}
+
 // One unit of the chunked-prefill kernels: the key blocks [b_lo, b_hi) of kv head kvh
 // (physical id of block b: blocks[b], a window of the arena's ids) against the
 // workgroup's query columns (column_of(f), bounds_of(wave)), through the key steps
-// described at the top of this file; store(t, acc, m, lt, ve, col) then takes column
-// tile t of each wave (acc in units of 2^-ve, lt the row sums of lane (0, r)'s column).
-// prologue() runs (in uniform control flow) once the stages are cleared and the first
-// block ids are on their way, before any column is read: it returns false (uniformly)
-// to end the unit there, with nothing stored. mark(k) is called at the unit's timeline
-// marks 2-5 (the tile kernel's trace builds).
-template <typename QT, int D, int G, typename ColumnOf, typename BoundsOf, typename Store,
+// described at the top of this file; store(t, acc, m, l, ve, col) then takes column
+// tile t of each wave (acc in units of 2^-ve, l the sums of the column's weights).
+// prologue() runs (in uniform control flow) once the first block ids are on their way,
+// before any column is read: it returns false (uniformly) to end the unit there, with
+// nothing stored. mark(k) is called at the unit's timeline marks 2-5 (the tile kernel's
+// trace builds).
+template <typename QT, int D, typename ColumnOf, typename BoundsOf, typename Store,
           typename Prologue, typename Mark>
 __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L, int kvh,
                                              int b_lo, int b_hi, const int32_t* blocks, int q0,
                                              int t0, ColumnOf column_of, BoundsOf bounds_of,
                                              Store store, Prologue prologue, Mark mark) {
-  using S = Stage<D>;
   constexpr int NT = PrefillShape<D>::NT;
-  constexpr int NPV = D / 16;
-  constexpr int NB = PrefillLds<D>::NB;
+  constexpr int kRowsN = D / 32;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int lane = threadIdx.x % kWave;
-  const int r = lane & 15, qg = lane >> 4;
-  char* const lds = L.stages;
   const int nsteps = (b_hi - b_lo + kWaves - 1) / kWaves;
 
-  // The block ids of the first 64 steps go out first, so that their load overlaps the
-  // clearing of the stages and the prologue. After each load the ids pass through an
-  // empty asm that redefines them: the one wait for their load happens there (once per
-  // 64 steps), and the compiler's wait tracking no longer treats them as a pending load
-  // at every issue below (where it would wait for every stage in flight, vmcnt(0), each
-  // step).
+  // Block b_lo + 4 * step + w is wave w's. Lane i of `ids` holds the id for step
+  // i + 64 * k; reloaded every 64 steps. A block past the range repeats the last one
+  // (its keys are not used).
   int ids = 0;
   auto fetch_ids = [&](int s0) __attribute__((always_inline)) {
     const int blk = b_lo + (s0 + lane) * kWaves + wave;
-    ids = (s0 + lane < nsteps && blk < b_hi) ? blocks[blk] : 0;
-  };
-  auto load_ids = [&](int s0) __attribute__((always_inline)) {
-    fetch_ids(s0);
-    asm volatile("" : "+v"(ids));
+    if (s0 + lane < nsteps) ids = blocks[min(blk, b_hi - 1)];
   };
   if (nsteps > 0) fetch_ids(0);
+  __syncthreads();  // what the stage memory held before (the dispatch plan) has been read
+  if (!prologue()) return;
 
-  // zero scales in every stage, once every wave is past its last read of what the
-  // stages held before (the dispatch plan): a stage that no step writes (a block past
-  // the range) then feeds finite products; stages written by loads only ever hold arena
-  // scales, which are finite (the append writes no non-finite value). Every int8 and
-  // E4M3FN byte is a finite code, but E5M2 bytes with all exponent bits set are Inf/NaN,
-  // so there the codes are zeroed too.
-  __syncthreads();
-  for (int j = lane; j < NB * 32; j += kWave)
-    reinterpret_cast<float*>(lds + (j / 32) * kWaves * S::kBytes + wave * S::kBytes + S::kS)[j % 32] = 0.f;
-  if constexpr (KF == kE5M2) {
-    for (int j = lane; j < NB * 2 * D; j += kWave)
-      reinterpret_cast<uint4*>(lds + (j / (2 * D)) * kWaves * S::kBytes + wave * S::kBytes +
-                               S::kK)[j % (2 * D)] = uint4{0u, 0u, 0u, 0u};
-  }
-  __syncthreads();
-  if (!prologue()) {
-    wait_vmcnt<0>();
-    return;
-  }
-
-  // ---- this wave's columns: the query goes out, then the first steps' loads, before
-  // the query is quantized.
-  int lo[NT], hi[NT], ctok[NT], chead[NT];
-  bool cvalid[NT];
-  QueryColumn<QT, D> qraw[NT];
+  int lo[NT], hi[NT];
+  QueryTile<QT, D> qraw[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const ColumnInfo c = column_of((wave * NT + t) * 16 + r);
-    ctok[t] = c.tok;
-    chead[t] = c.head;
-    cvalid[t] = c.valid;
+    const ColumnInfo c = column_of((wave * NT + t) * 32 + (lane & 31));
     lo[t] = c.valid ? c.lo : INT_MAX;
     hi[t] = c.valid ? c.hi : -1;
-    // an invalid column reads token t0's row (in range) and is zeroed when quantized
-    const QT* qp = static_cast<const QT*>(a.q) + (int64_t)(q0 + (c.valid ? c.tok : t0)) * a.q_tok +
-                   (int64_t)c.head * a.q_head + 16 * qg;
-    load_query_column<QT, D>(qp, qraw[t]);
+    // an invalid column reads token t0's row (in range) and is zeroed
+    load_query_tile<QT, D>(static_cast<const QT*>(a.q) + (int64_t)(q0 + (c.valid ? c.tok : t0)) * a.q_tok +
+                               (int64_t)c.head * a.q_head + 8 * (lane >> 5), qraw[t]);
   }
 
-  // ---- key steps: block b_lo + 4*step + w is staged by wave w. Lane i of `ids`
-  // holds the id for step (i + 64*k); reloaded every 64 steps.
   bool bad_index = false, bad_score = false;
   const bool masks = a.cache.key_valid != nullptr;  // the arena has key padding bytes
-  auto issue = [&](int step, char* buf) __attribute__((always_inline)) -> bool {
-    if (b_lo + step * kWaves + wave >= b_hi) return false;
-    const int id = __builtin_amdgcn_readlane(ids, step % kWave);
+  RawBlock<D> raw;
+  auto load_step = [&](int step) __attribute__((always_inline)) {
+    if (step % kWave == 0 && step > 0) fetch_ids(step);
+    int id = __builtin_amdgcn_readlane(ids, step % kWave);
     if ((unsigned)id >= (unsigned)a.cache.num_blocks) {
       bad_index = true;
-      return false;
+      id = 0;
     }
-    stage_block<D>(a, id, kvh, lane, buf + wave * S::kBytes);
-    return true;
+    load_raw<D, QOp<QT, D>::kAhead>(a, id, kvh, lane, masks, raw);
   };
-  auto buffer = [&](int step) __attribute__((always_inline)) -> char* {
-    return lds + (step % NB) * kWaves * S::kBytes;
-  };
-  asm volatile("" : "+v"(ids));  // the first ids have landed
-  // bit (step % NB): this wave issued loads for that step (uniform over the wave)
-  uint32_t inflight = 0;
-  for (int j = 0; j < NB - 1 && j < nsteps; ++j)
-    if (issue(j, buffer(j))) inflight |= 1u << (j % NB);
+  if (QOp<QT, D>::kAhead && nsteps > 0) load_step(0);
 
-  QOp<D> qop[NT];
-  float cf[NT], cfe[NT];
+  QOp<QT, D> qop[NT];
+  float back[NT];
+  bool scaled = false;
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    if constexpr (KF == kInt8)
-      cf[t] = query_column_i8<QT, D>(qraw[t], cvalid[t], a.qk_scale_log2, qop[t].hi, qop[t].lo);
-    else
-      cf[t] = query_column_f16<QT, D>(qraw[t], cvalid[t], a.qk_scale_log2, qop[t].op);
-    cfe[t] = cf[t] > 0.f ? cf[t] : FLT_MIN;  // cf >= 0 or NaN (scale > 0)
+    back[t] = query_operand<QT, D>(qraw[t], hi[t] >= 0, qop[t]);
+    scaled |= __ballot(back[t] != 1.f) != 0;
   }
   const WaveBounds wb = bounds_of(wave);
   mark(2);
 
-  const ColumnRefs<NT> cols{q0, t0, ctok, chead, cvalid};
-  float4_t acc[NT][NPV + 1];  // [NPV]: row sums in row 0 (lanes qg = 0)
-  const _Float16 one = r == 0 ? (_Float16)1.f : (_Float16)0.f;
-  const half8_t ones = {one, one, one, one, one, one, one, one};  // A operand: row 0 all ones
-  float m[NT];
+  float16v_t acc[NT][kRowsN];
+  float m[NT], l[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
 #pragma unroll
-    for (int k = 0; k <= NPV; ++k) acc[t][k] = float4_t{0.f, 0.f, 0.f, 0.f};
-    m[t] = -FLT_MAX;  // finite start: fully masked blocks give exp2(-inf) = 0
+    for (int n = 0; n < kRowsN; ++n)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) acc[t][n][j] = 0.f;
+    m[t] = -FLT_MAX;
+    l[t] = 0.f;
   }
   // The PV accumulators are in units of 2^-ve: ve is the largest block exponent so far
-  // (0 unless a block's V scales need more, see convert_v); vlim is its scale limit.
+  // (0 unless a block's V scales need more, see convert_raw); vlim is its scale limit.
   int ve = 0;
   float vlim = 32768.f / format_max<KF>();
 
+  // steps [inner_lo, inner_hi) see every key of theirs with every valid column
+  const int keys0 = b_lo * kBlockTokens;
+  constexpr int kStepKeys = kWaves * kBlockTokens;
+  const int inner_lo = max(0, (wb.lo_max - keys0 + kStepKeys - 1) / kStepKeys);
+  const int inner_end = min(wb.hi_min, b_hi * kBlockTokens - 1) + 1 - keys0;
+  const int inner_hi = wb.any && inner_end > 0 ? inner_end / kStepKeys : 0;
+  if (nsteps > 0) {
+    if constexpr (!QOp<QT, D>::kAhead) load_step(0);
+    convert_raw<D, QOp<QT, D>::kAhead>(a, raw, L, 0, wave, lane, masks, ve, vlim);
+    if (nsteps > 1) load_step(1);
+    __syncthreads();
+  }
   for (int i = 0; i < nsteps; ++i) {
-    const int ahead = i + NB - 1;
-    if (ahead < nsteps) {
-      if (ahead % kWave == 0) load_ids(ahead);
-      // its buffer was last read in step i - 1 (barrier below)
-      if (issue(ahead, buffer(ahead))) inflight |= 1u << (ahead % NB);
-      else inflight &= ~(1u << (ahead % NB));
-    }
-    // wait for step i's loads; the later steps' loads stay in flight
-    int younger = 0;
-#pragma unroll
-    for (int k = 1; k < NB; ++k)
-      if (i + k < nsteps && (inflight >> ((i + k) % NB) & 1u)) ++younger;
-    if (younger >= 3) wait_vmcnt<3 * S::kLoads>();
-    else if (younger == 2) wait_vmcnt<2 * S::kLoads>();
-    else if (younger == 1) wait_vmcnt<S::kLoads>();
-    else wait_vmcnt<0>();
-    char* const cur = buffer(i);
-    // this wave's block of step i is in; its V operands go to the wave's slab (the
-    // previous step's readers are past the barrier that ended that step)
-    const int eb = convert_v<D>(cur + wave * S::kBytes, lane, wave % 2,
-                                reinterpret_cast<uint2*>(L.vt[wave / 2]), ve, vlim);
-    if (lane == 0) L.vexp[wave] = eb;
-    __syncthreads();  // every wave's block of step i has landed and been converted
-    // the step's block exponents (each at least ve): a larger one becomes the new ve
-    // (the PV tiles, not the row sums, scale by the exact 2^(ve_old - ve)); blocks
-    // converted below ve weigh their products by 2^(e_b - ve)
-    bool vmix = false;
+    const int buf = i & 1;
+    half8_t kop[D / 16];
+    if constexpr (QOp<QT, D>::kAhead) load_k_operands<D>(L, buf, 0, lane, kop);
+    // the step's block exponents (each at least ve at its conversion): a larger one
+    // becomes the new ve (the accumulators scale by the exact 2^(ve_old - ve)); blocks
+    // converted below it weigh their products by 2^(e_w - ve)
+    const int4_t fv = *reinterpret_cast<const int4_t*>(L.flags[buf]);
+    const int f0 = __builtin_amdgcn_readfirstlane(fv[0]), f1 = __builtin_amdgcn_readfirstlane(fv[1]);
+    const int f2 = __builtin_amdgcn_readfirstlane(fv[2]), f3 = __builtin_amdgcn_readfirstlane(fv[3]);
+    bool vmix = false, large = false;
     half4_t vf = {(_Float16)1.f, (_Float16)1.f, (_Float16)1.f, (_Float16)1.f};
-    {
-      const int4_t ev = *reinterpret_cast<const int4_t*>(L.vexp);
-      int e4[kWaves];
-#pragma unroll
-      for (int w = 0; w < kWaves; ++w) e4[w] = __builtin_amdgcn_readfirstlane(ev[w]);
+    if (__builtin_expect((f0 | f1 | f2 | f3 | ve) != 0, 0)) {
+      large = ((f0 | f1 | f2 | f3) & kLargeFlag) != 0;
+      const int e4[kWaves] = {f0 & (kLargeFlag - 1), f1 & (kLargeFlag - 1), f2 & (kLargeFlag - 1),
+                              f3 & (kLargeFlag - 1)};
       const int emax = max(max(e4[0], e4[1]), max(e4[2], e4[3]));
-      if (emax != ve) {
+      if (emax > ve) {
         const float down = ldexpf(1.f, ve - emax);
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-          for (int n = 0; n < NPV; ++n) acc[t][n] *= down;
+          for (int n = 0; n < kRowsN; ++n) acc[t][n] *= down;
         ve = emax;
         vlim = ldexpf(32768.f / format_max<KF>(), ve);
       }
-      vmix = e4[0] != ve || e4[1] != ve || e4[2] != ve || e4[3] != ve;
-      if (vmix) {
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) vf[w] = (_Float16)ldexpf(1.f, e4[w] - ve);
+      for (int w = 0; w < kWaves; ++w) {
+        vmix |= e4[w] != ve;
+        vf[w] = (_Float16)ldexpf(1.f, e4[w] - ve);
       }
     }
-    {
-      const int kb0 = (b_lo + i * kWaves) * kBlockTokens;
+    const int kb0 = (b_lo + i * kWaves) * kBlockTokens;
+    uint32_t use = 15, bounded = 0;
+    if (i < inner_lo || i >= inner_hi) {
       const int kend = b_hi * kBlockTokens;
-      uint32_t use = 0, bounded = 0;
+      use = 0;
 #pragma unroll
       for (int w = 0; w < kWaves; ++w) {
         const int kb = kb0 + w * kBlockTokens;
@@ -912,11 +830,25 @@ __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L
           use |= 1u << w;
         if (!(kb >= wb.lo_max && kb + kBlockTokens - 1 <= wb.hi_min)) bounded |= 1u << w;
       }
-      if (use != 0)
-        prefill_step<QT, D, NT>(cur, L.vt[0], use, bounded & use, masks, kb0, qop, cf, cfe, lo, hi,
-                                r, qg, ones, vf, acc, m, bad_score, a, cols);
+      bounded &= use;
     }
-    __syncthreads();  // step i's stage may be refilled
+    if (use != 0) {
+      prefill_half<QT, D, NT>(L, buf, 0, use & 3u, bounded & 3u, masks, scaled | large, kb0, kop,
+                              [&]() __attribute__((always_inline)) {
+                                load_k_operands<D>(L, buf, 1, lane, kop);
+                              },
+                              qop, back, lo, hi, lane, vmix, half2_t{vf[0], vf[1]}, acc, m, l,
+                              bad_score);
+      prefill_half<QT, D, NT>(L, buf, 1, use >> 2, bounded >> 2, masks, scaled | large, kb0 + 32,
+                              kop, []() {}, qop, back, lo, hi, lane, vmix, half2_t{vf[2], vf[3]},
+                              acc, m, l, bad_score);
+    }
+    if (i + 1 < nsteps) {
+      // the other buffer was last read in step i - 1, before the barrier that ended it
+      convert_raw<D, QOp<QT, D>::kAhead>(a, raw, L, buf ^ 1, wave, lane, masks, ve, vlim);
+      if (i + 2 < nsteps) load_step(i + 2);
+    }
+    __syncthreads();
     if (i == 0) mark(3);
   }
   mark(4);
@@ -925,33 +857,39 @@ __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L
 
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const float lt = __shfl(acc[t][NPV][0], r, kWave);  // row 0 of the sum tile: lane (0, r)
-    store(t, acc[t], m[t], lt, ve, ColumnInfo{ctok[t], chead[t], lo[t], hi[t], cvalid[t]});
+    // worked out again: kept through the steps it would cost registers (the empty asm hides
+    // that it is the same value)
+    int f = (wave * NT + t) * 32 + (lane_id() & 31);
+    asm volatile("" : "+v"(f));
+    store(t, acc[t], m[t], sum32(l[t]), ve, column_of(f));
   }
   mark(5);
 }
 
 template <typename QT, int D, int G>
-__global__ __launch_bounds__(256) void prefill_mfma_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256, PrefillShape<D>::kOccupancy) void prefill_mfma_kernel(AttnArgs a) {
   static_assert(D == 64 || D == 128 || D == 256, "head_dim");
   constexpr int NT = PrefillShape<D>::NT;
   constexpr int TQ = PrefillShape<D>::kCols / G;
-  constexpr int NPV = D / 16;
-  constexpr int VB = D / 16;
   static_assert(PrefillShape<D>::kCols % G == 0, "GQA group must divide the column tile");
 
-  __shared__ PrefillLds<D> L;
-  __shared__ int s_wsum[kWaves];
-  __shared__ int s_found[2];
+  // one struct, the operand buffers at its start: every LDS address of the key steps then
+  // has a constant offset
+  __shared__ struct {
+    PrefillLds<D> unit;
+    int wsum[kWaves], found[2];
+  } lds;
+  PrefillLds<D>& L = lds.unit;
+  int* const s_wsum = lds.wsum;
+  int* const s_found = lds.found;
 
   const int lane = threadIdx.x % kWave;
-  const int qg = lane >> 4;
   const int hkv = a.cache.num_kv_heads;
 
   // ---- 1. this workgroup's unit (uniform over the workgroup). The plan lives in the
-  // stage buffers until the first load.
-  static_assert(PlanTab::kInts * sizeof(int) <= sizeof(L.stages), "the dispatch plan fits the stages");
-  int* const tab = reinterpret_cast<int*>(L.stages);
+  // operand buffers until the first conversion.
+  static_assert(PlanTab::kInts * sizeof(int) <= sizeof(L.k), "the dispatch plan fits the buffers");
+  int* const tab = reinterpret_cast<int*>(L.k);
   int per_kv = 0;
   const int nrows = plan_rows(a, TQ, tab, s_wsum, per_kv);
   if (nrows < 0) per_kv = scan_tiles(a, TQ, -1, s_wsum, s_found);
@@ -1006,28 +944,28 @@ __global__ __launch_bounds__(256) void prefill_mfma_kernel(AttnArgs a) {
   };
   // key bounds over the wave's valid columns (positions grow with f)
   auto bounds_of = [&](int wave) __attribute__((always_inline)) -> WaveBounds {
-    const int tk_lo = t0 + (wave * NT * 16) / G;
-    const int tk_hi = min(t1 - 1, t0 + ((wave + 1) * NT * 16 - 1) / G);
+    const int tk_lo = t0 + (wave * NT * 32) / G;
+    const int tk_hi = min(t1 - 1, t0 + ((wave + 1) * NT * 32 - 1) / G);
     return WaveBounds{a.window > 0 ? max(0, pos0 + tk_lo - a.window + 1) : 0,
                       a.window > 0 ? max(0, pos0 + tk_hi - a.window + 1) : 0,
                       a.causal ? pos0 + tk_lo : ctx - 1, a.causal ? pos0 + tk_hi : ctx - 1,
                       tk_lo < t1};
   };
   // normalise and store (fully masked columns: l = 0, acc = 0 -> 0)
-  auto store = [&](int t, const float4_t (&acc)[NPV + 1], float, float lt, int ve,
+  auto store = [&](int, const float16v_t (&acc)[D / 32], float, float l, int ve,
                    const ColumnInfo& c) __attribute__((always_inline)) {
     if (!c.valid) return;
-    const float inv = ldexpf(1.f, ve) / fmaxf(lt, FLT_MIN);  // the PV tiles carry 2^-ve
-    QT* op = static_cast<QT*>(a.out) + (int64_t)(q0 + c.tok) * a.o_tok + (int64_t)c.head * a.o_head;
+    const float inv = ldexpf(1.f, ve) / fmaxf(l, FLT_MIN);  // the PV tiles carry 2^-ve
+    QT* op = static_cast<QT*>(a.out) + (int64_t)(q0 + c.tok) * a.o_tok + (int64_t)c.head * a.o_head +
+             D / 8 * (lane >> 5);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float v[VB];
-#pragma unroll
-      for (int k = 0; k < NPV; ++k) v[k] = acc[k][j] * inv;
-      store_run<QT, VB>(op + VB * (4 * qg + j), v);
+    for (int x = 0; x < 4; ++x) {
+      float v[D / 8];
+      acc_run<D>(acc, x, inv, v);
+      store_run<QT, D / 8>(op + D / 4 * x, v);
     }
   };
-  prefill_unit<QT, D, G>(a, L, kvh, span.b_lo, span.b_hi,
+  prefill_unit<QT, D>(a, L, kvh, span.b_lo, span.b_hi,
                          a.block_tables + (int64_t)seq * a.bt_stride, q0, t0, column_of,
                          bounds_of, store, []() { return true; }, [](int) {});
 }
@@ -1043,21 +981,25 @@ __global__ __launch_bounds__(256) void prefill_mfma_kernel(AttnArgs a) {
 constexpr int kTileWords = 8, kMemberWords = 3;
 
 template <typename QT, int D, int G>
-__global__ __launch_bounds__(256) void prefix_tiles_kernel(PlanArgs p) {
+__global__ __launch_bounds__(256, PrefillShape<D>::kOccupancy) void prefix_tiles_kernel(PlanArgs p) {
   static_assert(D == 64 || D == 128 || D == 256, "head_dim");
   constexpr int TQ = PrefillShape<D>::kCols / G;
-  constexpr int NPV = D / 16;
-  constexpr int VB = D / 16;
   static_assert(PrefillShape<D>::kCols % G == 0, "GQA group must divide the column tile");
   const AttnArgs& a = p.a;
 
-  __shared__ PrefillLds<D> L;
-  __shared__ int s_row[TQ];      // member j's query token row
-  __shared__ int s_slot[TQ];     // its chunk slot for this tile's kv head and range
-  __shared__ int s_bad;
+  // one struct, the operand buffers at its start: every LDS address of the key steps then
+  // has a constant offset
+  __shared__ struct {
+    PrefillLds<D> unit;
+    int row[TQ];   // member j's query token row
+    int slot[TQ];  // its chunk slot for this tile's kv head and range
+    int ctx[QOp<QT, D>::kAhead ? 1 : TQ];  // its length (fp32 queries leave no register for it)
+    int bad;
+  } lds;
+  PrefillLds<D>& L = lds.unit;
 
   const int lane = threadIdx.x % kWave;
-  const int qg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int hkv = a.cache.num_kv_heads;
   long long tm[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // trace marks (kTrace)
   if constexpr (kTrace) tm[0] = wall_clock64();
@@ -1078,7 +1020,7 @@ __global__ __launch_bounds__(256) void prefix_tiles_kernel(PlanArgs p) {
     if (threadIdx.x == 0) atomicOr(a.err_flag, ASTR_FLAG_BAD_INDEX);
     return;  // the whole workgroup (every thread read the same record)
   }
-  if (threadIdx.x == 0) s_bad = 0;  // ordered before the prologue by the unit's barriers
+  if (threadIdx.x == 0) lds.bad = 0;  // ordered before the prologue by the unit's barriers
   int mctx = 0;  // thread j < n: member j's context length, checked after the unit
   auto prologue = [&]() __attribute__((always_inline)) -> bool {
     if ((int)threadIdx.x < n) {
@@ -1086,95 +1028,102 @@ __global__ __launch_bounds__(256) void prefix_tiles_kernel(PlanArgs p) {
       const int seq = mem[0], c0 = mem[1], span = mem[2];
       if (!(seq >= 0 && seq < a.num_seqs && c0 >= 0 && span > range &&
             (int64_t)c0 + (int64_t)hkv * span <= p.info.num_chunks)) {
-        s_bad = 1;
+        lds.bad = 1;
       } else {
-        s_row[threadIdx.x] = seq;  // decode rows: sequence s's query token is row s
-        s_slot[threadIdx.x] = c0 + kvh * span + range;
+        lds.row[threadIdx.x] = seq;  // decode rows: sequence s's query token is row s
+        lds.slot[threadIdx.x] = c0 + kvh * span + range;
         mctx = a.context_lens[seq];  // its wait falls after the key steps
+        if constexpr (!QOp<QT, D>::kAhead) lds.ctx[threadIdx.x] = mctx;
       }
     }
     __syncthreads();
     if constexpr (kTrace) tm[1] = wall_clock64();
-    return __builtin_amdgcn_readfirstlane(s_bad) == 0;
+    return __builtin_amdgcn_readfirstlane(lds.bad) == 0;
   };
 
   // an invalid column reads member 0's query row (and is zeroed when quantized)
   auto column_of = [&](int f) __attribute__((always_inline)) -> ColumnInfo {
     const int j = f / G;
-    return ColumnInfo{s_row[j < n ? j : 0], kvh * G + f % G, 0, INT_MAX, j < n};
+    return ColumnInfo{lds.row[j < n ? j : 0], kvh * G + f % G, 0, INT_MAX, j < n};
   };
   // every key of the range is visible to every column: no step is bounded
   auto bounds_of = [&](int wave) __attribute__((always_inline)) -> WaveBounds {
-    return WaveBounds{0, 0, INT_MAX, INT_MAX, (wave * PrefillShape<D>::NT * 16) / G < n};
+    return WaveBounds{0, 0, INT_MAX, INT_MAX, (wave * PrefillShape<D>::NT * 32) / G < n};
   };
   // the partial of column (member j, head g): m, l and acc into the member's chunk
   // slot, head g, with acc and l in the decode kernels' units (both times norm_scale,
-  // as the decode partials they merge with). Lane (qg, r) holds elements
-  // [D/4 qg, D/4 (qg + 1)) of column r: written as they are, every store instruction
-  // would touch 64 cache lines. The tile goes through the wave's share of the stage
-  // buffers (free after the last key step's barrier) instead, and each store
-  // instruction then writes 1 KB of whole columns (4 to 16 cache lines).
+  // as the decode partials they merge with). A lane holds 64-byte runs of its column: the
+  // columns go through the wave's share of the operand buffers (free after the last key
+  // step's barrier), 16 at a time, and each store instruction then writes 1 KB of whole
+  // columns.
   constexpr int kRow = D + 4;  // floats per staged column (padded against bank conflicts)
-  static_assert(kWaves * 16 * kRow * (int)sizeof(float) <= (int)sizeof(L.stages),
-                "a wave's column tile fits its share of the stages");
-  auto store = [&](int t, const float4_t (&acc)[NPV + 1], float m, float lt, int ve,
+  static_assert(kWaves * 16 * kRow * sizeof(float) <= sizeof(L.k) + sizeof(L.v) &&
+                    offsetof(PrefillLds<D>, v) == sizeof(L.k),
+                "a wave's half tile fits its share of the buffers");
+  auto store = [&](int t, const float16v_t (&acc)[D / 32], float m, float l, int ve,
                    const ColumnInfo& c) __attribute__((always_inline)) {
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int f0 = (wave * PrefillShape<D>::NT + t) * 16;  // the tile's first column
-    float* const tile = reinterpret_cast<float*>(L.stages) + wave * 16 * kRow;
+    const int f0 = (wave * PrefillShape<D>::NT + t) * 32;  // the tile's first column
+    float* const tile = reinterpret_cast<float*>(&L) + wave * 16 * kRow;
     const float up = ldexpf(norm_scale<KF>(), ve);  // the PV tiles carry 2^-ve
-    __builtin_amdgcn_wave_barrier();  // after the previous tile's reads of this share
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float v[VB];
+    for (int half = 0; half < 2; ++half) {
+      __builtin_amdgcn_wave_barrier();  // after the previous half's reads of this share
+      if (((lane >> 4) & 1) == half) {
 #pragma unroll
-      for (int k = 0; k < NPV; ++k) v[k] = acc[k][j] * up;
+        for (int x = 0; x < 4; ++x) {
+          float v[D / 8];
+          acc_run<D>(acc, x, up, v);
 #pragma unroll
-      for (int k = 0; k < VB / 4; ++k)
-        *reinterpret_cast<float4_t*>(tile + (lane & 15) * kRow + VB * (4 * qg + j) + 4 * k) =
-            float4_t{v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]};
-    }
-    __builtin_amdgcn_wave_barrier();  // a wave's LDS accesses complete in issue order
+          for (int k = 0; k < D / 32; ++k)
+            *reinterpret_cast<float4_t*>(tile + (lane & 15) * kRow + D / 4 * x + D / 8 * (lane >> 5) +
+                                         4 * k) =
+                float4_t{v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]};
+        }
+      }
+      __builtin_amdgcn_wave_barrier();  // a wave's LDS accesses complete in issue order
 #pragma unroll
-    for (int i = 0; i < D / 16; ++i) {
-      const int e = i * kWave + lane;  // float4 e of the tile: column e / (D/4)
-      const int cc = e / (D / 4), q = e % (D / 4);
-      const int f = f0 + cc;
-      const float4_t v = *reinterpret_cast<const float4_t*>(tile + cc * kRow + 4 * q);
-      if (f / G < n) {
-        // non-temporal: the decode kernel reads the partials only after streaming the
-        // rows' own blocks, long after they would have left the cache, and dirty lines
-        // left in the cache are written back at this kernel's end (measured: config 4's
-        // call 69.2 -> 68.6 us)
-        const int64_t col = plan_chunk_slot(p, s_slot[f / G], G) + f % G;
-        __builtin_nontemporal_store(v, reinterpret_cast<float4_t*>(a.ws_o + col * D + 4 * q));
+      for (int i = 0; i < D / 16; ++i) {
+        const int e = i * kWave + lane;  // float4 e of the half tile: column e / (D/4)
+        const int cc = e / (D / 4), q = e % (D / 4);
+        const int f = f0 + 16 * half + cc;
+        const float4_t v = *reinterpret_cast<const float4_t*>(tile + cc * kRow + 4 * q);
+        if (f / G < n) {
+          // non-temporal: the decode kernel reads the partials only after streaming the
+          // rows' own blocks, long after they would have left the cache, and dirty lines
+          // left in the cache are written back at this kernel's end (measured: config 4's
+          // call 69.2 -> 68.6 us)
+          const int64_t col = plan_chunk_slot(p, lds.slot[f / G], G) + f % G;
+          __builtin_nontemporal_store(v, reinterpret_cast<float4_t*>(a.ws_o + col * D + 4 * q));
+        }
       }
     }
-    if (c.valid && qg == 0) {
-      const int f = f0 + (lane & 15);
-      const int64_t col = plan_chunk_slot(p, s_slot[f / G], G) + f % G;
+    if (c.valid && lane < 32) {
+      const int f = f0 + lane;
+      const int64_t col = plan_chunk_slot(p, lds.slot[f / G], G) + f % G;
       a.ws_ml[col * 2] = m;
-      a.ws_ml[col * 2 + 1] = lt * norm_scale<KF>();
+      a.ws_ml[col * 2 + 1] = l * norm_scale<KF>();
     }
   };
   const int32_t* ids = p.plan + p.info.off_ids + ids_off - blk0;  // id of block b at ids[b]
   auto mark = [&](int k) __attribute__((always_inline)) {
     if constexpr (kTrace) tm[k] = wall_clock64();
   };
-  prefill_unit<QT, D, G>(a, L, kvh, blk0, blk0 + nblk, ids, 0, 0, column_of, bounds_of, store,
+  prefill_unit<QT, D>(a, L, kvh, blk0, blk0 + nblk, ids, 0, 0, column_of, bounds_of, store,
                          prologue, mark);
-  if (s_bad) {  // a member failed its checks: nothing was stored
-    if (threadIdx.x == 0) atomicOr(a.err_flag, ASTR_FLAG_BAD_INDEX);
+  const int tid = wave * kWave + lane_id();
+  if (lds.bad) {  // a member failed its checks: nothing was stored
+    if (tid == 0) atomicOr(a.err_flag, ASTR_FLAG_BAD_INDEX);
     return;
   }
   // every key of the range must be visible to each member (its length as planned)
-  if ((int)threadIdx.x < n) {
+  if (tid < n) {
+    if constexpr (!QOp<QT, D>::kAhead) mctx = lds.ctx[tid];
     const RowSpan sp = row_span(a, mctx);
     if (sp.kv_begin > blk0 * kBlockTokens || (int64_t)sp.ctx < (int64_t)(blk0 + nblk) * kBlockTokens)
       atomicOr(a.err_flag, ASTR_FLAG_BAD_INDEX);
   }
 #if ASTR_TRACE
-  const int64_t tw = unit * kWaves + threadIdx.x / kWave;
+  const int64_t tw = unit * kWaves + wave;
   if (lane == 0 && tw < kTileTraceWaves) {
     for (int k = 0; k < 8; ++k) g_ttrace[tw][k] = tm[k];
     g_ttrace_info[tw][0] = (nblk + kWaves - 1) / kWaves;

@@ -1,0 +1,111 @@
+"""The chunked-prefill kernel against the float64 oracle where its tiles can go wrong: chunk
+lengths around the 128-column tile and the 32-key half steps, histories that end inside a
+block, columns scaled out of f16's range, key factors past the safe range of scores, V
+scales of very different exponents in one step, and id windows past 64 steps."""
+
+import numpy as np
+import pytest
+import torch
+
+from aster_amd import KVQuantization, PagedKVCache
+from tests.gpu_util import oracle_decode
+
+pytestmark = pytest.mark.gpu
+
+
+def _cache(device, rows, dim, kv, fmt, seed):
+    """Random codes and scales under shuffled tables for contexts ``rows``."""
+    gen = torch.Generator(device=device).manual_seed(seed)
+    pages = [-(-n // 16) for n in rows]
+    perm = np.random.default_rng(seed).permutation(sum(pages) + 2).astype(np.int32)
+    tables = np.zeros((len(rows), max(pages)), np.int32)
+    at = 0
+    for row, n in enumerate(pages):
+        tables[row, :n] = perm[at:at + n]
+        at += n
+    cache = PagedKVCache(num_blocks=len(perm), num_layers=1, num_kv_heads=kv, head_dim=dim,
+                         device=device, quantization=KVQuantization(fmt))
+    x = torch.randn(cache.codes.shape, generator=gen, device=device)
+    most = {"int8": 127.0, "fp8_e4m3fn": 448.0, "fp8_e5m2": 57344.0}[fmt]
+    amax = x.abs().amax(-1)
+    units = x / amax[..., None] * most
+    codes = units.round() if fmt == "int8" else units
+    cache.codes.copy_(codes.to(cache.quantization.dtype).view(torch.int8))
+    cache.scales.copy_(amax / most)
+    return cache, tables, gen
+
+
+def _check(cache, tables, lens, counts, query, window=None, atol=2e-3, rtol=2e-3):
+    device = query.device
+    starts = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    out = cache.paged_attention(0, query, torch.from_numpy(tables).to(device),
+                                torch.from_numpy(np.array(lens, np.int32)).to(device),
+                                max_context_len=max(lens), window=window,
+                                query_start_loc=torch.from_numpy(starts).to(device),
+                                max_query_len=max(counts), check=True)
+    want = oracle_decode(tables, cache, query, context_lens=np.array(lens, np.int32),
+                         scale=cache.head_dim ** -0.5, window=window,
+                         query_lens=np.array(counts, np.int32), fp64=True)
+    bf16 = query.dtype == torch.bfloat16  # outputs rounded to 2^-9 of themselves
+    np.testing.assert_allclose(out.float().cpu().numpy(), want, atol=atol,
+                               rtol=5e-3 if bf16 else rtol)
+
+
+@pytest.mark.parametrize("fmt", ["int8", "fp8_e4m3fn", "fp8_e5m2"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dim,kv,group", [(64, 2, 4), (128, 2, 1), (128, 1, 16), (256, 2, 2)])
+def test_tile_edges(device, dim, kv, group, dtype, fmt):
+    tile = 128 // group
+    counts = [2, tile - 1 if tile > 2 else 3, tile, tile + 1, 2 * tile + 5]
+    priors = [0, 31, 32, 33, 64]
+    lens = [n + p for n, p in zip(counts, priors)]
+    cache, tables, gen = _cache(device, lens, dim, kv, fmt, dim + group)
+    query = torch.randn((sum(counts), kv * group, dim), generator=gen, device=device).to(dtype)
+    _check(cache, tables, lens, counts, query)
+    _check(cache, tables, lens, counts, query, window=37)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("power", [-40, -14, -9, 13])
+def test_scaled_columns(device, dtype, power):
+    """Queries whose columns leave the unscaled range, one head in two; the scale keeps
+    the scores ordinary."""
+    if dtype == torch.float16 and power not in (-9, 13):
+        pytest.skip("outside fp16")
+    lens, counts = [100, 50], [40, 17]
+    cache, tables, gen = _cache(device, lens, 128, 2, "int8", 7)
+    query = torch.randn((sum(counts), 8, 128), generator=gen, device=device)
+    query[:, ::2] *= 2.0 ** power
+    if power > 0:  # scores stay within exp's range
+        cache.scales[:, :, 0] *= 2.0 ** -power
+    _check(cache, tables, lens, counts, query.to(dtype))
+
+
+@pytest.mark.parametrize("fmt", ["int8", "fp8_e4m3fn", "fp8_e5m2"])
+def test_large_scales(device, fmt):
+    """V scales up to 2^20 larger in some blocks, alone and beside ordinary ones: the
+    tolerance scales with the largest values (the weights' f16 rounding)."""
+    lens, counts = [300, 90], [70, 33]
+    cache, tables, gen = _cache(device, lens, 128, 2, fmt, 11)
+    cache.scales[::3, :, 1] *= 2.0 ** 20
+    cache.scales[1::6, :, 1] *= 2.0 ** 11
+    query = torch.randn((sum(counts), 8, 128), generator=gen, device=device).half().float()
+    _check(cache, tables, lens, counts, query, atol=2.0 ** 20 * 2e-3)
+
+
+def test_overflowing_scores_raise(device):
+    lens, counts = [80], [40]
+    cache, tables, gen = _cache(device, lens, 128, 1, "int8", 3)
+    cache.scales[int(tables[0, 1]), 0, 0] = 3e37
+    query = 1e3 * torch.randn((40, 4, 128), generator=gen, device=device)
+    with pytest.raises(ValueError, match="overflow"):
+        _check(cache, tables, lens, counts, query)
+
+
+def test_long_history(device):
+    """More than 64 key steps (the block ids are fetched 64 steps at a time)."""
+    lens, counts = [64 * 64 * 2 + 77], [9]
+    cache, tables, gen = _cache(device, lens, 64, 1, "int8", 5)
+    query = torch.randn((9, 2, 64), generator=gen, device=device).half()
+    _check(cache, tables, lens, counts, query)
+    _check(cache, tables, lens, counts, query, window=5000)
