@@ -99,6 +99,15 @@ struct AttnArgs {
   const void* new_v;
   int64_t nk_tok, nk_head, nv_tok, nv_head;
   const int64_t* new_slots;
+  // chunked prefill: the fewest query tokens of a row it takes (2; 1 where no decode launch
+  // precedes it), and the key split of its units, settled by the launcher: units of more
+  // than pf_steps key steps run as up to pf_pieces pieces that leave partials in pf_ws
+  // (pf_bytes long), for a merge launch
+  int32_t pf_min_rows, pf_pieces, pf_steps;
+  int32_t pf_cus;       // compute units per XCD
+  int32_t max_context;  // host bound of context_lens
+  float* pf_ws;
+  size_t pf_bytes;
   int32_t* err_flag;
 };
 

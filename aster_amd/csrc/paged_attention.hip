@@ -146,6 +146,24 @@ namespace astr {
 namespace attn {
 namespace {
 
+// Whether a mixed call goes to the prefill kernel alone, one-token rows included. The
+// decode and merge launches cost 4.6 us each also where they find no row (they read that
+// from device memory):
+//   - every row must carry max_query_len tokens where the call has num_seqs times as many
+//     (a prompt alone, equal chunks); an offset array that says otherwise is served all
+//     the same;
+//   - contexts up to 512 keys are at most 8 key steps of ~2 us for a one-token row, which
+//     runs beside the chunks' units, no longer than the launches it replaces, while every
+//     row has a CU of its own. Not for fp32 queries, whose one-token rows are attended in
+//     exact fp32.
+constexpr int kOnlyChunksContext = 512;
+bool only_chunks(int32_t q_dtype, int32_t tokens, int32_t max_query_len, int32_t num_seqs,
+                 int32_t num_kv_heads, int32_t max_context_len) {
+  if ((int64_t)num_seqs * max_query_len == tokens) return true;
+  return q_dtype != ASTR_F32 && max_context_len <= kOnlyChunksContext &&
+         (int64_t)num_seqs * num_kv_heads <= device_cus();
+}
+
 size_t required_workspace(int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
                           int32_t head_dim, int32_t max_context_len, int32_t partition_tokens,
                        int32_t num_packs, int32_t pack_rows) {
@@ -340,8 +358,20 @@ int paged_attention(const astr_paged_kv* cache, const void* query, int32_t q_dty
   a.stats = stats;
   a.err_flag = err_flag;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool chunks = query_start_loc != nullptr && max_query_len >= 2;
+  // The prefill launch reuses the workspace: the decode launches before it on the stream
+  // have merged what they left there.
+  a.pf_min_rows = 2;
+  a.max_context = max_context_len;
+  a.pf_ws = static_cast<float*>(workspace);
+  a.pf_bytes = fixed_scratch || need == 0 ? 0 : need;
+  if (chunks && only_chunks(q_dtype, num_query_tokens, max_query_len, num_seqs,
+                            cache->num_kv_heads, max_context_len)) {
+    a.pf_min_rows = 1;
+    return launch_prefill(a, q_dtype, s);
+  }
   const int rc = streamk ? launch_streamk(a, q_dtype, s) : launch_partitioned(a, q_dtype, s);
-  if (rc != 0 || query_start_loc == nullptr || max_query_len < 2) return rc;
+  if (rc != 0 || !chunks) return rc;
   return launch_prefill(a, q_dtype, s);
 }
 

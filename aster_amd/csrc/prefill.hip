@@ -24,6 +24,7 @@
 // and the linear workgroup id is remapped so that each XCD (workgroups are dealt
 // to the 8 XCDs round robin) runs one contiguous range of units: the tiles
 // sharing a sequence's K/V then share that XCD's L2.
+#include <algorithm>
 #include <climits>
 #include <cstddef>
 #include <type_traits>
@@ -61,8 +62,15 @@ template <int D>
 struct PrefillShape {
   static constexpr int NT = 1;                    // 32-column MFMA tiles per wave
   static constexpr int kCols = kWaves * 32 * NT;  // (token, head) columns per workgroup
-  static constexpr int kOccupancy = D == 256 ? 1 : 2;  // workgroups per CU (LDS: 130 KB at 256)
 };
+
+// Workgroups per CU: the LDS holds one at head dim 256 (130 KB), the registers two at 128
+// and, with 16-bit queries, three at 64 (four, 128 registers each, spill: 91.3 against
+// 76.8 us for ragged FP8 prompts with their append).
+template <typename QT, int D>
+constexpr int prefill_occupancy() {
+  return D == 256 ? 1 : D == 64 && sizeof(QT) == 2 ? 3 : 2;
+}
 
 // Keys visible to query tile `tile` (tokens [t0, t1) of the sequence's n query tokens,
 // context ctx): positions [lo, hi], blocks [b_lo, b_hi).
@@ -87,12 +95,12 @@ constexpr int kOrderMax = 256;  // chunk rows ordered longest first; beyond this
 __device__ __forceinline__ int query_tiles(const AttnArgs& a, int s, int tq) {
   int begin;
   const int n = seq_queries(a, s, begin);
-  return n > 1 ? (n + tq - 1) / tq : 0;
+  return n >= a.pf_min_rows ? (n + tq - 1) / tq : 0;
 }
 
 // The dispatch plan, from one round of loads of the offsets and context lengths, in
-// the LDS table `tab` (PlanTab::kInts ints): the chunk rows (sequences with more than
-// one query token) with their sequence, query offset, query count and context length
+// the LDS table `tab` (PlanTab::kInts ints): the chunk rows (sequences with at least
+// pf_min_rows query tokens) with their sequence, query offset, query count and context length
 // as loaded, and the rows in dispatch order, longest first (key: key blocks of the
 // row's last tile, which sees the most keys; ties by index), with the inclusive prefix
 // of their tile counts in that order. Returns the number of rows and the total tile
@@ -116,7 +124,7 @@ __device__ int plan_rows(const AttnArgs& a, int tq, int* tab, int* s_wsum, int& 
     int key = -1, tiles = 0, q0 = 0, n = 0, ctx_raw = 0;
     if (s < a.num_seqs) {
       n = seq_queries(a, s, q0);
-      if (n > 1) {
+      if (n >= a.pf_min_rows) {
         ctx_raw = a.context_lens[s];
         const TileSpan sp = tile_span(a, clamp_ctx(a, ctx_raw, false), n, (n - 1) / tq, tq);
         key = sp.b_hi - sp.b_lo;
@@ -221,8 +229,11 @@ __device__ __forceinline__ float sum32(float x) {
 }
 
 // The lane's index, from the lane mask: no register holds it through the key steps.
+// (as an asm, so that the compiler does not work it out ahead and keep it after all)
 __device__ __forceinline__ int lane_id() {
-  return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+  int lane;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+  return lane;
 }
 
 // Query operands of one 32-column tile: B operands of the 16-wide d chunks (lane (c, h):
@@ -232,8 +243,9 @@ template <typename QT, int D>
 struct QOp {
   static constexpr int kTerms = sizeof(QT) == 4 ? 2 : 1;
   // whether the registers hold key-step operands ahead of their use beside the query's (two
-  // terms at head dim 128 and 256 leave none)
-  static constexpr bool kAhead = !(kTerms == 2 && D >= 128);
+  // terms at head dim 128 and 256 leave none; at head dim 64 a third wave per SIMD is worth
+  // more, ragged FP8 prompts 83.9 -> 76.8 us)
+  static constexpr bool kAhead = kTerms == 1 && D >= 128;
   half8_t op[kTerms][D / 16];
 };
 
@@ -693,7 +705,7 @@ __device__ __forceinline__ void acc_run(const float16v_t (&acc)[D / 32], int x, 
 // workgroup's query columns (column_of(f), bounds_of(wave)), through the key steps
 // described at the top of this file; store(t, acc, m, l, ve, col) then takes column
 // tile t of each wave (acc in units of 2^-ve, l the sums of the column's weights).
-// prologue() runs (in uniform control flow) once the first block ids are on their way,
+// prologue() runs (in uniform control flow) once the first block id is on its way,
 // before any column is read: it returns false (uniformly) to end the unit there, with
 // nothing stored. mark(k) is called at the unit's timeline marks 2-5 (the tile kernel's
 // trace builds).
@@ -709,15 +721,14 @@ __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L
   const int lane = threadIdx.x % kWave;
   const int nsteps = (b_hi - b_lo + kWaves - 1) / kWaves;
 
-  // Block b_lo + 4 * step + w is wave w's. Lane i of `ids` holds the id for step
-  // i + 64 * k; reloaded every 64 steps. A block past the range repeats the last one
-  // (its keys are not used).
-  int ids = 0;
-  auto fetch_ids = [&](int s0) __attribute__((always_inline)) {
-    const int blk = b_lo + (s0 + lane) * kWaves + wave;
-    if (s0 + lane < nsteps) ids = blocks[min(blk, b_hi - 1)];
+  // Block b_lo + 4 * step + w is wave w's; its id is read (a scalar load) one step before
+  // its block. A block past the range repeats the last one (its keys are not used).
+  typedef const __attribute__((address_space(4))) int32_t* scalar_ids_t;
+  const scalar_ids_t sids = (scalar_ids_t)blocks;
+  auto id_of = [&](int step) __attribute__((always_inline)) -> int {
+    return sids[min(b_lo + step * kWaves + wave, b_hi - 1)];
   };
-  if (nsteps > 0) fetch_ids(0);
+  int next_id = nsteps > 0 ? id_of(0) : 0;
   __syncthreads();  // what the stage memory held before (the dispatch plan) has been read
   if (!prologue()) return;
 
@@ -737,8 +748,8 @@ __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L
   const bool masks = a.cache.key_valid != nullptr;  // the arena has key padding bytes
   RawBlock<D> raw;
   auto load_step = [&](int step) __attribute__((always_inline)) {
-    if (step % kWave == 0 && step > 0) fetch_ids(step);
-    int id = __builtin_amdgcn_readlane(ids, step % kWave);
+    int id = next_id;
+    if (step + 1 < nsteps) next_id = id_of(step + 1);
     if ((unsigned)id >= (unsigned)a.cache.num_blocks) {
       bad_index = true;
       id = 0;
@@ -866,8 +877,85 @@ __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L
   mark(5);
 }
 
+// A unit of the prefill launch: query tile `tile` of sequence `seq`.
+struct UnitRef {
+  int seq, tile, q0, n, ctx_raw;
+  bool last;  // the sequence's last tile
+};
+
+// Units of one kv head, from the dispatch plan (in `tab` when rows >= 0) or the scan in
+// index order beyond kOrderMax rows. Every thread calls both.
+__device__ __forceinline__ int count_units(const AttnArgs& a, int tq, int* tab, int* s_wsum,
+                                           int* s_found, int& rows) {
+  int per_kv = 0;
+  rows = plan_rows(a, tq, tab, s_wsum, per_kv);
+  if (rows < 0) per_kv = scan_tiles(a, tq, -1, s_wsum, s_found);
+  return per_kv;
+}
+__device__ __forceinline__ bool unit_ref(const AttnArgs& a, int tq, int* tab, int* s_wsum,
+                                         int* s_found, int rows, int unit, UnitRef& u) {
+  int within;
+  if (rows >= 0) {
+    // the first row whose inclusive prefix exceeds the unit (prefixes strictly grow)
+    const int* const o_incl = PlanTab::at(tab, PlanTab::kIncl);
+    int lo_r = 0, hi_r = rows - 1;
+    while (lo_r < hi_r) {
+      const int mid = (lo_r + hi_r) / 2;
+      if (o_incl[mid] > unit) hi_r = mid;
+      else lo_r = mid + 1;
+    }
+    // uniform values read from LDS: readfirstlane keeps them (and all they derive) scalar
+    const int row = __builtin_amdgcn_readfirstlane(PlanTab::at(tab, PlanTab::kOrder)[lo_r]);
+    within = __builtin_amdgcn_readfirstlane(unit - (lo_r > 0 ? o_incl[lo_r - 1] : 0));
+    u.seq = __builtin_amdgcn_readfirstlane(PlanTab::at(tab, PlanTab::kSeq)[row]);
+    u.q0 = __builtin_amdgcn_readfirstlane(PlanTab::at(tab, PlanTab::kQ0)[row]);
+    u.n = __builtin_amdgcn_readfirstlane(PlanTab::at(tab, PlanTab::kN)[row]);
+    u.ctx_raw = __builtin_amdgcn_readfirstlane(PlanTab::at(tab, PlanTab::kCtx)[row]);
+  } else {
+    if (threadIdx.x == 0) s_found[0] = -1;  // ordered before the scan's writes by its barriers
+    scan_tiles(a, tq, unit, s_wsum, s_found);
+    u.seq = __builtin_amdgcn_readfirstlane(s_found[0]);
+    within = __builtin_amdgcn_readfirstlane(s_found[1]);
+    if (u.seq < 0) return false;  // unreachable for unit < per_kv; keeps every index in range
+    u.n = seq_queries(a, u.seq, u.q0);
+    u.ctx_raw = a.context_lens[u.seq];
+  }
+  const int tiles = (u.n + tq - 1) / tq;
+  u.tile = tiles - 1 - within;  // latest (longest) tiles first
+  u.last = within == 0;
+  return true;
+}
+
+// The partial of one piece of a split unit: the accumulators as the lanes hold them
+// (float4 x of operand n of wave w at ((w * D / 32 + n) * 4 + x) * 64 + lane), then (m, l)
+// per column.
+template <int D>
+struct PiecePartial {
+  static constexpr int kAcc = kWaves * (D / 32) * 4 * kWave * 4;  // floats
+  static constexpr int kFloats = kAcc + PrefillShape<D>::kCols * 2;
+  static_assert(PrefillShape<D>::NT == 1, "one column tile per wave");
+  __device__ static float4_t* acc(float* base, int wave, int n, int x, int lane) {
+    return reinterpret_cast<float4_t*>(base) + ((wave * (D / 32) + n) * 4 + x) * kWave + lane;
+  }
+};
+
+// The outputs of one column of each lane pair, normalised (fully masked columns: l = 0,
+// acc = 0 -> 0).
+template <typename QT, int D>
+__device__ __forceinline__ void store_column(const AttnArgs& a, const float16v_t (&acc)[D / 32],
+                                             float inv, int token, int head, int lane) {
+  QT* op = static_cast<QT*>(a.out) + (int64_t)token * a.o_tok + (int64_t)head * a.o_head +
+           D / 8 * (lane >> 5);
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    float v[D / 8];
+    acc_run<D>(acc, x, inv, v);
+    store_run<QT, D / 8>(op + D / 4 * x, v);
+  }
+}
+
 template <typename QT, int D, int G>
-__global__ __launch_bounds__(256, PrefillShape<D>::kOccupancy) void prefill_mfma_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256, (prefill_occupancy<QT, D>())) void prefill_mfma_kernel(AttnArgs a) {
   static_assert(D == 64 || D == 128 || D == 256, "head_dim");
   constexpr int NT = PrefillShape<D>::NT;
   constexpr int TQ = PrefillShape<D>::kCols / G;
@@ -880,60 +968,59 @@ __global__ __launch_bounds__(256, PrefillShape<D>::kOccupancy) void prefill_mfma
     int wsum[kWaves], found[2];
   } lds;
   PrefillLds<D>& L = lds.unit;
-  int* const s_wsum = lds.wsum;
-  int* const s_found = lds.found;
 
-  const int lane = threadIdx.x % kWave;
+  const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int hkv = a.cache.num_kv_heads;
 
   // ---- 1. this workgroup's unit (uniform over the workgroup). The plan lives in the
   // operand buffers until the first conversion.
   static_assert(PlanTab::kInts * sizeof(int) <= sizeof(L.k), "the dispatch plan fits the buffers");
   int* const tab = reinterpret_cast<int*>(L.k);
-  int per_kv = 0;
-  const int nrows = plan_rows(a, TQ, tab, s_wsum, per_kv);
-  if (nrows < 0) per_kv = scan_tiles(a, TQ, -1, s_wsum, s_found);
-  const int64_t units = (int64_t)per_kv * hkv;
+  int rows;
+  const int per_kv = count_units(a, TQ, tab, lds.wsum, lds.found, rows);
+  const int64_t units = (int64_t)per_kv * hkv * a.pf_pieces;
   const int64_t per_xcd = (units + kXcds - 1) / kXcds;
-  const int64_t slot = blockIdx.x / kXcds;
-  const int64_t logical = (int64_t)(blockIdx.x % kXcds) * per_xcd + slot;
-  if (slot >= per_xcd || logical >= units) return;
-  const int kvh = (int)(logical / per_kv);
-  const int unit = (int)(logical % per_kv);
-  int seq, within, q0, n, ctx_raw;
-  if (nrows >= 0) {
-    // the first row whose inclusive prefix exceeds the unit (prefixes strictly grow)
-    const int* const o_incl = PlanTab::at(tab, PlanTab::kIncl);
-    int lo_r = 0, hi_r = nrows - 1;
-    while (lo_r < hi_r) {
-      const int mid = (lo_r + hi_r) / 2;
-      if (o_incl[mid] > unit) hi_r = mid;
-      else lo_r = mid + 1;
-    }
-    // uniform values read from LDS: readfirstlane keeps them (and all they derive) scalar
-    const int row = __builtin_amdgcn_readfirstlane(PlanTab::at(tab, PlanTab::kOrder)[lo_r]);
-    within = __builtin_amdgcn_readfirstlane(unit - (lo_r > 0 ? o_incl[lo_r - 1] : 0));
-    seq = __builtin_amdgcn_readfirstlane(PlanTab::at(tab, PlanTab::kSeq)[row]);
-    q0 = __builtin_amdgcn_readfirstlane(PlanTab::at(tab, PlanTab::kQ0)[row]);
-    n = __builtin_amdgcn_readfirstlane(PlanTab::at(tab, PlanTab::kN)[row]);
-    ctx_raw = __builtin_amdgcn_readfirstlane(PlanTab::at(tab, PlanTab::kCtx)[row]);
-  } else {
-    if (threadIdx.x == 0) s_found[0] = -1;  // ordered before the scan's writes by its barriers
-    scan_tiles(a, TQ, unit, s_wsum, s_found);
-    seq = __builtin_amdgcn_readfirstlane(s_found[0]);
-    within = __builtin_amdgcn_readfirstlane(s_found[1]);
-    if (seq < 0) return;  // unreachable for unit < per_kv; keeps every index below in range
-    n = seq_queries(a, seq, q0);
-    ctx_raw = a.context_lens[seq];
+  int64_t slot = blockIdx.x / kXcds;
+  if (slot >= per_xcd) return;
+  // Where every unit is resident at once, an XCD's CUs take its units in rows of one per
+  // CU, longest first: every second row is reversed, so that the CU with the longest unit
+  // of one gets the shortest of the next (a causal prompt's tiles grow linearly).
+  if (per_xcd <= (int64_t)prefill_occupancy<QT, D>() * a.pf_cus) {
+    const int64_t r = slot / a.pf_cus, c = slot % a.pf_cus;
+    const int64_t len = min((int64_t)a.pf_cus, per_xcd - r * a.pf_cus);
+    if (r & 1) slot = r * a.pf_cus + len - 1 - c;
   }
-  const int ntq = (n + TQ - 1) / TQ;
-  const int tile = ntq - 1 - within;  // latest (longest) tiles first
-  const bool reporter = kvh == 0 && tile == ntq - 1 && threadIdx.x == 0;
-  const int ctx = clamp_ctx(a, ctx_raw, reporter);
-  if (ctx < n && reporter) atomicOr(a.err_flag, ASTR_FLAG_BAD_INDEX);  // chunk longer than the context
+  const int64_t logical = (int64_t)(blockIdx.x % kXcds) * per_xcd + slot;
+  if (logical >= units) return;
+  const int piece = (int)(logical % a.pf_pieces);
+  const int head_unit = (int)(logical / a.pf_pieces);
+  const int kvh = head_unit / per_kv;
+  UnitRef u;
+  if (!unit_ref(a, TQ, tab, lds.wsum, lds.found, rows, head_unit % per_kv, u)) return;
+  const int seq = u.seq, q0 = u.q0, n = u.n;
+  const bool reporter = kvh == 0 && u.last && threadIdx.x == 0;
+  const int ctx = clamp_ctx(a, u.ctx_raw, reporter);
+  // chunk longer than the context (a one-token row may be empty, as in a decode launch)
+  if (ctx < n && n > 1 && reporter) atomicOr(a.err_flag, ASTR_FLAG_BAD_INDEX);
 
-  const TileSpan span = tile_span(a, ctx, n, tile, TQ);
+  TileSpan span = tile_span(a, ctx, n, u.tile, TQ);
   const int pos0 = span.pos0, t0 = span.t0, t1 = span.t1;
+  // the piece's key steps; a unit within pf_steps is its first piece alone
+  float* part = nullptr;
+  if (a.pf_pieces > 1) {
+    const int steps = (span.b_hi - span.b_lo + kWaves - 1) / kWaves;
+    if (piece > 0 && piece * a.pf_steps >= steps) return;
+    if (steps > a.pf_steps) {
+      if ((uint64_t)(logical + 1) * PiecePartial<D>::kFloats * sizeof(float) > a.pf_bytes) {
+        if (threadIdx.x == 0) atomicOr(a.err_flag, ASTR_FLAG_BAD_INDEX);  // offsets past the bound
+        return;
+      }
+      part = a.pf_ws + logical * PiecePartial<D>::kFloats;
+      span.b_lo += piece * a.pf_steps * kWaves;
+      // (the last piece takes whatever a context past the host's bound adds)
+      if (piece < a.pf_pieces - 1) span.b_hi = min(span.b_hi, span.b_lo + a.pf_steps * kWaves);
+    }
+  }
 
   // flat column f -> token t0 + f / G, head kvh * G + f % G, keys by its position
   auto column_of = [&](int f) __attribute__((always_inline)) -> ColumnInfo {
@@ -951,23 +1038,81 @@ __global__ __launch_bounds__(256, PrefillShape<D>::kOccupancy) void prefill_mfma
                       a.causal ? pos0 + tk_lo : ctx - 1, a.causal ? pos0 + tk_hi : ctx - 1,
                       tk_lo < t1};
   };
-  // normalise and store (fully masked columns: l = 0, acc = 0 -> 0)
-  auto store = [&](int, const float16v_t (&acc)[D / 32], float, float l, int ve,
+  auto store = [&](int, const float16v_t (&acc)[D / 32], float m, float l, int ve,
                    const ColumnInfo& c) __attribute__((always_inline)) {
-    if (!c.valid) return;
-    const float inv = ldexpf(1.f, ve) / fmaxf(l, FLT_MIN);  // the PV tiles carry 2^-ve
-    QT* op = static_cast<QT*>(a.out) + (int64_t)(q0 + c.tok) * a.o_tok + (int64_t)c.head * a.o_head +
-             D / 8 * (lane >> 5);
+    const float up = ldexpf(1.f, ve);  // the PV tiles carry 2^-ve
+    const int lane = lane_id();
+    if (part != nullptr) {
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      float v[D / 8];
-      acc_run<D>(acc, x, inv, v);
-      store_run<QT, D / 8>(op + D / 4 * x, v);
+      for (int k = 0; k < D / 32; ++k)
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          *PiecePartial<D>::acc(part, wave_id, k, x, lane) =
+              float4_t{acc[k][4 * x] * up, acc[k][4 * x + 1] * up, acc[k][4 * x + 2] * up,
+                       acc[k][4 * x + 3] * up};
+      if (lane < 32) {
+        float* ml = part + PiecePartial<D>::kAcc + (wave_id * 32 + lane) * 2;
+        ml[0] = m;
+        ml[1] = l;
+      }
+    } else if (c.valid) {
+      store_column<QT, D>(a, acc, up / fmaxf(l, FLT_MIN), q0 + c.tok, c.head, lane);
     }
   };
   prefill_unit<QT, D>(a, L, kvh, span.b_lo, span.b_hi,
-                         a.block_tables + (int64_t)seq * a.bt_stride, q0, t0, column_of,
-                         bounds_of, store, []() { return true; }, [](int) {});
+                      a.block_tables + (int64_t)seq * a.bt_stride, q0, t0, column_of,
+                      bounds_of, store, []() { return true; }, [](int) {});
+}
+
+// Merges the pieces of split units, one workgroup per unit: each lane the part of its
+// column that it held in the pieces, with the merge_softmax rule
+// (online_attention.py:42-63).
+template <typename QT, int D, int G>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(AttnArgs a) {
+  constexpr int TQ = PrefillShape<D>::kCols / G;
+  __shared__ int tab[PlanTab::kInts];
+  __shared__ int s_wsum[kWaves], s_found[2];
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  int rows;
+  const int per_kv = count_units(a, TQ, tab, s_wsum, s_found, rows);
+  if ((int64_t)blockIdx.x >= (int64_t)per_kv * a.cache.num_kv_heads) return;
+  const int kvh = blockIdx.x / per_kv;
+  UnitRef u;
+  if (!unit_ref(a, TQ, tab, s_wsum, s_found, rows, blockIdx.x % per_kv, u)) return;
+  const TileSpan span = tile_span(a, clamp_ctx(a, u.ctx_raw, false), u.n, u.tile, TQ);
+  const int steps = (span.b_hi - span.b_lo + kWaves - 1) / kWaves;
+  const int pieces = min((steps + a.pf_steps - 1) / a.pf_steps, a.pf_pieces);
+  const int64_t first = (int64_t)blockIdx.x * a.pf_pieces;
+  if (pieces <= 1 || (uint64_t)(first + pieces) * PiecePartial<D>::kFloats * sizeof(float) > a.pf_bytes)
+    return;
+  float* const base = a.pf_ws + first * PiecePartial<D>::kFloats;
+  const int64_t col = PiecePartial<D>::kAcc + (wave * 32 + (lane & 31)) * 2;
+  float mx = -FLT_MAX;
+  for (int j = 0; j < pieces; ++j) mx = fmaxf(mx, base[j * (int64_t)PiecePartial<D>::kFloats + col]);
+  float16v_t acc[D / 32];
+#pragma unroll
+  for (int n = 0; n < D / 32; ++n)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[n][j] = 0.f;
+  float l = 0.f;
+  for (int j = 0; j < pieces; ++j) {
+    float* const p = base + j * (int64_t)PiecePartial<D>::kFloats;
+    const float w = __builtin_amdgcn_exp2f(p[col] - mx);
+    l = fmaf(p[col + 1], w, l);
+#pragma unroll
+    for (int n = 0; n < D / 32; ++n)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const float4_t v = *PiecePartial<D>::acc(p, wave, n, x, lane);
+#pragma unroll
+        for (int y = 0; y < 4; ++y) acc[n][4 * x + y] = fmaf(v[y], w, acc[n][4 * x + y]);
+      }
+  }
+  const int f = wave * 32 + (lane & 31);
+  const int token = span.t0 + f / G;
+  if (token < span.t1)
+    store_column<QT, D>(a, acc, 1.f / fmaxf(l, FLT_MIN), u.q0 + token, kvh * G + f % G, lane);
 }
 
 // Prefix tiles of a decode plan (decode_plan.cpp): the shared blocks of sequences whose
@@ -981,7 +1126,7 @@ __global__ __launch_bounds__(256, PrefillShape<D>::kOccupancy) void prefill_mfma
 constexpr int kTileWords = 8, kMemberWords = 3;
 
 template <typename QT, int D, int G>
-__global__ __launch_bounds__(256, PrefillShape<D>::kOccupancy) void prefix_tiles_kernel(PlanArgs p) {
+__global__ __launch_bounds__(256, (prefill_occupancy<QT, D>())) void prefix_tiles_kernel(PlanArgs p) {
   static_assert(D == 64 || D == 128 || D == 256, "head_dim");
   constexpr int TQ = PrefillShape<D>::kCols / G;
   static_assert(PrefillShape<D>::kCols % G == 0, "GQA group must divide the column tile");
@@ -1134,19 +1279,54 @@ __global__ __launch_bounds__(256, PrefillShape<D>::kOccupancy) void prefix_tiles
 #endif
 }
 
+// Compute units of the current device (256 where that cannot be read).
+int prefill_cus() {
+  int dev = 0, v = 0;
+  if (hipGetDevice(&dev) == hipSuccess &&
+      hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
+    return v;
+  return 256;
+}
+
+// Key steps below which a unit is not split: a piece costs its start (~2 steps) and its
+// partial, written and read again.
+constexpr int kLeastPieceSteps = 8;
+constexpr int kMostPieces = 16;
+
 template <typename QT, int D, int G>
-int launch(const AttnArgs& a, hipStream_t stream) {
+int launch(AttnArgs a, hipStream_t stream) {
   constexpr int TQ = PrefillShape<D>::kCols / G;
-  // Sum over sequences of ceil(n/TQ) for n >= 2 is at most tokens/TQ + sequences
-  // (and at most tokens/2 sequences have n >= 2).
-  const int64_t seqs = a.num_seqs < a.num_q_tokens / 2 ? a.num_seqs : a.num_q_tokens / 2;
-  const int64_t max_units = ((int64_t)a.num_q_tokens + TQ - 1) / TQ + seqs;
-  const int64_t total = max_units * a.cache.num_kv_heads;
+  // Sum over sequences of ceil(n / TQ) for n >= pf_min_rows: each adds at most TQ - 1 to
+  // the token count, and there are at most tokens / pf_min_rows of them.
+  const int64_t seqs = std::min<int64_t>(a.num_seqs, a.num_q_tokens / a.pf_min_rows);
+  const int64_t max_units =
+      ((int64_t)a.num_q_tokens + seqs * (TQ - 1)) / TQ * a.cache.num_kv_heads;
+  if (max_units == 0) return 0;
+  // Units that leave half the resident workgroups or more without work are cut into equal
+  // key ranges, as many as there are idle workgroups per unit and the workspace holds (512
+  // tokens on 16000: 128 units of 258 steps on 512 workgroups, 477 -> 186 us in 4 pieces).
+  const int cus = prefill_cus();
+  a.pf_cus = cus >= kXcds ? cus / kXcds : 1;
+  int64_t keys = a.max_context;
+  if (a.window > 0) keys = std::min<int64_t>(keys, (int64_t)a.window + TQ + kBlockTokens);
+  const int64_t steps = (keys + kWaves * kBlockTokens - 1) / (kWaves * kBlockTokens) + 1;
+  const int64_t room = (int64_t)(a.pf_bytes / (PiecePartial<D>::kFloats * sizeof(float)));
+  const int64_t resident = (int64_t)cus * prefill_occupancy<QT, D>();
+  int64_t pieces = std::min<int64_t>(std::min(resident, room) / max_units, kMostPieces);
+  a.pf_pieces = 1;
+  a.pf_steps = INT32_MAX / kWaves;
+  if (pieces >= 2 && steps >= 2 * kLeastPieceSteps) {
+    a.pf_steps = (int32_t)std::max<int64_t>((steps + pieces - 1) / pieces, kLeastPieceSteps);
+    a.pf_pieces = (int32_t)((steps + a.pf_steps - 1) / a.pf_steps);
+  }
+  const int64_t total = max_units * a.pf_pieces;
   const int64_t grid = (total + kXcds - 1) / kXcds * kXcds;
-  if (grid == 0) return 0;
   if (grid > INT32_MAX) return fail(ASTR_EUNSUPPORTED, "prefill grid too large");
   hipLaunchKernelGGL((prefill_mfma_kernel<QT, D, G>), dim3((uint32_t)grid), dim3(kWaves * kWave),
                      0, stream, a);
+  if (a.pf_pieces > 1)
+    hipLaunchKernelGGL((prefill_merge_kernel<QT, D, G>), dim3((uint32_t)max_units),
+                       dim3(kWaves * kWave), 0, stream, a);
   const hipError_t err = hipGetLastError();
   return err == hipSuccess ? 0 : hip_fail(err, "paged_attention (prefill) launch");
 }

@@ -35,12 +35,12 @@ def _cache(device, rows, dim, kv, fmt, seed):
     return cache, tables, gen
 
 
-def _check(cache, tables, lens, counts, query, window=None, atol=2e-3, rtol=2e-3):
+def _check(cache, tables, lens, counts, query, window=None, atol=2e-3, rtol=2e-3, bound=None):
     device = query.device
     starts = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
     out = cache.paged_attention(0, query, torch.from_numpy(tables).to(device),
                                 torch.from_numpy(np.array(lens, np.int32)).to(device),
-                                max_context_len=max(lens), window=window,
+                                max_context_len=bound or max(lens), window=window,
                                 query_start_loc=torch.from_numpy(starts).to(device),
                                 max_query_len=max(counts), check=True)
     want = oracle_decode(tables, cache, query, context_lens=np.array(lens, np.int32),
@@ -109,3 +109,42 @@ def test_long_history(device):
     query = torch.randn((9, 2, 64), generator=gen, device=device).half()
     _check(cache, tables, lens, counts, query)
     _check(cache, tables, lens, counts, query, window=5000)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dim,kv,group", [(128, 1, 4), (64, 2, 2), (256, 1, 8)])
+@pytest.mark.parametrize("counts,priors", [([5], [3000]), ([40, 33], [2500, 100]),
+                                           ([129, 2, 60], [1100, 2048, 0])])
+def test_split_units(device, dim, kv, group, dtype, counts, priors):
+    """Few units over long histories: cut into key ranges and merged, shorter units beside
+    them whole, windows that leave a tile few keys, a history far below the declared bound."""
+    lens = [n + p for n, p in zip(counts, priors)]
+    cache, tables, gen = _cache(device, lens, dim, kv, "int8", dim)
+    query = torch.randn((sum(counts), kv * group, dim), generator=gen, device=device).to(dtype)
+    _check(cache, tables, lens, counts, query)
+    _check(cache, tables, lens, counts, query, window=700)
+    wide = np.zeros((len(lens), 2048), np.int32)
+    wide[:, :tables.shape[1]] = tables
+    _check(cache, wide, lens, counts, query, bound=16 * 2048)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_one_token_rows_beside_chunks(device, dtype):
+    """Short contexts: the prefill launch serves the one-token rows (16-bit queries), an
+    empty context included; equal chunks whose offsets hold a one-token row all the same."""
+    counts, priors = [1, 30, 1, 1, 7], [100, 0, 0, 400, 33]
+    lens = [n + p for n, p in zip(counts, priors)]
+    cache, tables, gen = _cache(device, lens, 128, 2, "int8", 9)
+    query = torch.randn((sum(counts), 8, 128), generator=gen, device=device).to(dtype)
+    _check(cache, tables, lens, counts, query)
+    lens[2] = 0
+    _check(cache, tables, lens, counts, query)
+    # 3 rows x 4 tokens declared, offsets that give 1 + 4 + 4
+    starts = torch.tensor([0, 1, 5, 9], dtype=torch.int32, device=device)
+    sub = torch.from_numpy(tables[:3]).to(device)
+    ctx = torch.tensor([50, 30, 16], dtype=torch.int32, device=device)
+    out = cache.paged_attention(0, query[:12], sub, ctx, max_context_len=64,
+                                query_start_loc=starts, max_query_len=4, check=True)
+    want = oracle_decode(tables[:3], cache, query[:9], context_lens=np.array([50, 30, 16], np.int32),
+                         scale=128 ** -0.5, query_lens=np.array([1, 4, 4], np.int32), fp64=True)
+    np.testing.assert_allclose(out[:9].float().cpu().numpy(), want, atol=2e-3, rtol=5e-3)
