@@ -434,7 +434,8 @@ def hip_forward(runner, sequences, chunks, *, return_all_logits=False, padding_m
         runner.model_execution_seconds += time.monotonic() - started
         runner.forward_calls += 1
         runner.input_tokens_computed += ids.numel()
-    rows = [(row if return_all_logits else row[-1]).detach().float().cpu() for row in logits]
+    # one device-to-host copy for the batch (a copy per row waits for the device each time)
+    rows = list((logits if return_all_logits else logits[:, -1]).detach().float().cpu())
     if features is not None:
         return [(row, feature.detach()) for row, feature in zip(rows, features)]
     return rows
