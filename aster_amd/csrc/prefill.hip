@@ -335,16 +335,16 @@ struct PrefillLds {
 };
 
 // One block of the wave's own as loaded from the arena, on its way to the operands. K:
-// lane (key = lane % 16, lane / 16) takes 16 consecutive d per 64. V: D / 4 lanes take the
-// dwords of a token row, for the lane's quads of four tokens (quad q: tokens 4 q + [0, 4)).
+// lane (key = lane % 16, lane / 16) takes 16 consecutive d per 64. V: 16 lanes take a token
+// row, D / 16 bytes each, and lane group g = lane / 16 the tokens 4 g + [0, 4): four loads
+// of D / 16 bytes a lane (dwords of whole rows took eight at head dim 128, and the loads
+// were 14 % of the kernel).
 template <int D>
 struct RawBlock {
-  static constexpr int kRowLanes = D / 4;             // lanes across a token row
-  static constexpr int kGroups = kWave / kRowLanes;   // 4, 2, 1
-  static constexpr int kQuads = 4 / kGroups;          // quads per lane: g, g + kGroups, ...
+  static constexpr int kWords = D / 64;  // dwords of a token row per lane
   uint4 k[D / 64];
-  uint32_t v[kQuads][4];
-  float4_t vs[kQuads];
+  uint32_t v[4][kWords];
+  float4_t vs;
   float ks;
   uint32_t pad;
   int id;
@@ -356,28 +356,33 @@ __device__ __forceinline__ uint32_t load_pad(const AttnArgs& a, int id, int lane
                                             4 * (lane & 3));
 }
 
-// kPad: the padding bytes too (else convert_raw reads them)
+// kPad: the padding bytes too (else convert_raw reads them). Every address is a uniform
+// base and a 32-bit lane offset.
 template <int D, bool kPad>
 __device__ __forceinline__ void load_raw(const AttnArgs& a, int id, int kvh, int lane, bool masks,
                                          RawBlock<D>& b) {
-  using R = RawBlock<D>;
-  const int8_t* kp = a.cache.k_codes + id * a.cache.code_block_stride + kvh * a.cache.code_head_stride;
-  const int8_t* vp = a.cache.v_codes + id * a.cache.code_block_stride + kvh * a.cache.code_head_stride;
-  const float* ksp = a.cache.k_scales + id * a.cache.scale_block_stride + kvh * a.cache.scale_head_stride;
-  const float* vsp = a.cache.v_scales + id * a.cache.scale_block_stride + kvh * a.cache.scale_head_stride;
+  const int64_t code = id * a.cache.code_block_stride + kvh * a.cache.code_head_stride;
+  const int64_t scale = id * a.cache.scale_block_stride + kvh * a.cache.scale_head_stride;
+  const int8_t* const kp = a.cache.k_codes + code;
+  const int8_t* const vp = a.cache.v_codes + code;
+  const float* const ksp = a.cache.k_scales + scale;
+  const float* const vsp = a.cache.v_scales + scale;
+  const uint32_t r = lane & 15, g = lane >> 4;
+  const uint32_t koff = r * D + g * 16;
 #pragma unroll
-  for (int i = 0; i < D / 64; ++i)
-    b.k[i] = *reinterpret_cast<const uint4*>(kp + (lane & 15) * D + (lane >> 4) * 16 + 64 * i);
-  const int g = lane / R::kRowLanes, dg = lane % R::kRowLanes;
+  for (int i = 0; i < D / 64; ++i) b.k[i] = *reinterpret_cast<const uint4*>(kp + (koff + 64 * i));
+  struct alignas(D / 16) Row {
+    uint32_t w[RawBlock<D>::kWords];
+  };
+  const uint32_t voff = 4 * g * D + r * (D / 16);
 #pragma unroll
-  for (int q = 0; q < R::kQuads; ++q) {
-    const int quad = g + q * R::kGroups;
+  for (int t = 0; t < 4; ++t) {
+    const Row row = *reinterpret_cast<const Row*>(vp + (voff + t * D));
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
-      b.v[q][t] = *reinterpret_cast<const uint32_t*>(vp + (4 * quad + t) * D + 4 * dg);
-    b.vs[q] = *reinterpret_cast<const float4_t*>(vsp + 4 * quad);
+    for (int i = 0; i < RawBlock<D>::kWords; ++i) b.v[t][i] = row.w[i];
   }
-  b.ks = ksp[lane & 15];
+  b.vs = *reinterpret_cast<const float4_t*>(vsp + 4 * g);
+  b.ks = ksp[r];
   b.id = id;
   if constexpr (kPad) b.pad = masks ? load_pad<D>(a, id, lane) : 0x01010101u;
 }
@@ -389,7 +394,6 @@ template <int D, bool kPad>
 __device__ __forceinline__ void convert_raw(const AttnArgs& a, const RawBlock<D>& b,
                                             PrefillLds<D>& L, int buf, int w, int lane, bool masks,
                                             int ve, float vlim) {
-  using R = RawBlock<D>;
   using Lds = PrefillLds<D>;
   // K: 16 codes -> the two lane halves' entries of one chunk
   uint4* kd = L.k[buf] + (w / 2) * Lds::kChunks * kWave + 16 * (w % 2) + (lane & 15);
@@ -406,16 +410,13 @@ __device__ __forceinline__ void convert_raw(const AttnArgs& a, const RawBlock<D>
     e[32] = uint4{word(4), word(5), word(6), word(7)};
   }
   // V
-  float vsm = 0.f;
-#pragma unroll
-  for (int q = 0; q < R::kQuads; ++q)
-    vsm = fmaxf(vsm, fmaxf(fmaxf(b.vs[q][0], b.vs[q][1]), fmaxf(b.vs[q][2], b.vs[q][3])));
+  const float vsm = fmaxf(fmaxf(b.vs[0], b.vs[1]), fmaxf(b.vs[2], b.vs[3]));
   constexpr float cs = v_weight_scale<KF>();
   int e = ve;
   float c = cs;
   if (__ballot(vsm > vlim) != 0 || ve != 0) {
     if (__ballot(vsm > vlim) != 0) {
-      float wm = 0.f;  // a group of lanes holds the same scales: 16 lanes or more
+      float wm = 0.f;  // each group of 16 lanes holds the same scales
 #pragma unroll
       for (int i = 0; i < kWave; i += 16)
         wm = fmaxf(wm, __builtin_bit_cast(float, __builtin_amdgcn_readlane(
@@ -426,45 +427,28 @@ __device__ __forceinline__ void convert_raw(const AttnArgs& a, const RawBlock<D>
     }
     c = ldexpf(cs, -e);
   }
-  const int g = lane / R::kRowLanes, dg = lane % R::kRowLanes;
-  half4_t vop[4][R::kQuads];
+  // dimension d = (D / 16) (lane % 16) + i is row r = d / (D / 32) of operand n =
+  // d % (D / 32); the lane's quad of tokens, 2 a' + h, is half a' of lane half h's entry
+  const int g = lane >> 4;
+  const half4_t vsh = {(_Float16)(b.vs[0] * c), (_Float16)(b.vs[1] * c), (_Float16)(b.vs[2] * c),
+                       (_Float16)(b.vs[3] * c)};
+  uint2* vd = reinterpret_cast<uint2*>(L.v[buf] + w * Lds::kRowsN * kWave + 32 * (g & 1) +
+                                       2 * (lane & 15)) + (g >> 1);
 #pragma unroll
-  for (int q = 0; q < R::kQuads; ++q) {
-    const half4_t vsh = {(_Float16)(b.vs[q][0] * c), (_Float16)(b.vs[q][1] * c),
-                         (_Float16)(b.vs[q][2] * c), (_Float16)(b.vs[q][3] * c)};
-    vop[0][q] = v_operand<0, KF>(b.v[q]);
-    vop[1][q] = v_operand<1, KF>(b.v[q]);
-    vop[2][q] = v_operand<2, KF>(b.v[q]);
-    vop[3][q] = v_operand<3, KF>(b.v[q]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if constexpr (KF == kE5M2) {
-        constexpr _Float16 down = (_Float16)(1.f / 256.f);
-        vop[i][q] = vop[i][q] * half4_t{down, down, down, down};  // exact: E5M2 times 2^-8 fits f16
-      }
-      vop[i][q] = vop[i][q] * vsh;
+  for (int i = 0; i < D / 16; ++i) {
+    const uint32_t col[4] = {b.v[0][i / 4], b.v[1][i / 4], b.v[2][i / 4], b.v[3][i / 4]};
+    half4_t v;
+    switch (i % 4) {
+      case 0: v = v_operand<0, KF>(col); break;
+      case 1: v = v_operand<1, KF>(col); break;
+      case 2: v = v_operand<2, KF>(col); break;
+      default: v = v_operand<3, KF>(col); break;
     }
-  }
-  // dimension d = 4 dg + i is row r = d / (D / 32) of operand n = d % (D / 32); quad
-  // 2 a' + h is half a' of lane half h's entry
-  uint4* vd = L.v[buf] + w * Lds::kRowsN * kWave;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int d = 4 * dg + i, r = d / Lds::kRowsN, n = d % Lds::kRowsN;
-    if constexpr (R::kGroups == 4) {
-      reinterpret_cast<uint2*>(vd + n * kWave + 32 * (g & 1) + r)[g >> 1] =
-          __builtin_bit_cast(uint2, vop[i][0]);
-    } else if constexpr (R::kGroups == 2) {
-      const uint2 lo = __builtin_bit_cast(uint2, vop[i][0]), hi = __builtin_bit_cast(uint2, vop[i][1]);
-      vd[n * kWave + 32 * g + r] = uint4{lo.x, lo.y, hi.x, hi.y};
-    } else {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const uint2 lo = __builtin_bit_cast(uint2, vop[i][h]);
-        const uint2 hi = __builtin_bit_cast(uint2, vop[i][2 + h]);
-        vd[n * kWave + 32 * h + r] = uint4{lo.x, lo.y, hi.x, hi.y};
-      }
+    if constexpr (KF == kE5M2) {
+      constexpr _Float16 down = (_Float16)(1.f / 256.f);
+      v = v * half4_t{down, down, down, down};  // exact: E5M2 values times 2^-8 fit f16
     }
+    vd[2 * (i % Lds::kRowsN * kWave + i / Lds::kRowsN)] = __builtin_bit_cast(uint2, v * vsh);
   }
   // key factors: at least FLT_MIN, so that a masked score's -inf stays -inf
   const float ksf = fmaxf(b.ks * (a.qk_scale_log2 * code_scale<KF>()), FLT_MIN);
@@ -531,7 +515,7 @@ __device__ __forceinline__ void prefill_half(const PrefillLds<D>& L, int buf, in
     padded = __ballot(pw.x != 0x01010101u || pw.y != 0x01010101u || pw.z != 0x01010101u ||
                       pw.w != 0x01010101u) != 0;
   }
-  constexpr int kAhead = QOp<QT, D>::kAhead ? D == 128 ? 6 : 2 * Lds::kRowsN : 0;
+  constexpr int kAhead = QOp<QT, D>::kAhead ? 2 * Lds::kRowsN : 0;
   half8_t vop[2 * Lds::kRowsN];
   auto load_v = [&](int n0, int n1) __attribute__((always_inline)) {
 #pragma unroll
