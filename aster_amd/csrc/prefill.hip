@@ -6,19 +6,19 @@
 // already appended) sits at position p = ctx - n + i and sees key k iff
 //   k <= p (causal; else k < ctx)  and  k > p - window (window > 0).
 //
-// Work unit: (kv head, sequence, tile of TQ query tokens), TQ * G = 64 * NT
-// (token, head) columns of one kv head, 16 * NT columns per wave. The unit's
-// visible key range is streamed in steps of four 16-token blocks; each wave
-// stages one block of the step into LDS with direct global->LDS loads and then
-// all four waves run all four blocks through the MFMAs:
-//   S^T[t][c]  = K[t][:] . Q[c][:]     v_mfma_i32_16x16x64_i8: the K codes as stored,
-//                                        the query as two int8 terms (exact int32 dot),
-//                                        three on steps with large key scales
-//   O^T[d][c] += V^T[d][t] . P^T[t][c]  v_mfma_f32_16x16x32_f16 over two blocks (P^T
-//                                        carries V's scales)
+// Work unit: (kv head, sequence, tile of TQ query tokens), TQ * G = 128 (token, head)
+// columns of one kv head, 32 per wave. The unit's visible key range is streamed in steps
+// of four 16-token blocks; each wave loads one block of the step into registers and
+// converts it once, one step ahead, into f16 operands in LDS that all four waves read:
+//   S^T[t][c]  = K[t][:] . Q[c][:]     v_mfma_f32_32x32x16_f16: the K codes (exact in f16)
+//                                        against the query, 16-bit queries exact, fp32
+//                                        queries as two f16 terms
+//   O^T[d][c] += V^T[d][t] . P^T[t][c]  v_mfma_f32_32x32x16_f16 (V times its f16 scale)
 // so every K/V byte of the unit's range is read once per query tile and shared by
 // the G heads and TQ tokens of the tile. Softmax statistics are per column, in
-// base 2, with the lazy rescale of the decode kernels.
+// base 2, with the lazy rescale of the decode kernels. Converting per workgroup instead
+// of per wave and per score took a 512-token chunk on 16000 keys (bf16, int8, 32/8 heads
+// of 128) from 583 to 486 us, cutting its units into key ranges (below) to 195 us.
 //
 // Units of one (kv head, sequence) are consecutive, longest (latest) tile first,
 // and the linear workgroup id is remapped so that each XCD (workgroups are dealt
@@ -450,8 +450,10 @@ __device__ __forceinline__ void convert_raw(const AttnArgs& a, const RawBlock<D>
     }
     vd[2 * (i % Lds::kRowsN * kWave + i / Lds::kRowsN)] = __builtin_bit_cast(uint2, v * vsh);
   }
-  // key factors: at least FLT_MIN, so that a masked score's -inf stays -inf
-  const float ksf = fmaxf(b.ks * (a.qk_scale_log2 * code_scale<KF>()), FLT_MIN);
+  // key factors: above zero, so that a masked score's -inf stays -inf; a NaN scale counts as
+  // infinite, which the steps' edge path reports where a key of it is seen
+  float ksf = fmaxf(b.ks * (a.qk_scale_log2 * code_scale<KF>()), __FLT_DENORM_MIN__);
+  ksf = b.ks == b.ks ? ksf : INFINITY;
   const bool large = __ballot(!(ksf <= safe_factor())) != 0;
   if (lane < 16) L.ks[buf][16 * w + lane] = ksf;
   if (masks && lane < 4) L.pad[buf][4 * w + lane] = kPad ? b.pad : load_pad<D>(a, b.id, lane);
@@ -566,13 +568,14 @@ __device__ __forceinline__ void prefill_half(const PrefillLds<D>& L, int buf, in
           // -1 when key < lo or key > hi (either difference negative), else 0
           const int32_t outside = bnd ? ((key - lo[t]) | (hi[t] - key)) >> 31 : 0;
           const uint32_t hide = used ? (uint32_t)(outside | padding) : 0xffffffffu;
-          const float sv = s[t][j] * back[t];
-          const uint32_t xb = __builtin_bit_cast(uint32_t, sv * ks[x][y]);
+          // (the factors first: a large query's beside a small key's stays in range)
+          const uint32_t xb = __builtin_bit_cast(uint32_t, s[t][j] * (back[t] * ks[x][y]));
           // exponent field all ones (inf or NaN) -> bit 31 after the carry
           nonfinite |= ((xb & 0x7f800000u) + 0x00800000u) & ~hide;
-          s[t][j] = __builtin_bit_cast(
-              float, (__builtin_bit_cast(uint32_t, sv) & ~hide) | (0xff800000u & hide));  // -inf
+          s[t][j] = __builtin_bit_cast(float, (xb & ~hide) | (0xff800000u & hide));  // -inf
         }
+        static_assert(NT == 1, "the scores hold the one column tile's factors from here on");
+        ks[x][y] = 1.f;
       }
     }
     if (__ballot((nonfinite >> 31) != 0) != 0) bad_score = true;

@@ -102,6 +102,34 @@ def test_overflowing_scores_raise(device):
         _check(cache, tables, lens, counts, query)
 
 
+@pytest.mark.parametrize("fmt", ["int8", "fp8_e4m3fn"])
+@pytest.mark.parametrize("slot", [0, 70, 79])
+def test_nan_key_scale(device, fmt, slot):
+    """A NaN key scale is reported where a query sees its key, and nowhere else: past the
+    context (the block's last slot) it changes nothing."""
+    lens, counts = [79], [40]
+    cache, tables, gen = _cache(device, lens, 128, 1, fmt, 3)
+    query = torch.randn((40, 4, 128), generator=gen, device=device).bfloat16()
+    cache.scales[int(tables[0, slot // 16]), 0, 0, 0, slot % 16] = float("nan")
+    if slot < 79:
+        with pytest.raises(ValueError, match="overflow"):
+            _check(cache, tables, lens, counts, query)
+    else:
+        _check(cache, tables, lens, counts, query)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_smallest_key_scales(device, dtype):
+    """Key scales at the quantizer's least (the smallest normal number) under queries large
+    enough for ordinary scores: their factor is below the normal range, which costs it
+    2^-21 of itself."""
+    lens, counts = [79], [40]
+    cache, tables, gen = _cache(device, lens, 128, 1, "int8", 3)
+    cache.scales[:, :, 0] = 2.0 ** -126
+    query = (torch.randn((40, 4, 128), generator=gen, device=device) * 2.0 ** 119).to(dtype)
+    _check(cache, tables, lens, counts, query)
+
+
 def test_long_history(device):
     """More than 64 key steps (the block ids are fetched 64 steps at a time)."""
     lens, counts = [64 * 64 * 2 + 77], [9]
