@@ -154,13 +154,15 @@ namespace {
 //     the same;
 //   - contexts up to 512 keys are at most 8 key steps of ~2 us for a one-token row, which
 //     runs beside the chunks' units, no longer than the launches it replaces, while every
-//     row has a CU of its own. Not for fp32 queries, whose one-token rows are attended in
-//     exact fp32.
+//     row has a CU of its own.
+// Not for fp32 queries: one-token rows of theirs are attended in exact fp32, and only the
+// offsets on the device say whether there are any.
 constexpr int kOnlyChunksContext = 512;
 bool only_chunks(int32_t q_dtype, int32_t tokens, int32_t max_query_len, int32_t num_seqs,
                  int32_t num_kv_heads, int32_t max_context_len) {
+  if (q_dtype == ASTR_F32) return false;
   if ((int64_t)num_seqs * max_query_len == tokens) return true;
-  return q_dtype != ASTR_F32 && max_context_len <= kOnlyChunksContext &&
+  return max_context_len <= kOnlyChunksContext &&
          (int64_t)num_seqs * num_kv_heads <= device_cus();
 }
 
