@@ -434,8 +434,12 @@ def hip_forward(runner, sequences, chunks, *, return_all_logits=False, padding_m
         runner.model_execution_seconds += time.monotonic() - started
         runner.forward_calls += 1
         runner.input_tokens_computed += ids.numel()
-    # one device-to-host copy for the batch (a copy per row waits for the device each time)
-    rows = list((logits if return_all_logits else logits[:, -1]).detach().float().cpu())
+    # one device-to-host copy for the batch (a copy per row waits for the device each time);
+    # logits of every token row by row, so that no fp32 copy of all of them is on the device
+    if return_all_logits:
+        rows = [row.detach().float().cpu() for row in logits]
+    else:
+        rows = list(logits[:, -1].detach().float().cpu())
     if features is not None:
         return [(row, feature.detach()) for row, feature in zip(rows, features)]
     return rows
