@@ -99,16 +99,23 @@ struct AttnArgs {
   const void* new_v;
   int64_t nk_tok, nk_head, nv_tok, nv_head;
   const int64_t* new_slots;
-  // chunked prefill: the fewest query tokens of a row it takes (2; 1 where no decode launch
-  // precedes it), and the key split of its units, settled by the launcher: units of more
-  // than pf_steps key steps run as up to pf_pieces pieces that leave partials in pf_ws
-  // (pf_bytes long), for a merge launch
-  int32_t pf_min_rows, pf_pieces, pf_steps;
+  int32_t* err_flag;
+};
+
+// A chunked-prefill call. Apart from AttnArgs, which the planned decode's arguments hold
+// too: with these fields in between, its appending call took 62.5 us instead of 61.9
+// (64 rows of 128 to 4096 tokens, 32/8 heads of 128).
+struct ChunkArgs : AttnArgs {
+  int32_t pf_min_rows;  // fewest query tokens of a row it takes (2; 1 where no decode
+                        // launch precedes it)
+  // the key split of its units, settled by the launcher: units of more than pf_steps key
+  // steps run as up to pf_pieces pieces that leave partials in pf_ws (pf_bytes long), for
+  // a merge launch
+  int32_t pf_pieces, pf_steps;
   int32_t pf_cus;       // compute units per XCD
   int32_t max_context;  // host bound of context_lens
   float* pf_ws;
   size_t pf_bytes;
-  int32_t* err_flag;
 };
 
 // Statistics of one row from its merged base-2 state (maximum m, mass l, numerator
@@ -977,7 +984,7 @@ template <int KF>
 int launch_streamk_plain_kf(const AttnArgs& a, int32_t q_dtype, hipStream_t stream);
 // Rows with more than one query token (chunked prefill), one workgroup per
 // (kv head, sequence, tile of query tokens); needs q_start.
-template <int KF> int launch_prefill_kf(const AttnArgs& a, int32_t q_dtype, hipStream_t stream);
+template <int KF> int launch_prefill_kf(const ChunkArgs& a, int32_t q_dtype, hipStream_t stream);
 // Decode rows on a host plan (decode_planned.hip); with `resident` non-null nothing is
 // launched and the kernel's resident workgroups per CU land there.
 template <int KF>
@@ -990,7 +997,7 @@ int launch_prefix_tiles_kf(const PlanArgs& p, int32_t q_dtype, hipStream_t strea
   template <> int launch_partitioned_kf<KF>(const AttnArgs&, int32_t, hipStream_t);       \
   template <> int launch_streamk_kf<KF>(const AttnArgs&, int32_t, hipStream_t);           \
   template <> int launch_streamk_plain_kf<KF>(const AttnArgs&, int32_t, hipStream_t);     \
-  template <> int launch_prefill_kf<KF>(const AttnArgs&, int32_t, hipStream_t);             \
+  template <> int launch_prefill_kf<KF>(const ChunkArgs&, int32_t, hipStream_t);            \
   template <> int launch_planned_kf<KF>(const PlanArgs&, int32_t, hipStream_t, int*);     \
   template <> int launch_prefix_tiles_kf<KF>(const PlanArgs&, int32_t, hipStream_t);
 ASTR_DECLARE_LAUNCHERS(kInt8)
@@ -998,17 +1005,17 @@ ASTR_DECLARE_LAUNCHERS(kE4M3)
 ASTR_DECLARE_LAUNCHERS(kE5M2)
 #undef ASTR_DECLARE_LAUNCHERS
 
-#define ASTR_BY_FORMAT(name)                                                     \
-  inline int name(const AttnArgs& a, int32_t q_dtype, hipStream_t stream) {      \
+#define ASTR_BY_FORMAT(name, Args)                                               \
+  inline int name(const Args& a, int32_t q_dtype, hipStream_t stream) {          \
     switch (a.cache.code_format) {                                               \
       case kInt8: return name##_kf<kInt8>(a, q_dtype, stream);                   \
       case kE4M3: return name##_kf<kE4M3>(a, q_dtype, stream);                   \
       default: return name##_kf<kE5M2>(a, q_dtype, stream);                     \
     }                                                                            \
   }
-ASTR_BY_FORMAT(launch_partitioned)
-ASTR_BY_FORMAT(launch_streamk)
-ASTR_BY_FORMAT(launch_prefill)
+ASTR_BY_FORMAT(launch_partitioned, AttnArgs)
+ASTR_BY_FORMAT(launch_streamk, AttnArgs)
+ASTR_BY_FORMAT(launch_prefill, ChunkArgs)
 #undef ASTR_BY_FORMAT
 inline int launch_planned(const PlanArgs& p, int32_t q_dtype, hipStream_t stream, int* resident) {
   switch (p.a.cache.code_format) {

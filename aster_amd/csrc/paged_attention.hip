@@ -318,7 +318,7 @@ int paged_attention(const astr_paged_kv* cache, const void* query, int32_t q_dty
     return fail(ASTR_EINVAL, "a 256-byte aligned workspace of %zu bytes is required (%zu given)",
                 need, workspace_bytes);
 
-  AttnArgs a{};
+  ChunkArgs a{};
   a.q_start = query_start_loc;
   a.num_q_tokens = query_start_loc != nullptr ? num_query_tokens : num_seqs;
   a.max_q_len = query_start_loc != nullptr ? max_query_len : 1;

@@ -92,7 +92,7 @@ __device__ __forceinline__ TileSpan tile_span(const AttnArgs& a, int ctx, int n,
 
 constexpr int kOrderMax = 256;  // chunk rows ordered longest first; beyond this, index order
 
-__device__ __forceinline__ int query_tiles(const AttnArgs& a, int s, int tq) {
+__device__ __forceinline__ int query_tiles(const ChunkArgs& a, int s, int tq) {
   int begin;
   const int n = seq_queries(a, s, begin);
   return n >= a.pf_min_rows ? (n + tq - 1) / tq : 0;
@@ -112,7 +112,7 @@ struct PlanTab {
   __device__ static int* at(int* tab, int array) { return tab + array * kOrderMax; }
 };
 
-__device__ int plan_rows(const AttnArgs& a, int tq, int* tab, int* s_wsum, int& total) {
+__device__ int plan_rows(const ChunkArgs& a, int tq, int* tab, int* s_wsum, int& total) {
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   int* const r_tiles = PlanTab::at(tab, PlanTab::kTiles);
   int* const r_key = PlanTab::at(tab, PlanTab::kKey);
@@ -182,7 +182,7 @@ __device__ int plan_rows(const AttnArgs& a, int tq, int* tab, int* s_wsum, int& 
 // Workgroup-wide scan of the query-tile counts of all sequences in index order. Returns
 // the total; when `unit` >= 0, the sequence holding that unit and the unit's index
 // within the sequence land in found[0], found[1]. Every thread calls it.
-__device__ int scan_tiles(const AttnArgs& a, int tq, int unit, int* s_wsum, int* found) {
+__device__ int scan_tiles(const ChunkArgs& a, int tq, int unit, int* s_wsum, int* found) {
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   int base = 0;
   for (int c0 = 0; c0 < a.num_seqs; c0 += kWaves * kWave) {
@@ -872,14 +872,14 @@ struct UnitRef {
 
 // Units of one kv head, from the dispatch plan (in `tab` when rows >= 0) or the scan in
 // index order beyond kOrderMax rows. Every thread calls both.
-__device__ __forceinline__ int count_units(const AttnArgs& a, int tq, int* tab, int* s_wsum,
+__device__ __forceinline__ int count_units(const ChunkArgs& a, int tq, int* tab, int* s_wsum,
                                            int* s_found, int& rows) {
   int per_kv = 0;
   rows = plan_rows(a, tq, tab, s_wsum, per_kv);
   if (rows < 0) per_kv = scan_tiles(a, tq, -1, s_wsum, s_found);
   return per_kv;
 }
-__device__ __forceinline__ bool unit_ref(const AttnArgs& a, int tq, int* tab, int* s_wsum,
+__device__ __forceinline__ bool unit_ref(const ChunkArgs& a, int tq, int* tab, int* s_wsum,
                                          int* s_found, int rows, int unit, UnitRef& u) {
   int within;
   if (rows >= 0) {
@@ -942,7 +942,7 @@ __device__ __forceinline__ void store_column(const AttnArgs& a, const float16v_t
 }
 
 template <typename QT, int D, int G>
-__global__ __launch_bounds__(256, (prefill_occupancy<QT, D>())) void prefill_mfma_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256, (prefill_occupancy<QT, D>())) void prefill_mfma_kernel(ChunkArgs a) {
   static_assert(D == 64 || D == 128 || D == 256, "head_dim");
   constexpr int NT = PrefillShape<D>::NT;
   constexpr int TQ = PrefillShape<D>::kCols / G;
@@ -1055,7 +1055,7 @@ __global__ __launch_bounds__(256, (prefill_occupancy<QT, D>())) void prefill_mfm
 // column that it held in the pieces, with the merge_softmax rule
 // (online_attention.py:42-63).
 template <typename QT, int D, int G>
-__global__ __launch_bounds__(256) void prefill_merge_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256) void prefill_merge_kernel(ChunkArgs a) {
   constexpr int TQ = PrefillShape<D>::kCols / G;
   __shared__ int tab[PlanTab::kInts];
   __shared__ int s_wsum[kWaves], s_found[2];
@@ -1281,7 +1281,7 @@ constexpr int kLeastPieceSteps = 8;
 constexpr int kMostPieces = 16;
 
 template <typename QT, int D, int G>
-int launch(AttnArgs a, hipStream_t stream) {
+int launch(ChunkArgs a, hipStream_t stream) {
   constexpr int TQ = PrefillShape<D>::kCols / G;
   // Sum over sequences of ceil(n / TQ) for n >= pf_min_rows: each adds at most TQ - 1 to
   // the token count, and there are at most tokens / pf_min_rows of them.
@@ -1319,7 +1319,7 @@ int launch(AttnArgs a, hipStream_t stream) {
 }
 
 template <typename QT, int D>
-int dispatch_group(const AttnArgs& a, int G, hipStream_t s) {
+int dispatch_group(const ChunkArgs& a, int G, hipStream_t s) {
   switch (G) {
     case 1: return launch<QT, D, 1>(a, s);
     case 2: return launch<QT, D, 2>(a, s);
@@ -1331,7 +1331,7 @@ int dispatch_group(const AttnArgs& a, int G, hipStream_t s) {
 }
 
 template <typename QT>
-int dispatch_dim(const AttnArgs& a, int G, hipStream_t s) {
+int dispatch_dim(const ChunkArgs& a, int G, hipStream_t s) {
   switch (a.cache.head_dim) {
     case 64: return dispatch_group<QT, 64>(a, G, s);
     case 128: return dispatch_group<QT, 128>(a, G, s);
@@ -1398,7 +1398,7 @@ int launch_prefix_tiles_kf<KF>(const PlanArgs& p, int32_t q_dtype, hipStream_t s
 }
 
 template <>
-int launch_prefill_kf<KF>(const AttnArgs& a, int32_t q_dtype, hipStream_t stream) {
+int launch_prefill_kf<KF>(const ChunkArgs& a, int32_t q_dtype, hipStream_t stream) {
   const int G = a.num_q_heads / a.cache.num_kv_heads;
   switch (q_dtype) {
     case ASTR_F32: return dispatch_dim<float>(a, G, stream);
