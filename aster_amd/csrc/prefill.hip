@@ -213,6 +213,13 @@ __device__ int scan_tiles(const ChunkArgs& a, int tq, int unit, int* s_wsum, int
 // factor below this keeps every score finite (max code 127; 448 2^-8 for E4M3FN; 57344).
 constexpr float safe_factor() { return KF == kInt8 ? 1.0e29f : KF == kE4M3 ? 1.0e31f : 5.0e26f; }
 
+// A running maximum (base 2) at or below this is none yet to the key steps: they take the
+// scores as they are and then the maximum of these. Reduced by it, a later score far above
+// keeps only the digits that the maximum leaves it (down to kFarMax a step of 2^-13, near
+// -FLT_MAX none, and the difference overflows), however ordinary the score itself is. A column
+// whose scores all lie there takes the rescale on every step.
+constexpr float kFarMax = -2048.f;
+
 typedef float float16v_t __attribute__((ext_vector_type(16)));
 
 // Maximum and sum over a lane and the one 32 away (v_permlane32_swap_b32: the pair of
@@ -584,7 +591,7 @@ __device__ __forceinline__ void prefill_half(const PrefillLds<D>& L, int buf, in
   float me[NT], tmax[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    me[t] = m[t] > -FLT_MAX ? m[t] : 0.f;  // a column without a key so far: scores as they are
+    me[t] = m[t] > kFarMax ? m[t] : 0.f;  // (and in a column without a key so far)
     float mu = -INFINITY;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
@@ -592,7 +599,7 @@ __device__ __forceinline__ void prefill_half(const PrefillLds<D>& L, int buf, in
       mu = vmax(mu, s[t][j]);  // NaN-propagating
     }
     tmax[t] = mu;
-    need |= !(mu <= kRescaleSlack) || m[t] == -FLT_MAX;
+    need |= !(mu <= kRescaleSlack) || m[t] <= kFarMax;
   }
   if (__ballot(need) != 0) {
 #pragma unroll

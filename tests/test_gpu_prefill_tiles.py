@@ -178,3 +178,47 @@ def test_one_token_rows_beside_chunks(device, dtype):
     np.testing.assert_allclose(out[:9].float().cpu().numpy(), want, atol=2e-3, rtol=5e-3)
     if dtype == torch.float32:  # one-token rows in exact fp32: sums of 50 terms of order 1
         np.testing.assert_allclose(out[0].cpu().numpy(), want[0], atol=2e-5, rtol=0)
+
+
+def _two_groups(device, dim, fmt, n, first, codes, k_scale, v):
+    """One chunk of 9 queries after ``n`` keys of one head: keys below ``first`` and the rest
+    with K codes ``codes[0]`` and ``codes[1]`` in every dimension but the first (0 there), K
+    scales ``k_scale[0]`` and ``[1]``, values ``v[0]`` and ``v[1]``."""
+    cache, tables, _ = _cache(device, [n], dim, 1, fmt, 3)
+    most = {"int8": 127.0, "fp8_e4m3fn": 448.0, "fp8_e5m2": 57344.0}[fmt]
+    at = torch.arange(n, device=device)
+    pages, slots = torch.from_numpy(tables[0]).to(device).long()[at // 16], at % 16
+    pick = lambda pair: torch.where(at < first, float(pair[0]), float(pair[1]))
+    code = lambda x: x.to(cache.quantization.dtype).view(torch.int8)
+    cache.codes[pages, 0, 0, 0, slots] = code(pick(codes)[:, None].repeat(1, dim))
+    cache.codes[pages, 0, 0, 0, slots, 0] = 0
+    cache.codes[pages, 0, 1, 0, slots] = code(pick([most if x else 0 for x in v])[:, None].repeat(1, dim))
+    cache.scales[pages, 0, 0, 0, slots] = pick(k_scale)
+    cache.scales[pages, 0, 1, 0, slots] = pick([x / most if x else 1.0 for x in v])
+    return cache, tables
+
+
+@pytest.mark.parametrize("fmt,dim", [("int8", 128), ("fp8_e5m2", 256)])
+@pytest.mark.parametrize("low", [-2e38, -1e30, -1e6])
+@pytest.mark.parametrize("high", [2e38, 1.0])
+@pytest.mark.parametrize("first", [16, 40, 64, 200])
+def test_scores_far_above_all_before(device, fmt, dim, low, high, first):
+    """Keys whose scores (base 2) are near the lowest fp32 holds, or only far below, then
+    others far above them: the difference leaves fp32's range, or holds no digit of the later
+    scores. The later keys take the whole weight, by their own differences: scores equal at the
+    top, or spread over 4 with values that grow along them."""
+    n = 260
+    # base-2 score per K scale of a key of codes 96 in all dimensions but one
+    unit = (dim - 1) * 96 * dim ** -0.5 * 1.4426950408889634
+    cache, tables = _two_groups(device, dim, fmt, n, first, (-96, 96), (-low / unit, high / unit),
+                                (7.0, 1.0))
+    gen = torch.Generator(device=device).manual_seed(first)
+    later = [(int(tables[0, at // 16]), at % 16) for at in range(first, n)]
+    pages, slots = (torch.tensor(x, device=device) for x in zip(*later))
+    spread = torch.rand(len(later), generator=gen, device=device)
+    if high == 1.0:
+        cache.scales[pages, 0, 0, 0, slots] *= 4 * spread
+    cache.scales[pages, 0, 1, 0, slots] *= 0.5 + spread
+    query = torch.ones((9, 1, dim), device=device)
+    for dtype in (torch.float32, torch.bfloat16):
+        _check(cache, tables, [n], [9], query.to(dtype))
