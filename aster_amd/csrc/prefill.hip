@@ -213,6 +213,10 @@ __device__ int scan_tiles(const ChunkArgs& a, int tq, int unit, int* s_wsum, int
 // factor below this keeps every score finite (max code 127; 448 2^-8 for E4M3FN; 57344).
 constexpr float safe_factor() { return KF == kInt8 ? 1.0e29f : KF == kE4M3 ? 1.0e31f : 5.0e26f; }
 
+// A scaled column's factor 2^ex in [kBackLeast, 1] keeps its scores (before the key factor)
+// in range on either side; any other takes the edge path.
+constexpr float kBackLeast = 0x1p-64f;
+
 // A running maximum (base 2) at or below this is none yet to the key steps: they take the
 // scores as they are and then the maximum of these. Reduced by it, a later score far above
 // keeps only the digits that the maximum leaves it (down to kFarMax a step of 2^-13, near
@@ -271,13 +275,13 @@ __device__ __forceinline__ void load_query_tile(const QT* qp, QueryTile<QT, D>& 
       raw.w[cc][i] = reinterpret_cast<const uint4*>(qp + 16 * cc)[i];
 }
 
-// The column's f16 operands. A column whose largest |q| lies in [2^-10, 2^15) (fp32:
-// [2^-3, 2^15)) or is 0 enters as it is: f16 then holds a 16-bit element exactly down to
-// 2^-17, and its own step of 2^-24 is at most 2^-14 of the column's maximum anywhere
-// (fp32: both terms together 2^-21). Any other column is scaled by the exact 2^-ex that
-// brings its maximum into [2^14, 2^15); the return value 2^ex (1 when unscaled, NaN for a
-// non-finite column, which makes each of its scores non-finite as in fp32 arithmetic) goes
-// back onto its scores in the steps' edge path. Cross-lane: uniform control flow.
+// The column's f16 operands. A column whose largest |q| is below 2^15, and at least 2^-3
+// unless q is f16 already, or 0, enters as it is: f16's own step of 2^-24 then rounds an
+// element (a bf16 one below 2^-17, an fp32 one's second term) by 2^-22 of that maximum at
+// most. Any other column is scaled by the exact 2^-ex that brings its maximum into [2^14,
+// 2^15); the return value 2^ex (1 when unscaled, NaN for a non-finite column, which makes
+// each of its scores non-finite as in fp32 arithmetic) goes back onto its scores.
+// Cross-lane: uniform control flow.
 template <typename QT, int D>
 __device__ __forceinline__ float query_operand(const QueryTile<QT, D>& raw, bool valid,
                                                QOp<QT, D>& q) {
@@ -293,7 +297,7 @@ __device__ __forceinline__ float query_operand(const QueryTile<QT, D>& raw, bool
     }
   }
   mx = vmax(mx, shfl_xor(mx, 32));
-  constexpr float kLeast = sizeof(QT) == 4 ? 0x1p-3f : 0x1p-10f;
+  constexpr float kLeast = __is_same(QT, _Float16) ? 0.f : 0x1p-3f;
   float back = 1.f;
   const bool plain = mx == 0.f || (mx >= kLeast && mx < 32768.f);
   if (__ballot(!plain) != 0) {
@@ -489,11 +493,12 @@ struct WaveBounds {
 // the layout that P^T enters the second product in. t = s * ks - m is the base-2 score
 // over the running maximum, p = exp2(t). Bit w of `use` (wave-uniform): block w holds keys
 // some column of the wave sees; of `bounded`: the column bounds [lo, hi] cut into block w.
-// `slow`: a column is scaled or a key factor large. Keys that are all used, not bounded,
-// not padded and not slow take no per-score condition (no score can overflow); otherwise
-// scores are masked to -inf outside the bounds, for padding keys and for unused blocks
-// (whose operands are stale but finite) and checked for non-finite values. vf: the blocks'
-// exponent factors 2^(e_w - ve) on the weights of the numerator only, where `vmix`.
+// `scaled`: a column is scaled; `large`: a key factor is. Keys that are all used, not bounded,
+// not padded and not large take no per-score condition (no score can overflow) unless a column
+// is scaled beyond kBackLeast, only the scaled columns' factors; otherwise scores are masked to
+// -inf outside the bounds, for padding keys and for unused blocks (which repeat the range's
+// last one) and checked for non-finite values. vf: the blocks' exponent factors 2^(e_w - ve)
+// on the weights of the numerator only, where `vmix`.
 //
 // The operands come from LDS well ahead of their MFMAs (a read takes over 100 cycles, and a
 // wave that waits for each pair of them spends more time there than on the arithmetic): the
@@ -509,8 +514,9 @@ __device__ __forceinline__ void load_k_operands(const PrefillLds<D>& L, int buf,
 
 template <typename QT, int D, int NT, typename Between>
 __device__ __forceinline__ void prefill_half(const PrefillLds<D>& L, int buf, int kt, uint32_t use,
-                                             uint32_t bounded, bool masks, bool slow, int kb0,
-                                             half8_t (&kop)[D / 16], Between between,
+                                             uint32_t bounded, bool masks, bool scaled,
+                                             bool large, int kb0, half8_t (&kop)[D / 16],
+                                             Between between,
                                              const QOp<QT, D> (&qop)[NT], const float (&back)[NT],
                                              const int (&lo)[NT], const int (&hi)[NT], int lane,
                                              bool vmix, half2_t vf,
@@ -555,37 +561,48 @@ __device__ __forceinline__ void prefill_half(const PrefillLds<D>& L, int buf, in
   for (int x = 0; x < 4; ++x)
     ks[x] = *reinterpret_cast<const float4_t*>(&L.ks[buf][32 * kt + 8 * x + 4 * h]);
   if constexpr (QOp<QT, D>::kAhead) __builtin_amdgcn_sched_barrier(0);
-  if (use != 3u || bounded != 0 || slow || padded) {
+  if (use != 3u || bounded != 0 || scaled || large || padded) {
     asm volatile("");  // keeps this a branch: if-converted, the interior steps would pay for it
-    // Per-score masks as all-ones/zero words in VGPRs (sign bits of differences, bit
-    // selects): lane masks of unrolled compares would stay live in SGPRs and spill.
-    uint32_t nonfinite = 0;
+    bool far = false;
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const int w = x / 2;
-      const uint32_t pad = masks ? L.pad[buf][8 * kt + 2 * x + h] : 0x01010101u;
-      const bool used = (use >> w) & 1u, bnd = (bounded >> w) & 1u;  // wave-uniform
+    for (int t = 0; t < NT; ++t)
+      far |= __ballot(!(back[t] <= 1.f && back[t] >= kBackLeast)) != 0;
+    if (use == 3u && bounded == 0 && !far && !large && !padded) {  // scaled columns alone
 #pragma unroll
-      for (int y = 0; y < 4; ++y) {
-        const int j = 4 * x + y;
-        const int key = kb0 + 8 * x + 4 * h + y;
-        const int32_t padding = (int32_t)(((pad >> (8 * y)) & 0xffu) - 1u) >> 31;  // -1: padding
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          // -1 when key < lo or key > hi (either difference negative), else 0
-          const int32_t outside = bnd ? ((key - lo[t]) | (hi[t] - key)) >> 31 : 0;
-          const uint32_t hide = used ? (uint32_t)(outside | padding) : 0xffffffffu;
-          // (the factors first: a large query's beside a small key's stays in range)
-          const uint32_t xb = __builtin_bit_cast(uint32_t, s[t][j] * (back[t] * ks[x][y]));
-          // exponent field all ones (inf or NaN) -> bit 31 after the carry
-          nonfinite |= ((xb & 0x7f800000u) + 0x00800000u) & ~hide;
-          s[t][j] = __builtin_bit_cast(float, (xb & ~hide) | (0xff800000u & hide));  // -inf
+        for (int j = 0; j < 16; ++j) s[t][j] *= back[t];
+    } else {
+      // Per-score masks as all-ones/zero words in VGPRs (sign bits of differences, bit
+      // selects): lane masks of unrolled compares would stay live in SGPRs and spill.
+      uint32_t nonfinite = 0;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const int w = x / 2;
+        const uint32_t pad = masks ? L.pad[buf][8 * kt + 2 * x + h] : 0x01010101u;
+        const bool used = (use >> w) & 1u, bnd = (bounded >> w) & 1u;  // wave-uniform
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+          const int j = 4 * x + y;
+          const int key = kb0 + 8 * x + 4 * h + y;
+          const int32_t padding = (int32_t)(((pad >> (8 * y)) & 0xffu) - 1u) >> 31;  // -1: padding
+#pragma unroll
+          for (int t = 0; t < NT; ++t) {
+            // -1 when key < lo or key > hi (either difference negative), else 0
+            const int32_t outside = bnd ? ((key - lo[t]) | (hi[t] - key)) >> 31 : 0;
+            const uint32_t hide = used ? (uint32_t)(outside | padding) : 0xffffffffu;
+            // (the factors first: a large query's beside a small key's stays in range)
+            const uint32_t xb = __builtin_bit_cast(uint32_t, s[t][j] * (back[t] * ks[x][y]));
+            // exponent field all ones (inf or NaN) -> bit 31 after the carry
+            nonfinite |= ((xb & 0x7f800000u) + 0x00800000u) & ~hide;
+            s[t][j] = __builtin_bit_cast(float, (xb & ~hide) | (0xff800000u & hide));  // -inf
+          }
+          static_assert(NT == 1, "the scores hold the one column tile's factors from here on");
+          ks[x][y] = 1.f;
         }
-        static_assert(NT == 1, "the scores hold the one column tile's factors from here on");
-        ks[x][y] = 1.f;
       }
+      if (__ballot((nonfinite >> 31) != 0) != 0) bad_score = true;
     }
-    if (__ballot((nonfinite >> 31) != 0) != 0) bad_score = true;
   }
   bool need = false;
   float me[NT], tmax[NT];
@@ -838,15 +855,15 @@ __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L
       bounded &= use;
     }
     if (use != 0) {
-      prefill_half<QT, D, NT>(L, buf, 0, use & 3u, bounded & 3u, masks, scaled | large, kb0, kop,
+      prefill_half<QT, D, NT>(L, buf, 0, use & 3u, bounded & 3u, masks, scaled, large, kb0, kop,
                               [&]() __attribute__((always_inline)) {
                                 load_k_operands<D>(L, buf, 1, lane, kop);
                               },
                               qop, back, lo, hi, lane, vmix, half2_t{vf[0], vf[1]}, acc, m, l,
                               bad_score);
-      prefill_half<QT, D, NT>(L, buf, 1, use >> 2, bounded >> 2, masks, scaled | large, kb0 + 32,
-                              kop, []() {}, qop, back, lo, hi, lane, vmix, half2_t{vf[2], vf[3]},
-                              acc, m, l, bad_score);
+      prefill_half<QT, D, NT>(L, buf, 1, use >> 2, bounded >> 2, masks, scaled, large,
+                              kb0 + 32, kop, []() {}, qop, back, lo, hi, lane, vmix,
+                              half2_t{vf[2], vf[3]}, acc, m, l, bad_score);
     }
     if (i + 1 < nsteps) {
       // the other buffer was last read in step i - 1, before the barrier that ended it

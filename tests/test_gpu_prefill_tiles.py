@@ -66,18 +66,17 @@ def test_tile_edges(device, dim, kv, group, dtype, fmt):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("power", [-40, -14, -9, 13])
+@pytest.mark.parametrize("power", [-70, -40, -14, -9, -4, 13])
 def test_scaled_columns(device, dtype, power):
-    """Queries whose columns leave the unscaled range, one head in two; the scale keeps
-    the scores ordinary."""
-    if dtype == torch.float16 and power not in (-9, 13):
+    """Queries whose columns leave the unscaled range beside zero ones, in prompt and history
+    keys; key scales of 2^-power keep the scores ordinary."""
+    if dtype == torch.float16 and power < -9:
         pytest.skip("outside fp16")
-    lens, counts = [100, 50], [40, 17]
+    lens, counts = [100, 350], [40, 17]
     cache, tables, gen = _cache(device, lens, 128, 2, "int8", 7)
-    query = torch.randn((sum(counts), 8, 128), generator=gen, device=device)
-    query[:, ::2] *= 2.0 ** power
-    if power > 0:  # scores stay within exp's range
-        cache.scales[:, :, 0] *= 2.0 ** -power
+    query = torch.randn((sum(counts), 8, 128), generator=gen, device=device) * 2.0 ** power
+    query[:, 1::2] = 0
+    cache.scales[:, :, 0] *= 2.0 ** -power
     _check(cache, tables, lens, counts, query.to(dtype))
 
 
@@ -222,3 +221,19 @@ def test_scores_far_above_all_before(device, fmt, dim, low, high, first):
     query = torch.ones((9, 1, dim), device=device)
     for dtype in (torch.float32, torch.bfloat16):
         _check(cache, tables, [n], [9], query.to(dtype))
+
+
+@pytest.mark.parametrize("fmt", ["int8", "fp8_e4m3fn"])
+@pytest.mark.parametrize("power", [-10, -7, -4])
+def test_small_bf16_columns(device, power, fmt):
+    """A bf16 column with one element at 2^power that meets zero codes, and the others near
+    2^-19: f16's own step (2^-24) would cost those 1.5 % of themselves, 9 % of the later keys'
+    weight 6 nats below the first key's. Tolerance (5e-3, relative alone): the bf16 output
+    (2^-9) beside f16 weights and V scales (2^-12 each)."""
+    n, dim = 100, 128
+    query = torch.full((9, 2, dim), 2.0 ** -19 * (1 + 2 / 128), device=device)
+    query[..., 0] = 2.0 ** power
+    query = query.bfloat16()
+    unit = float(query[0, 0, 1]) * (dim - 1) * 2 * 96 * dim ** -0.5  # score difference per K scale
+    cache, tables = _two_groups(device, dim, fmt, n, 1, (96, -96), (6 / unit, 6 / unit), (0.0, 1.0))
+    _check(cache, tables, [n], [9], query, atol=0)
