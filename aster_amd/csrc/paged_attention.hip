@@ -152,15 +152,19 @@ namespace {
 //   - every row must carry max_query_len tokens where the call has num_seqs times as many
 //     (a prompt alone, equal chunks); an offset array that says otherwise is served all
 //     the same;
-//   - contexts up to 512 keys are at most 8 key steps of ~2 us for a one-token row, which
-//     runs beside the chunks' units, no longer than the launches it replaces, while every
-//     row has a CU of its own.
+//   - contexts up to 512 keys, where every row has a CU of its own. A one-token row is then a
+//     unit of 8 key steps at most, beside the chunks' units instead of before them. 20 such
+//     rows and 2 chunks of 16 to 64 tokens, 32/8 heads of 128, int8, with their append:
+//     contexts of 128 29.4 -> 19.3 us a call, 512 43.6 -> 27.6; two rows 28.2 -> 19.5 and
+//     39.2 -> 25.9; 50 rows, 16/4 heads of 256, 38.2 -> 22.7 and 67.1 -> 44.3. (It was faster
+//     up to the 2048 keys tried.)
 // Not for fp32 queries: one-token rows of theirs are attended in exact fp32, and only the
-// offsets on the device say whether there are any.
+// offsets on the device say whether there are any. Nor for the group that the decode kernels
+// refuse (16 heads of 256): whether a call is taken does not hang on its chunks' lengths.
 constexpr int kOnlyChunksContext = 512;
 bool only_chunks(int32_t q_dtype, int32_t tokens, int32_t max_query_len, int32_t num_seqs,
-                 int32_t num_kv_heads, int32_t max_context_len) {
-  if (q_dtype == ASTR_F32) return false;
+                 int32_t num_kv_heads, int32_t group, int32_t head_dim, int32_t max_context_len) {
+  if (q_dtype == ASTR_F32 || (head_dim == 256 && group == 16)) return false;
   if ((int64_t)num_seqs * max_query_len == tokens) return true;
   return max_context_len <= kOnlyChunksContext &&
          (int64_t)num_seqs * num_kv_heads <= device_cus();
@@ -368,7 +372,7 @@ int paged_attention(const astr_paged_kv* cache, const void* query, int32_t q_dty
   a.pf_ws = static_cast<float*>(workspace);
   a.pf_bytes = fixed_scratch || need == 0 ? 0 : need;
   if (chunks && only_chunks(q_dtype, num_query_tokens, max_query_len, num_seqs,
-                            cache->num_kv_heads, max_context_len)) {
+                            cache->num_kv_heads, group, cache->head_dim, max_context_len)) {
     a.pf_min_rows = 1;
     return launch_prefill(a, q_dtype, s);
   }

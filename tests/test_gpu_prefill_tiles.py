@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from aster_amd import KVQuantization, PagedKVCache
+from aster_amd.attention_backend import UnsupportedAttentionBackend
 from tests.gpu_util import oracle_decode
 
 pytestmark = pytest.mark.gpu
@@ -177,6 +178,16 @@ def test_one_token_rows_beside_chunks(device, dtype):
     np.testing.assert_allclose(out[:9].float().cpu().numpy(), want, atol=2e-3, rtol=5e-3)
     if dtype == torch.float32:  # one-token rows in exact fp32: sums of 50 terms of order 1
         np.testing.assert_allclose(out[0].cpu().numpy(), want[0], atol=2e-5, rtol=0)
+
+
+@pytest.mark.parametrize("counts", [[16], [16, 16], [16, 3]])
+def test_group_of_16_at_head_dim_256_is_refused(device, counts):
+    """16-bit queries in groups the decode kernels do not take, whatever the chunks' lengths."""
+    lens = [n + 40 for n in counts]
+    cache, tables, gen = _cache(device, lens, 256, 1, "int8", 3)
+    query = torch.randn((sum(counts), 16, 256), generator=gen, device=device).bfloat16()
+    with pytest.raises(UnsupportedAttentionBackend, match="group size 16"):
+        _check(cache, tables, lens, counts, query)
 
 
 def _two_groups(device, dim, fmt, n, first, codes, k_scale, v):
