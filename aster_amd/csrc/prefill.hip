@@ -224,6 +224,7 @@ constexpr float kBackLeast = 0x1p-64f;
 // whose scores all lie there takes the rescale on every step.
 constexpr float kFarMax = -2048.f;
 
+typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef float float16v_t __attribute__((ext_vector_type(16)));
 
 // Maximum and sum over a lane and the one 32 away (v_permlane32_swap_b32: the pair of
@@ -1075,55 +1076,99 @@ __global__ __launch_bounds__(256, (prefill_occupancy<QT, D>())) void prefill_mfm
                       bounds_of, store, []() { return true; }, [](int) {});
 }
 
-// Merges the pieces of split units, one workgroup per unit: each lane the part of its
-// column that it held in the pieces, with the merge_softmax rule
-// (online_attention.py:42-63).
+constexpr int kMostPieces = 16;
+
+// Merges the pieces of split units with the merge_softmax rule (online_attention.py:42-63). A
+// lane takes one of the four parts of its column as it held it in the pieces: a workgroup one
+// part of a unit's 128 columns. Bound by the chain of its loads: the statistics
+// and the first pieces' rows, whose place the unit's index alone gives, are on their way while
+// the dispatch plan is worked out (a place past the unit's own pieces is read, inside the
+// workspace, and not used). 512 tokens on 16000 (32/8 heads of 128: 34 MB of
+// partials) 14.1 -> 10.1 us against a workgroup per unit that read the plan, the statistics and
+// the rows of one piece after another; 256 tokens on 8000 (16/4 heads, 16 pieces a unit) 71.0 ->
+// 47.1 us a call.
+template <int D>
+struct MergeShape {
+  static constexpr int kParts = 4;         // parts of a lane's column
+  static constexpr int kRows = D / 32;     // float4 rows of one in a piece
+  static constexpr int kAtOnce = 512 / D;  // pieces whose rows are in flight together
+};
+
 template <typename QT, int D, int G>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(ChunkArgs a) {
+  using Partial = PiecePartial<D>;
+  using M = MergeShape<D>;
   constexpr int TQ = PrefillShape<D>::kCols / G;
   __shared__ int tab[PlanTab::kInts];
   __shared__ int s_wsum[kWaves], s_found[2];
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int part = blockIdx.x % M::kParts, unit = blockIdx.x / M::kParts;
+  const int64_t first = (int64_t)unit * a.pf_pieces;
+  if ((uint64_t)(first + a.pf_pieces) * Partial::kFloats * sizeof(float) > a.pf_bytes) return;
+  float* const base = a.pf_ws + first * Partial::kFloats;
+
+  const int col = Partial::kAcc + (wave * 32 + (lane & 31)) * 2;
+  float2_t ml[kMostPieces];
+#pragma unroll
+  for (int j = 0; j < kMostPieces; ++j)
+    if (j < a.pf_pieces)
+      ml[j] = *reinterpret_cast<const float2_t*>(base + j * (int64_t)Partial::kFloats + col);
+  float4_t v[M::kAtOnce][M::kRows];
+  auto load_rows = [&](int j0, int pieces) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < M::kAtOnce; ++j)
+      if (j0 + j < pieces)
+#pragma unroll
+        for (int n = 0; n < M::kRows; ++n)
+          v[j][n] = *Partial::acc(base + (j0 + j) * (int64_t)Partial::kFloats, wave, n, part, lane);
+  };
+  load_rows(0, a.pf_pieces);
+
   int rows;
   const int per_kv = count_units(a, TQ, tab, s_wsum, s_found, rows);
-  if ((int64_t)blockIdx.x >= (int64_t)per_kv * a.cache.num_kv_heads) return;
-  const int kvh = blockIdx.x / per_kv;
+  if ((int64_t)unit >= (int64_t)per_kv * a.cache.num_kv_heads) return;
+  const int kvh = unit / per_kv;
   UnitRef u;
-  if (!unit_ref(a, TQ, tab, s_wsum, s_found, rows, blockIdx.x % per_kv, u)) return;
+  if (!unit_ref(a, TQ, tab, s_wsum, s_found, rows, unit % per_kv, u)) return;
   const TileSpan span = tile_span(a, clamp_ctx(a, u.ctx_raw, false), u.n, u.tile, TQ);
   const int steps = (span.b_hi - span.b_lo + kWaves - 1) / kWaves;
   const int pieces = min((steps + a.pf_steps - 1) / a.pf_steps, a.pf_pieces);
-  const int64_t first = (int64_t)blockIdx.x * a.pf_pieces;
-  if (pieces <= 1 || (uint64_t)(first + pieces) * PiecePartial<D>::kFloats * sizeof(float) > a.pf_bytes)
-    return;
-  float* const base = a.pf_ws + first * PiecePartial<D>::kFloats;
-  const int64_t col = PiecePartial<D>::kAcc + (wave * 32 + (lane & 31)) * 2;
+  if (pieces <= 1) return;
   float mx = -FLT_MAX;
-  for (int j = 0; j < pieces; ++j) mx = fmaxf(mx, base[j * (int64_t)PiecePartial<D>::kFloats + col]);
-  float16v_t acc[D / 32];
 #pragma unroll
-  for (int n = 0; n < D / 32; ++n)
+  for (int j = 0; j < kMostPieces; ++j)
+    if (j < pieces) mx = fmaxf(mx, ml[j][0]);
+  float4_t acc[M::kRows];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) acc[n][j] = 0.f;
+  for (int n = 0; n < M::kRows; ++n) acc[n] = float4_t{};
   float l = 0.f;
-  for (int j = 0; j < pieces; ++j) {
-    float* const p = base + j * (int64_t)PiecePartial<D>::kFloats;
-    const float w = __builtin_amdgcn_exp2f(p[col] - mx);
-    l = fmaf(p[col + 1], w, l);
 #pragma unroll
-    for (int n = 0; n < D / 32; ++n)
+  for (int j0 = 0; j0 < kMostPieces; j0 += M::kAtOnce) {
+    if (j0 > 0) load_rows(j0, pieces);
 #pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        const float4_t v = *PiecePartial<D>::acc(p, wave, n, x, lane);
+    for (int j = 0; j < M::kAtOnce; ++j)
+      if (j0 + j < pieces) {
+        const float w = __builtin_amdgcn_exp2f(ml[j0 + j][0] - mx);
+        l = fmaf(ml[j0 + j][1], w, l);
 #pragma unroll
-        for (int y = 0; y < 4; ++y) acc[n][4 * x + y] = fmaf(v[y], w, acc[n][4 * x + y]);
+        for (int n = 0; n < M::kRows; ++n)
+#pragma unroll
+          for (int y = 0; y < 4; ++y) acc[n][y] = fmaf(v[j][n][y], w, acc[n][y]);
       }
   }
   const int f = wave * 32 + (lane & 31);
   const int token = span.t0 + f / G;
-  if (token < span.t1)
-    store_column<QT, D>(a, acc, 1.f / fmaxf(l, FLT_MIN), u.q0 + token, kvh * G + f % G, lane);
+  if (token >= span.t1) return;
+  const float inv = 1.f / fmaxf(l, FLT_MIN);
+  float o[D / 8];
+#pragma unroll
+  for (int y = 0; y < 4; ++y)
+#pragma unroll
+    for (int n = 0; n < M::kRows; ++n) o[y * M::kRows + n] = acc[n][y] * inv;
+  store_run<QT, D / 8>(static_cast<QT*>(a.out) + (int64_t)(u.q0 + token) * a.o_tok +
+                           (int64_t)(kvh * G + f % G) * a.o_head + D / 4 * part +
+                           D / 8 * (lane >> 5), o);
 }
 
 // Prefix tiles of a decode plan (decode_plan.cpp): the shared blocks of sequences whose
@@ -1302,8 +1347,6 @@ int prefill_cus() {
 // Key steps below which a unit is not split: a piece costs its start (~2 steps) and its
 // partial, written and read again.
 constexpr int kLeastPieceSteps = 8;
-constexpr int kMostPieces = 16;
-
 template <typename QT, int D, int G>
 int launch(ChunkArgs a, hipStream_t stream) {
   constexpr int TQ = PrefillShape<D>::kCols / G;
@@ -1336,8 +1379,9 @@ int launch(ChunkArgs a, hipStream_t stream) {
   hipLaunchKernelGGL((prefill_mfma_kernel<QT, D, G>), dim3((uint32_t)grid), dim3(kWaves * kWave),
                      0, stream, a);
   if (a.pf_pieces > 1)
-    hipLaunchKernelGGL((prefill_merge_kernel<QT, D, G>), dim3((uint32_t)max_units),
-                       dim3(kWaves * kWave), 0, stream, a);
+    hipLaunchKernelGGL((prefill_merge_kernel<QT, D, G>),
+                       dim3((uint32_t)max_units * MergeShape<D>::kParts), dim3(kWaves * kWave), 0,
+                       stream, a);
   const hipError_t err = hipGetLastError();
   return err == hipSuccess ? 0 : hip_fail(err, "paged_attention (prefill) launch");
 }

@@ -9,7 +9,7 @@ import torch
 
 from aster_amd import KVQuantization, PagedKVCache
 from aster_amd.attention_backend import UnsupportedAttentionBackend
-from tests.gpu_util import oracle_decode
+from tests.gpu_util import mark_padding, oracle_decode
 
 pytestmark = pytest.mark.gpu
 
@@ -36,16 +36,17 @@ def _cache(device, rows, dim, kv, fmt, seed):
     return cache, tables, gen
 
 
-def _check(cache, tables, lens, counts, query, window=None, atol=2e-3, rtol=2e-3, bound=None):
+def _check(cache, tables, lens, counts, query, window=None, atol=2e-3, rtol=2e-3, bound=None,
+           causal=True, **options):
     device = query.device
     starts = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
     out = cache.paged_attention(0, query, torch.from_numpy(tables).to(device),
                                 torch.from_numpy(np.array(lens, np.int32)).to(device),
                                 max_context_len=bound or max(lens), window=window,
                                 query_start_loc=torch.from_numpy(starts).to(device),
-                                max_query_len=max(counts), check=True)
+                                max_query_len=max(counts), causal=causal, check=True, **options)
     want = oracle_decode(tables, cache, query, context_lens=np.array(lens, np.int32),
-                         scale=cache.head_dim ** -0.5, window=window,
+                         scale=cache.head_dim ** -0.5, window=window, causal=causal,
                          query_lens=np.array(counts, np.int32), fp64=True)
     bf16 = query.dtype == torch.bfloat16  # outputs rounded to 2^-9 of themselves
     np.testing.assert_allclose(out.float().cpu().numpy(), want, atol=atol,
@@ -248,3 +249,42 @@ def test_small_bf16_columns(device, power, fmt):
     unit = float(query[0, 0, 1]) * (dim - 1) * 2 * 96 * dim ** -0.5  # score difference per K scale
     cache, tables = _two_groups(device, dim, fmt, n, 1, (96, -96), (6 / unit, 6 / unit), (0.0, 1.0))
     _check(cache, tables, [n], [9], query, atol=0)
+
+
+@pytest.mark.parametrize("fmt", ["int8", "fp8_e4m3fn"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("part", [0, 256])
+def test_split_units_beside_decode_rows(device, part, dtype, fmt):
+    """A split chunk's partials take the workspace that the decode rows' partials, tables and
+    merges of the same call used, in group 1, with padding, and with rows that see every key
+    (non-causal) within a window, whose last piece takes what the bound left out."""
+    counts, priors = [1, 40, 1, 1, 9], [2500, 3000, 17, 4096, 1500]
+    lens = [n + p for n, p in zip(counts, priors)]
+    cache, tables, gen = _cache(device, lens, 128, 2, fmt, 19)
+    query = torch.randn((sum(counts), 2, 128), generator=gen, device=device).to(dtype)
+    _check(cache, tables, lens, counts, query, partition_tokens=part)
+    _check(cache, tables, lens, counts, query, partition_tokens=part, window=700, causal=False)
+    mark_padding(cache, tables, lens, 0.2, seed=3)
+    _check(cache, tables, lens, counts, query, partition_tokens=part)
+
+
+def test_split_units_of_many_rows(device):
+    """More chunk rows than the dispatch plan orders (256), with histories that split."""
+    rng = np.random.default_rng(23)
+    priors = rng.integers(0, 60, 300)
+    priors[::50] = rng.integers(900, 1500, 6)
+    counts = [2] * 299 + [3]
+    lens = [int(n + p) for n, p in zip(counts, priors)]
+    cache, tables, gen = _cache(device, lens, 64, 1, "int8", 23)
+    query = torch.randn((sum(counts), 1, 64), generator=gen, device=device).half()
+    _check(cache, tables, lens, counts, query)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_split_units_by_number_of_pieces(device, dtype):
+    """One to sixteen pieces a unit under one bound, heads in groups of 1."""
+    counts, priors = [7, 130, 3, 2], [100, 1030, 5000, 17000]
+    lens = [n + p for n, p in zip(counts, priors)]
+    cache, tables, gen = _cache(device, lens, 128, 1, "int8", 29)
+    query = torch.randn((sum(counts), 1, 128), generator=gen, device=device).to(dtype)
+    _check(cache, tables, lens, counts, query)
