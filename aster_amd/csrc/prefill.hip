@@ -7,7 +7,8 @@
 //   k <= p (causal; else k < ctx)  and  k > p - window (window > 0).
 //
 // Work unit: (kv head, sequence, tile of TQ query tokens), TQ * G = 128 (token, head)
-// columns of one kv head, 32 per wave. The unit's visible key range is streamed in steps
+// columns of one kv head, 32 per wave (64 columns and half of each key step per wave where a
+// head-dim 256 call leaves CUs idle, PrefillShape). The unit's visible key range is streamed in steps
 // of four 16-token blocks; each wave loads one block of the step into registers and
 // converts it once, one step ahead, into f16 operands in LDS that all four waves read:
 //   S^T[t][c]  = K[t][:] . Q[c][:]     v_mfma_f32_32x32x16_f16: the K codes (exact in f16)
@@ -58,10 +59,14 @@ static __device__ long long g_ttrace[kTileTraceWaves][8];
 static __device__ int g_ttrace_info[kTileTraceWaves][4];
 #endif
 
-template <int D>
+// KS = 2: the waves are two column groups and two halves of every key step (32 of its 64
+// keys), whose states merge at the unit's end: half the columns, and half the chain of MFMAs
+// and operand reads per step, for grids that leave CUs idle (launch()).
+template <int D, int KS = 1>
 struct PrefillShape {
-  static constexpr int NT = 1;                    // 32-column MFMA tiles per wave
-  static constexpr int kCols = kWaves * 32 * NT;  // (token, head) columns per workgroup
+  static constexpr int NT = 1;                         // 32-column MFMA tiles per wave
+  static constexpr int kGroups = kWaves / KS;          // column groups (waves that store)
+  static constexpr int kCols = kGroups * 32 * NT;      // (token, head) columns per workgroup
 };
 
 // Workgroups per CU: the LDS holds one at head dim 256 (130 KB), the registers two at 128
@@ -224,8 +229,8 @@ constexpr float kBackLeast = 0x1p-64f;
 // whose scores all lie there takes the rescale on every step.
 constexpr float kFarMax = -2048.f;
 
-typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef float float16v_t __attribute__((ext_vector_type(16)));
+typedef float float2_t __attribute__((ext_vector_type(2)));
 
 // Maximum and sum over a lane and the one 32 away (v_permlane32_swap_b32: the pair of
 // results holds the low half's and the high half's value in every lane).
@@ -258,6 +263,13 @@ struct QOp {
   // terms at head dim 128 and 256 leave none; at head dim 64 a third wave per SIMD is worth
   // more, ragged FP8 prompts 83.9 -> 76.8 us)
   static constexpr bool kAhead = kTerms == 1 && D >= 128;
+  // else how many operands are read ahead of their use (one wave per SIMD at head dim 256 has
+  // no other to cover a read: 1500 tokens, 16/4 heads, 119 -> 101 us)
+  static constexpr int kDepth = !kAhead && D == 256 ? 4 : 0;
+  // whether a block's padding bytes are loaded with it (at head dim 256 their register spills,
+  // and the spill waits for every load of the block right after its issue: 1500 tokens in bf16,
+  // 16/4 heads, 98.2 us instead of 86.5)
+  static constexpr bool kPad = kAhead && D < 256;
   half8_t op[kTerms][D / 16];
 };
 
@@ -542,6 +554,12 @@ __device__ __forceinline__ void prefill_half(const PrefillLds<D>& L, int buf, in
     load_v(0, kAhead);
     __builtin_amdgcn_sched_barrier(0);
   }
+  constexpr int kDepth = QOp<QT, D>::kDepth;
+  auto load_k = [&](int cc) __attribute__((always_inline)) {
+    kop[cc] = __builtin_bit_cast(half8_t, L.k[buf][(kt * Lds::kChunks + cc) * kWave + lane]);
+  };
+#pragma unroll
+  for (int cc = 0; cc < kDepth; ++cc) load_k(cc);
   float16v_t s[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
@@ -549,8 +567,12 @@ __device__ __forceinline__ void prefill_half(const PrefillLds<D>& L, int buf, in
     for (int j = 0; j < 16; ++j) s[t][j] = 0.f;
 #pragma unroll
   for (int cc = 0; cc < Lds::kChunks; ++cc) {
-    if constexpr (!QOp<QT, D>::kAhead)
-      kop[cc] = __builtin_bit_cast(half8_t, L.k[buf][(kt * Lds::kChunks + cc) * kWave + lane]);
+    if constexpr (kDepth > 0) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (cc + kDepth < Lds::kChunks) load_k(cc + kDepth);
+    } else if constexpr (!QOp<QT, D>::kAhead) {
+      load_k(cc);
+    }
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -655,6 +677,7 @@ __device__ __forceinline__ void prefill_half(const PrefillLds<D>& L, int buf, in
     between();
     __builtin_amdgcn_sched_barrier(0);
   }
+  load_v(0, kDepth);
   // (the sums are done here: sunk past the branch, they would keep a second copy of the weights)
 #pragma unroll
   for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(l[t]));
@@ -673,7 +696,12 @@ __device__ __forceinline__ void prefill_half(const PrefillLds<D>& L, int buf, in
 #pragma unroll
     for (int n = 0; n < Lds::kRowsN; ++n) {
       const int x = w * Lds::kRowsN + n;
-      if constexpr (!QOp<QT, D>::kAhead) load_v(x, x + 1);
+      if constexpr (kDepth > 0) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (x + kDepth < 2 * Lds::kRowsN) load_v(x + kDepth, x + kDepth + 1);
+      } else if constexpr (!QOp<QT, D>::kAhead) {
+        load_v(x, x + 1);
+      }
 #pragma unroll
       for (int t = 0; t < NT; ++t)
         acc[t][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
@@ -721,16 +749,19 @@ __device__ __forceinline__ void acc_run(const float16v_t (&acc)[D / 32], int x, 
 // before any column is read: it returns false (uniformly) to end the unit there, with
 // nothing stored. mark(k) is called at the unit's timeline marks 2-5 (the tile kernel's
 // trace builds).
-template <typename QT, int D, typename ColumnOf, typename BoundsOf, typename Store,
+template <typename QT, int D, int KS, typename ColumnOf, typename BoundsOf, typename Store,
           typename Prologue, typename Mark>
 __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L, int kvh,
                                              int b_lo, int b_hi, const int32_t* blocks, int q0,
                                              int t0, ColumnOf column_of, BoundsOf bounds_of,
                                              Store store, Prologue prologue, Mark mark) {
-  constexpr int NT = PrefillShape<D>::NT;
+  using Shape = PrefillShape<D, KS>;
+  constexpr int NT = Shape::NT;
   constexpr int kRowsN = D / 32;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int lane = threadIdx.x % kWave;
+  const int group = KS == 1 ? wave : wave % Shape::kGroups;
+  const int half = KS == 1 ? 0 : wave / Shape::kGroups;
   const int nsteps = (b_hi - b_lo + kWaves - 1) / kWaves;
 
   // Block b_lo + 4 * step + w is wave w's; its id is read (a scalar load) one step before
@@ -748,7 +779,7 @@ __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L
   QueryTile<QT, D> qraw[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const ColumnInfo c = column_of((wave * NT + t) * 32 + (lane & 31));
+    const ColumnInfo c = column_of((group * NT + t) * 32 + (lane & 31));
     lo[t] = c.valid ? c.lo : INT_MAX;
     hi[t] = c.valid ? c.hi : -1;
     // an invalid column reads token t0's row (in range) and is zeroed
@@ -766,7 +797,7 @@ __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L
       bad_index = true;
       id = 0;
     }
-    load_raw<D, QOp<QT, D>::kAhead>(a, id, kvh, lane, masks, raw);
+    load_raw<D, QOp<QT, D>::kPad>(a, id, kvh, lane, masks, raw);
   };
   if (QOp<QT, D>::kAhead && nsteps > 0) load_step(0);
 
@@ -778,7 +809,7 @@ __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L
     back[t] = query_operand<QT, D>(qraw[t], hi[t] >= 0, qop[t]);
     scaled |= __ballot(back[t] != 1.f) != 0;
   }
-  const WaveBounds wb = bounds_of(wave);
+  const WaveBounds wb = bounds_of(group);
   mark(2);
 
   float16v_t acc[NT][kRowsN];
@@ -805,14 +836,14 @@ __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L
   const int inner_hi = wb.any && inner_end > 0 ? inner_end / kStepKeys : 0;
   if (nsteps > 0) {
     if constexpr (!QOp<QT, D>::kAhead) load_step(0);
-    convert_raw<D, QOp<QT, D>::kAhead>(a, raw, L, 0, wave, lane, masks, ve, vlim);
+    convert_raw<D, QOp<QT, D>::kPad>(a, raw, L, 0, wave, lane, masks, ve, vlim);
     if (nsteps > 1) load_step(1);
     __syncthreads();
   }
   for (int i = 0; i < nsteps; ++i) {
     const int buf = i & 1;
     half8_t kop[D / 16];
-    if constexpr (QOp<QT, D>::kAhead) load_k_operands<D>(L, buf, 0, lane, kop);
+    if constexpr (QOp<QT, D>::kAhead) load_k_operands<D>(L, buf, KS == 2 ? half : 0, lane, kop);
     // the step's block exponents (each at least ve at its conversion): a larger one
     // becomes the new ve (the accumulators scale by the exact 2^(ve_old - ve)); blocks
     // converted below it weigh their products by 2^(e_w - ve)
@@ -855,7 +886,14 @@ __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L
       }
       bounded &= use;
     }
-    if (use != 0) {
+    if constexpr (KS == 2) {
+      const uint32_t mine = use >> (2 * half) & 3u;
+      if (mine != 0)
+        prefill_half<QT, D, NT>(L, buf, half, mine, bounded >> (2 * half) & 3u, masks, scaled,
+                                large, kb0 + 32 * half, kop, []() {}, qop, back, lo, hi, lane, vmix,
+                                half != 0 ? half2_t{vf[2], vf[3]} : half2_t{vf[0], vf[1]}, acc, m,
+                                l, bad_score);
+    } else if (use != 0) {
       prefill_half<QT, D, NT>(L, buf, 0, use & 3u, bounded & 3u, masks, scaled, large, kb0, kop,
                               [&]() __attribute__((always_inline)) {
                                 load_k_operands<D>(L, buf, 1, lane, kop);
@@ -868,7 +906,7 @@ __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L
     }
     if (i + 1 < nsteps) {
       // the other buffer was last read in step i - 1, before the barrier that ended it
-      convert_raw<D, QOp<QT, D>::kAhead>(a, raw, L, buf ^ 1, wave, lane, masks, ve, vlim);
+      convert_raw<D, QOp<QT, D>::kPad>(a, raw, L, buf ^ 1, wave, lane, masks, ve, vlim);
       if (i + 2 < nsteps) load_step(i + 2);
     }
     __syncthreads();
@@ -877,12 +915,46 @@ __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L
   mark(4);
   if (bad_index && lane == 0) atomicOr(a.err_flag, ASTR_FLAG_BAD_INDEX);
   if (bad_score && lane == 0) atomicOr(a.err_flag, ASTR_FLAG_NONFINITE_SCORE);
+  if constexpr (KS == 2) {
+    // the second half's state through the operand buffers (last read before the barrier that
+    // ended the last step), in the merge_softmax rule (online_attention.py:42-63)
+    static_assert(Shape::kGroups * kRowsN * 4 * kWave * sizeof(float4_t) <= sizeof(L.k) &&
+                      Shape::kGroups * kWave * sizeof(float2_t) <= sizeof(L.v),
+                  "the groups' states fit the buffers");
+    float4_t* const o = reinterpret_cast<float4_t*>(L.k) + group * kRowsN * 4 * kWave + lane;
+    float2_t* const ml = reinterpret_cast<float2_t*>(L.v) + group * kWave + lane;
+    if (half != 0) {
+#pragma unroll
+      for (int n = 0; n < kRowsN; ++n)
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          o[(n * 4 + x) * kWave] = float4_t{acc[0][n][4 * x], acc[0][n][4 * x + 1],
+                                            acc[0][n][4 * x + 2], acc[0][n][4 * x + 3]};
+      *ml = float2_t{m[0], l[0]};
+    }
+    __syncthreads();
+    if (half != 0) return;
+    const float2_t other = *ml;
+    const float mn = fmaxf(m[0], other[0]);
+    const float w0 = __builtin_amdgcn_exp2f(m[0] - mn), w1 = __builtin_amdgcn_exp2f(other[0] - mn);
+    m[0] = mn;
+    l[0] = l[0] * w0 + other[1] * w1;
+#pragma unroll
+    for (int n = 0; n < kRowsN; ++n)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const float4_t v = o[(n * 4 + x) * kWave];
+#pragma unroll
+        for (int y = 0; y < 4; ++y)
+          acc[0][n][4 * x + y] = fmaf(v[y], w1, acc[0][n][4 * x + y] * w0);
+      }
+  }
 
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     // worked out again: kept through the steps it would cost registers (the empty asm hides
     // that it is the same value)
-    int f = (wave * NT + t) * 32 + (lane_id() & 31);
+    int f = (group * NT + t) * 32 + (lane_id() & 31);
     asm volatile("" : "+v"(f));
     store(t, acc[t], m[t], sum32(l[t]), ve, column_of(f));
   }
@@ -941,11 +1013,11 @@ __device__ __forceinline__ bool unit_ref(const ChunkArgs& a, int tq, int* tab, i
 // The partial of one piece of a split unit: the accumulators as the lanes hold them
 // (float4 x of operand n of wave w at ((w * D / 32 + n) * 4 + x) * 64 + lane), then (m, l)
 // per column.
-template <int D>
+template <int D, int KS>
 struct PiecePartial {
-  static constexpr int kAcc = kWaves * (D / 32) * 4 * kWave * 4;  // floats
-  static constexpr int kFloats = kAcc + PrefillShape<D>::kCols * 2;
-  static_assert(PrefillShape<D>::NT == 1, "one column tile per wave");
+  static constexpr int kAcc = PrefillShape<D, KS>::kGroups * (D / 32) * 4 * kWave * 4;  // floats
+  static constexpr int kFloats = kAcc + PrefillShape<D, KS>::kCols * 2;
+  static_assert(PrefillShape<D, KS>::NT == 1, "one column tile per wave");
   __device__ static float4_t* acc(float* base, int wave, int n, int x, int lane) {
     return reinterpret_cast<float4_t*>(base) + ((wave * (D / 32) + n) * 4 + x) * kWave + lane;
   }
@@ -966,12 +1038,12 @@ __device__ __forceinline__ void store_column(const AttnArgs& a, const float16v_t
   }
 }
 
-template <typename QT, int D, int G>
+template <typename QT, int D, int G, int KS>
 __global__ __launch_bounds__(256, (prefill_occupancy<QT, D>())) void prefill_mfma_kernel(ChunkArgs a) {
   static_assert(D == 64 || D == 128 || D == 256, "head_dim");
-  constexpr int NT = PrefillShape<D>::NT;
-  constexpr int TQ = PrefillShape<D>::kCols / G;
-  static_assert(PrefillShape<D>::kCols % G == 0, "GQA group must divide the column tile");
+  constexpr int NT = PrefillShape<D, KS>::NT;
+  constexpr int TQ = PrefillShape<D, KS>::kCols / G;
+  static_assert(PrefillShape<D, KS>::kCols % G == 0, "GQA group must divide the column tile");
 
   // one struct, the operand buffers at its start: every LDS address of the key steps then
   // has a constant offset
@@ -1023,11 +1095,11 @@ __global__ __launch_bounds__(256, (prefill_occupancy<QT, D>())) void prefill_mfm
     const int steps = (span.b_hi - span.b_lo + kWaves - 1) / kWaves;
     if (piece > 0 && piece * a.pf_steps >= steps) return;
     if (steps > a.pf_steps) {
-      if ((uint64_t)(logical + 1) * PiecePartial<D>::kFloats * sizeof(float) > a.pf_bytes) {
+      if ((uint64_t)(logical + 1) * PiecePartial<D, KS>::kFloats * sizeof(float) > a.pf_bytes) {
         if (threadIdx.x == 0) atomicOr(a.err_flag, ASTR_FLAG_BAD_INDEX);  // offsets past the bound
         return;
       }
-      part = a.pf_ws + logical * PiecePartial<D>::kFloats;
+      part = a.pf_ws + logical * PiecePartial<D, KS>::kFloats;
       span.b_lo += piece * a.pf_steps * kWaves;
       // (the last piece takes whatever a context past the host's bound adds)
       if (piece < a.pf_pieces - 1) span.b_hi = min(span.b_hi, span.b_lo + a.pf_steps * kWaves);
@@ -1059,11 +1131,11 @@ __global__ __launch_bounds__(256, (prefill_occupancy<QT, D>())) void prefill_mfm
       for (int k = 0; k < D / 32; ++k)
 #pragma unroll
         for (int x = 0; x < 4; ++x)
-          *PiecePartial<D>::acc(part, wave_id, k, x, lane) =
+          *PiecePartial<D, KS>::acc(part, wave_id, k, x, lane) =
               float4_t{acc[k][4 * x] * up, acc[k][4 * x + 1] * up, acc[k][4 * x + 2] * up,
                        acc[k][4 * x + 3] * up};
       if (lane < 32) {
-        float* ml = part + PiecePartial<D>::kAcc + (wave_id * 32 + lane) * 2;
+        float* ml = part + PiecePartial<D, KS>::kAcc + (wave_id * 32 + lane) * 2;
         ml[0] = m;
         ml[1] = l;
       }
@@ -1071,7 +1143,7 @@ __global__ __launch_bounds__(256, (prefill_occupancy<QT, D>())) void prefill_mfm
       store_column<QT, D>(a, acc, up / fmaxf(l, FLT_MIN), q0 + c.tok, c.head, lane);
     }
   };
-  prefill_unit<QT, D>(a, L, kvh, span.b_lo, span.b_hi,
+  prefill_unit<QT, D, KS>(a, L, kvh, span.b_lo, span.b_hi,
                       a.block_tables + (int64_t)seq * a.bt_stride, q0, t0, column_of,
                       bounds_of, store, []() { return true; }, [](int) {});
 }
@@ -1080,7 +1152,7 @@ constexpr int kMostPieces = 16;
 
 // Merges the pieces of split units with the merge_softmax rule (online_attention.py:42-63). A
 // lane takes one of the four parts of its column as it held it in the pieces: a workgroup one
-// part of a unit's 128 columns. Bound by the chain of its loads: the statistics
+// part of a unit's 128 columns, or two of 64 (KS = 2). Bound by the chain of its loads: the statistics
 // and the first pieces' rows, whose place the unit's index alone gives, are on their way while
 // the dispatch plan is worked out (a place past the unit's own pieces is read, inside the
 // workspace, and not used). 512 tokens on 16000 (32/8 heads of 128: 34 MB of
@@ -1094,21 +1166,25 @@ struct MergeShape {
   static constexpr int kAtOnce = 512 / D;  // pieces whose rows are in flight together
 };
 
-template <typename QT, int D, int G>
+template <typename QT, int D, int G, int KS>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(ChunkArgs a) {
-  using Partial = PiecePartial<D>;
+  using Shape = PrefillShape<D, KS>;
+  using Partial = PiecePartial<D, KS>;
   using M = MergeShape<D>;
-  constexpr int TQ = PrefillShape<D>::kCols / G;
+  constexpr int TQ = Shape::kCols / G;
+  constexpr int kGrid = M::kParts / KS;  // workgroups per unit
   __shared__ int tab[PlanTab::kInts];
   __shared__ int s_wsum[kWaves], s_found[2];
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int part = blockIdx.x % M::kParts, unit = blockIdx.x / M::kParts;
+  const int group = wave % Shape::kGroups;
+  const int part = (int)(blockIdx.x % kGrid) * KS + wave / Shape::kGroups;
+  const int unit = blockIdx.x / kGrid;
   const int64_t first = (int64_t)unit * a.pf_pieces;
   if ((uint64_t)(first + a.pf_pieces) * Partial::kFloats * sizeof(float) > a.pf_bytes) return;
   float* const base = a.pf_ws + first * Partial::kFloats;
 
-  const int col = Partial::kAcc + (wave * 32 + (lane & 31)) * 2;
+  const int col = Partial::kAcc + (group * 32 + (lane & 31)) * 2;
   float2_t ml[kMostPieces];
 #pragma unroll
   for (int j = 0; j < kMostPieces; ++j)
@@ -1121,7 +1197,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(ChunkArgs a) {
       if (j0 + j < pieces)
 #pragma unroll
         for (int n = 0; n < M::kRows; ++n)
-          v[j][n] = *Partial::acc(base + (j0 + j) * (int64_t)Partial::kFloats, wave, n, part, lane);
+          v[j][n] = *Partial::acc(base + (j0 + j) * (int64_t)Partial::kFloats, group, n, part, lane);
   };
   load_rows(0, a.pf_pieces);
 
@@ -1157,7 +1233,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(ChunkArgs a) {
           for (int y = 0; y < 4; ++y) acc[n][y] = fmaf(v[j][n][y], w, acc[n][y]);
       }
   }
-  const int f = wave * 32 + (lane & 31);
+  const int f = group * 32 + (lane & 31);
   const int token = span.t0 + f / G;
   if (token >= span.t1) return;
   const float inv = 1.f / fmaxf(l, FLT_MIN);
@@ -1309,7 +1385,7 @@ __global__ __launch_bounds__(256, (prefill_occupancy<QT, D>())) void prefix_tile
   auto mark = [&](int k) __attribute__((always_inline)) {
     if constexpr (kTrace) tm[k] = wall_clock64();
   };
-  prefill_unit<QT, D>(a, L, kvh, blk0, blk0 + nblk, ids, 0, 0, column_of, bounds_of, store,
+  prefill_unit<QT, D, 1>(a, L, kvh, blk0, blk0 + nblk, ids, 0, 0, column_of, bounds_of, store,
                          prologue, mark);
   const int tid = wave * kWave + lane_id();
   if (lds.bad) {  // a member failed its checks: nothing was stored
@@ -1345,45 +1421,83 @@ int prefill_cus() {
 }
 
 // Key steps below which a unit is not split: a piece costs its start (~2 steps) and its
-// partial, written and read again.
-constexpr int kLeastPieceSteps = 8;
-template <typename QT, int D, int G>
-int launch(ChunkArgs a, hipStream_t stream) {
-  constexpr int TQ = PrefillShape<D>::kCols / G;
-  // Sum over sequences of ceil(n / TQ) for n >= pf_min_rows: each adds at most TQ - 1 to
-  // the token count, and there are at most tokens / pf_min_rows of them.
+// partial, written and read again; at head dim 256, where a step takes twice as long, less.
+template <int D>
+constexpr int least_piece_steps() { return D == 256 ? 4 : 8; }
+
+// Head dim 256, in thirds of a key step of KS = 2 (1.8 us): a step by KS, and what a split
+// costs beside its steps (starts, partials and the merge launch, 10 us).
+constexpr int kSplitTime = 17;
+template <int KS>
+constexpr int step_time() { return KS == 2 ? 3 : 4; }
+
+// Units of a call: the sum over sequences of ceil(n / tq) for n >= pf_min_rows, at most (each
+// adds at most tq - 1 to the token count, and there are at most tokens / pf_min_rows of them).
+int64_t unit_bound(const ChunkArgs& a, int tq) {
   const int64_t seqs = std::min<int64_t>(a.num_seqs, a.num_q_tokens / a.pf_min_rows);
-  const int64_t max_units =
-      ((int64_t)a.num_q_tokens + seqs * (TQ - 1)) / TQ * a.cache.num_kv_heads;
-  if (max_units == 0) return 0;
-  // Units that leave half the resident workgroups or more without work are cut into equal
-  // key ranges, as many as there are idle workgroups per unit and the workspace holds (512
-  // tokens on 16000: 128 units of 258 steps on 512 workgroups, 477 -> 186 us in 4 pieces).
-  const int cus = prefill_cus();
-  a.pf_cus = cus >= kXcds ? cus / kXcds : 1;
+  return ((int64_t)a.num_q_tokens + seqs * (tq - 1)) / tq * a.cache.num_kv_heads;
+}
+
+// The call's units and their key split. Units that leave half the resident workgroups or more
+// without work are cut into equal key ranges, as many as there are idle workgroups per unit
+// and the workspace holds (512 tokens on 16000: 128 units of 258 steps on 512 workgroups,
+// 477 -> 186 us in 4 pieces).
+struct Split {
+  int64_t units;
+  int32_t pieces, steps;  // as pf_pieces, pf_steps
+  int64_t time;           // of the longest unit (step_time, kSplitTime)
+};
+template <typename QT, int D, int G, int KS>
+Split key_split(const ChunkArgs& a, int cus) {
+  constexpr int TQ = PrefillShape<D, KS>::kCols / G;
   int64_t keys = a.max_context;
   if (a.window > 0) keys = std::min<int64_t>(keys, (int64_t)a.window + TQ + kBlockTokens);
   const int64_t steps = (keys + kWaves * kBlockTokens - 1) / (kWaves * kBlockTokens) + 1;
-  const int64_t room = (int64_t)(a.pf_bytes / (PiecePartial<D>::kFloats * sizeof(float)));
+  const int64_t room = (int64_t)(a.pf_bytes / (PiecePartial<D, KS>::kFloats * sizeof(float)));
   const int64_t resident = (int64_t)cus * prefill_occupancy<QT, D>();
-  int64_t pieces = std::min<int64_t>(std::min(resident, room) / max_units, kMostPieces);
-  a.pf_pieces = 1;
-  a.pf_steps = INT32_MAX / kWaves;
-  if (pieces >= 2 && steps >= 2 * kLeastPieceSteps) {
-    a.pf_steps = (int32_t)std::max<int64_t>((steps + pieces - 1) / pieces, kLeastPieceSteps);
-    a.pf_pieces = (int32_t)((steps + a.pf_steps - 1) / a.pf_steps);
-  }
-  const int64_t total = max_units * a.pf_pieces;
-  const int64_t grid = (total + kXcds - 1) / kXcds * kXcds;
+  Split s{unit_bound(a, TQ), 1, INT32_MAX / kWaves, steps * step_time<KS>()};
+  if (s.units == 0) return s;
+  const int64_t pieces = std::min<int64_t>(std::min(resident, room) / s.units, kMostPieces);
+  if (pieces < 2 || steps < 2 * least_piece_steps<D>()) return s;
+  const int64_t longest = std::max<int64_t>((steps + pieces - 1) / pieces, least_piece_steps<D>());
+  const int64_t time = longest * step_time<KS>() + kSplitTime;
+  if (D == 256 && time >= s.time) return s;
+  return Split{s.units, (int32_t)((steps + longest - 1) / longest), (int32_t)longest, time};
+}
+
+template <typename QT, int D, int G, int KS>
+int launch_shape(ChunkArgs a, const Split& split, int cus, hipStream_t stream) {
+  a.pf_cus = cus >= kXcds ? cus / kXcds : 1;
+  a.pf_pieces = split.pieces;
+  a.pf_steps = split.steps;
+  const int64_t grid = (split.units * a.pf_pieces + kXcds - 1) / kXcds * kXcds;
   if (grid > INT32_MAX) return fail(ASTR_EUNSUPPORTED, "prefill grid too large");
-  hipLaunchKernelGGL((prefill_mfma_kernel<QT, D, G>), dim3((uint32_t)grid), dim3(kWaves * kWave),
-                     0, stream, a);
+  hipLaunchKernelGGL((prefill_mfma_kernel<QT, D, G, KS>), dim3((uint32_t)grid),
+                     dim3(kWaves * kWave), 0, stream, a);
   if (a.pf_pieces > 1)
-    hipLaunchKernelGGL((prefill_merge_kernel<QT, D, G>),
-                       dim3((uint32_t)max_units * MergeShape<D>::kParts), dim3(kWaves * kWave), 0,
-                       stream, a);
+    hipLaunchKernelGGL((prefill_merge_kernel<QT, D, G, KS>),
+                       dim3((uint32_t)split.units * (MergeShape<D>::kParts / KS)),
+                       dim3(kWaves * kWave), 0, stream, a);
   const hipError_t err = hipGetLastError();
   return err == hipSuccess ? 0 : hip_fail(err, "paged_attention (prefill) launch");
+}
+
+// At head dim 256, where one workgroup holds a CU, KS = 2 takes what fits the GPU and is done
+// sooner: 500 tokens (16 query / 2 KV heads, bf16) 37.7 us with KS = 1, 31.6 with KS = 2, split
+// 34.4; 16 tokens on 900, 3 sequences (32/8 heads) 54.0, 47.4 and, split, 36.0; 256 on 8000 (16/4
+// heads) stay with KS = 1 and 8 pieces, 75.8 us. Past the GPU's CUs its units queue: 1500 tokens
+// (16/4 heads) 86.5 us with KS = 1, 96.8 with KS = 2.
+template <typename QT, int D, int G>
+int launch(const ChunkArgs& a, hipStream_t stream) {
+  const int cus = prefill_cus();
+  const Split whole = key_split<QT, D, G, 1>(a, cus);
+  if (whole.units == 0) return 0;
+  if constexpr (D == 256) {
+    const Split halves = key_split<QT, D, G, 2>(a, cus);
+    if (halves.units <= cus && halves.time < whole.time)
+      return launch_shape<QT, D, G, 2>(a, halves, cus, stream);
+  }
+  return launch_shape<QT, D, G, 1>(a, whole, cus, stream);
 }
 
 template <typename QT, int D>

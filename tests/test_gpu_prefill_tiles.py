@@ -251,6 +251,23 @@ def test_small_bf16_columns(device, power, fmt):
     _check(cache, tables, [n], [9], query, atol=0)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("fmt", ["int8", "fp8_e4m3fn"])
+@pytest.mark.parametrize("counts,priors", [([16], [700]), ([33, 2], [250, 40]), ([250], [0]),
+                                           ([300, 64], [129, 1000])])
+@pytest.mark.parametrize("group", [1, 4, 8])
+def test_key_halves_at_head_dim_256(device, group, counts, priors, fmt, dtype):
+    """Few units at head dim 256: the waves share 64 columns and take half of every key step
+    each, in units that end in either half, whole and cut into key ranges, and with padding."""
+    lens = [n + p for n, p in zip(counts, priors)]
+    cache, tables, gen = _cache(device, lens, 256, 1, fmt, group)
+    query = torch.randn((sum(counts), group, 256), generator=gen, device=device).to(dtype)
+    _check(cache, tables, lens, counts, query)
+    _check(cache, tables, lens, counts, query, window=45)
+    mark_padding(cache, tables, lens, 0.3, seed=3)
+    _check(cache, tables, lens, counts, query)
+
+
 @pytest.mark.parametrize("fmt", ["int8", "fp8_e4m3fn"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("part", [0, 256])
