@@ -972,7 +972,7 @@ __device__ __forceinline__ int64_t plan_chunk_slot(const PlanArgs& p, int64_t c,
 }
 // Column capacity of a prefix tile (decode_plan.cpp): the chunked-prefill kernel's
 // columns per workgroup, the most tile_rows * G may be.
-constexpr int prefix_tile_columns(int head_dim) { return head_dim == 256 ? 64 : 128; }
+constexpr int kPrefixTileColumns = 128;
 
 // Kernel entry points, one translation unit per code format KF (the source built
 // with -DASTR_KF=KF), dispatched on query dtype, head dim and GQA group inside.

@@ -615,9 +615,9 @@ int planned_attention(const astr_paged_kv* cache, const void* query, int32_t q_d
     return fail(ASTR_EINVAL, "num_q_heads %d must be a multiple of num_kv_heads %d", num_q_heads,
                 cache->num_kv_heads);
   if (pi.num_tiles > 0 &&
-      (int64_t)pi.tile_rows * (num_q_heads / cache->num_kv_heads) > prefix_tile_columns(cache->head_dim))
+      (int64_t)pi.tile_rows * (num_q_heads / cache->num_kv_heads) > kPrefixTileColumns)
     return fail(ASTR_EINVAL, "prefix tiles of %d rows exceed the %d query columns of a tile",
-                pi.tile_rows, prefix_tile_columns(cache->head_dim));
+                pi.tile_rows, kPrefixTileColumns);
   if (cache->num_blocks < 1) return fail(ASTR_EINVAL, "cache has no blocks");
   if (q_dtype != ASTR_F16 && q_dtype != ASTR_BF16 &&
       !(q_dtype == ASTR_F32 && cache->code_format == ASTR_KV_INT8))

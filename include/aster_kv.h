@@ -379,10 +379,10 @@ int64_t astr_decode_plan_words_bound(int32_t num_seqs, int32_t num_kv_heads,
  * Shared prefixes (the pages PrefixCache hands to several sequences, state.py:547-640,
  * forked at state.py:210-216): with tile_rows >= 2, sequences whose tables begin with
  * the same min_shared_blocks blocks or more, all of them visible, are read in prefix
- * tiles of up to tile_rows sequences (tile_rows * G <= the prefix-tile kernel's
- * columns: 128 at head dims up to 128, 64 at 256), each kv head's shared blocks cut
- * into tile_ranges key ranges (0: chosen from the workgroup count); the rows' own
- * blocks remain items. tile_rows = 0 plans no tiles.
+ * tiles of up to tile_rows sequences (tile_rows * G <= the prefix-tile kernel's 128
+ * columns), each kv head's shared blocks cut into tile_ranges key ranges (0: chosen
+ * from the workgroup count); the rows' own blocks remain items. tile_rows = 0 plans
+ * no tiles.
  */
 int astr_decode_plan(const int32_t* block_tables, int32_t block_table_stride,
                      const int32_t* context_lens, int32_t num_seqs, int32_t num_kv_heads,

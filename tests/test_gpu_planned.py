@@ -147,6 +147,19 @@ def test_shared_prefixes_in_tiles(device, dim, hq, hkv, qdtype, ranges):
     assert_attention_close(out, oracle_decode(w, cache, q))
 
 
+@pytest.mark.parametrize("dim", [64, 128, 256])
+@pytest.mark.parametrize("hq,hkv", [(8, 8), (16, 4), (16, 2)])
+def test_full_prefix_tiles(device, dim, hq, hkv):
+    """Tiles of 128 / G rows, every query column in use at each head dim, and one row more."""
+    w = _shared_workload(dim, hq, hkv, torch.bfloat16, seed=7, groups=(128 * hkv // hq + 1,),
+                         shared=(17,), own_max=40)
+    cache, tables, lens = _build(w, device)
+    q = wl.queries(w, device)
+    out, plan = _planned(cache, w, q, tables, lens)
+    assert plan.info.tile_rows == 128 * hkv // hq
+    assert_attention_close(out, oracle_decode(w, cache, q))
+
+
 @pytest.mark.parametrize("fmt", ["int8", "fp8_e4m3fn", "fp8_e5m2"])
 def test_shared_prefix_tiles_formats_and_padding(device, fmt):
     w = _shared_workload(128, 32, 8, torch.bfloat16, seed=3)
