@@ -474,11 +474,11 @@ __device__ __forceinline__ void convert_raw(const AttnArgs& a, const RawBlock<D>
     }
     vd[2 * (i % Lds::kRowsN * kWave + i / Lds::kRowsN)] = __builtin_bit_cast(uint2, v * vsh);
   }
-  // key factors: above zero, so that a masked score's -inf stays -inf; a NaN scale counts as
-  // infinite, which the steps' edge path reports where a key of it is seen
-  float ksf = fmaxf(b.ks * (a.qk_scale_log2 * code_scale<KF>()), __FLT_DENORM_MIN__);
+  // key factors: a NaN scale counts as infinite, which the steps' edge path reports where a
+  // key of it is seen
+  float ksf = b.ks * (a.qk_scale_log2 * code_scale<KF>());
   ksf = b.ks == b.ks ? ksf : INFINITY;
-  const bool large = __ballot(!(ksf <= safe_factor())) != 0;
+  const bool large = __ballot(!(fabsf(ksf) <= safe_factor())) != 0;
   if (lane < 16) L.ks[buf][16 * w + lane] = ksf;
   if (masks && lane < 4) L.pad[buf][4 * w + lane] = kPad ? b.pad : load_pad<D>(a, b.id, lane);
   if (lane == 0) L.flags[buf][w] = e | (large ? kLargeFlag : 0);
