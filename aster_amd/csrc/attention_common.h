@@ -447,58 +447,39 @@ __device__ __forceinline__ void load_query_column(const QT* qp, QueryColumn<QT, 
       raw.w[h][c] = reinterpret_cast<const uint4*>(qp + 64 * h)[c];
 }
 
-// Int8 B-operands of one query column for the QK MFMAs (lane r of its 16-lane group
-// qg holds d = 16*qg + 64*h + [0, 16)): the column is quantized once to integers
-// Q = 128 * hi + lo within 1/2 of q * kQRange / max|q|, hi and lo in int8, so that
-// K.Q = 128 (K.hi) + K.lo is exact in int32 (a ~15-bit query, finer than f16's 11 bits
-// for every element within 2^-4 of the column maximum).
-// Returns the score factor max|q| / kQRange * qk_scale_log2 (NaN for a non-finite
-// query, which makes every score of the column non-finite as in fp32 arithmetic).
-// kTerms > 2: more terms for blocks whose scores are large enough that the 15-bit
-// query's error would show. With x = q * kQRange / max|q| and r2 = x - Q (|r2| <= 1/2):
-// lo2 = rint(128 r2), so that 128 Q + lo2 is within 1/2 of 128 x (a ~22-bit query);
-// kTerms = 4 adds lo3 = rint(128 (128 r2 - lo2)), 2^14 Q + 2^7 lo2 + lo3 within 1/2 +
-// 2^-11 of 2^14 x (~29 bits). Every term is in [-64, 64]; the same raw column always
-// gives the same terms.
-// Cross-lane: uniform control flow.
 // The int8 terms of one query element xv (already lifted) at the column's inv, as floats
 // whose low bytes are the terms' two's-complement bytes: adding kQRound (1.5 * 2^23, unit
 // in the last place 1) to a value below 2^22 in magnitude rounds it to an integer held in
-// the low mantissa bits. Each fma rounds once; hi = rint(xv * inv / 128) and
-// lo = rint(xv * inv - 128 hi) (ties to even, |hi| <= 127, |lo| <= 64); with kTerms > 2,
-// lo2 = rint(128 r2) where r2 = xv * inv - (128 hi + lo) (|r2| <= 1/2), and with
-// kTerms > 3, lo3 = rint(128 (128 r2 - lo2)).
+// the low mantissa bits. Each fma rounds once; hi = rint(xv * inv / 128),
+// lo = rint(xv * inv - 128 hi) (ties to even, |hi| <= 127, |lo| <= 64) and
+// lo2 = rint(128 r2) where r2 = xv * inv - (128 hi + lo) (|r2| <= 1/2).
 constexpr float kQRound = 12582912.f;
 struct QueryTerms {
-  float hi, lo, lo2, lo3;
+  float hi, lo, lo2;
 };
-template <int kTerms>
 __device__ __forceinline__ QueryTerms query_terms(float xv, float inv) {
   QueryTerms t;
   t.hi = __builtin_fmaf(xv, inv * (1.f / 128.f), kQRound);  // inv / 128: exact
   const float hv = t.hi - kQRound;
   t.lo = __builtin_fmaf(xv, inv, __builtin_fmaf(hv, -128.f, kQRound));
-  if constexpr (kTerms > 2) {
-    // residual of Q = 128 hi + lo (exact integers), one rounding: |r2| <= 1/2
-    const float q2 = __builtin_fmaf(hv, 128.f, t.lo - kQRound);
-    const float r2 = __builtin_fmaf(xv, inv, -q2);
-    t.lo2 = __builtin_fmaf(r2, 128.f, kQRound);
-    if constexpr (kTerms > 3) {
-      const float r3 = __builtin_fmaf(r2, 128.f, kQRound - t.lo2);  // exact
-      t.lo3 = __builtin_fmaf(r3, 128.f, kQRound);
-    }
-  }
+  // residual of Q = 128 hi + lo (exact integers), one rounding: |r2| <= 1/2
+  const float q2 = __builtin_fmaf(hv, 128.f, t.lo - kQRound);
+  t.lo2 = __builtin_fmaf(__builtin_fmaf(xv, inv, -q2), 128.f, kQRound);
   return t;
 }
 
-template <typename QT, int D, int kTerms = 2>
+// Int8 B-operands of one query column for the QK MFMAs (lane r of its 16-lane group
+// qg holds d = 16*qg + 64*h + [0, 16)): with x = q * kQRange / max|q|, the column is
+// quantized to integers 128 Q + lo2 within 1/2 of 128 x (a ~22-bit query), Q = 128 hi + lo
+// within 1/2 of x, every term an int8, so that 128 (K.hi) + K.lo and K.lo2 are exact in
+// int32.
+// Returns the score factor max|q| / kQRange * qk_scale_log2 (NaN for a non-finite
+// query, which makes every score of the column non-finite as in fp32 arithmetic).
+// Cross-lane: uniform control flow.
+template <typename QT, int D>
 __device__ __forceinline__ float query_column_i8(const QueryColumn<QT, D>& raw, bool valid,
                                                  float qk_scale_log2, int4_t (&qhi)[D / 64],
-                                                 int4_t (&qlo)[D / 64],
-                                                 int4_t* qlo2 = nullptr, int4_t* qlo3 = nullptr,
-                                                 float* inv_out = nullptr,
-                                                 float* lift_out = nullptr) {
-  static_assert(kTerms >= 2 && kTerms <= 4, "query terms");
+                                                 int4_t (&qlo)[D / 64], int4_t (&qlo2)[D / 64]) {
   constexpr int kVec = 16 / (int)sizeof(QT);  // elements per 16-byte load
   float x[D / 64][16];
 #pragma unroll
@@ -534,25 +515,21 @@ __device__ __forceinline__ float query_column_i8(const QueryColumn<QT, D>& raw, 
     mx *= up;
   }
   const float inv = (finite && mx > 0.f) ? (float)kQRange / mx : 0.f;
-  if (inv_out != nullptr) *inv_out = inv;
-  if (lift_out != nullptr) *lift_out = up;
 #pragma unroll
   for (int h = 0; h < D / 64; ++h)
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
-      uint32_t hb[4], lb[4], fb[4], gb[4];
+      uint32_t hb[4], lb[4], fb[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const QueryTerms t = query_terms<kTerms>(x[h][4 * w + e], inv);
+        const QueryTerms t = query_terms(x[h][4 * w + e], inv);
         hb[e] = __builtin_bit_cast(uint32_t, t.hi);
         lb[e] = __builtin_bit_cast(uint32_t, t.lo);
-        if constexpr (kTerms > 2) fb[e] = __builtin_bit_cast(uint32_t, t.lo2);
-        if constexpr (kTerms > 3) gb[e] = __builtin_bit_cast(uint32_t, t.lo3);
+        fb[e] = __builtin_bit_cast(uint32_t, t.lo2);
       }
       qhi[h][w] = (int)low_bytes(hb);
       qlo[h][w] = (int)low_bytes(lb);
-      if constexpr (kTerms > 2) qlo2[h][w] = (int)low_bytes(fb);
-      if constexpr (kTerms > 3) qlo3[h][w] = (int)low_bytes(gb);
+      qlo2[h][w] = (int)low_bytes(fb);
     }
   return factor;
 }
@@ -651,12 +628,12 @@ template <int D, int KF>
 struct QkOperand {
   half8_t op[D / 32];
 };
-// INT8 codes: the query column as 128 Q + lo2 within 1/2 of 128 x (query_column_i8 with
-// three terms, x = q * kQRange / max|q|), i.e. within 2^-8 of a ~15-bit step of q, about
+// INT8 codes: the query column as 128 Q + lo2 within 1/2 of 128 x (query_column_i8,
+// x = q * kQRange / max|q|), i.e. within 2^-8 of a ~15-bit step of q, about
 // 2^-22 of max|q| per element: the score K.q carries, per unit of K, the error an fp32
 // dot product's own rounding has. Every block takes all three terms (the third on a
-// separate int32 accumulator: 128 (K.Q) + K.lo2 can exceed int32), so no key scale,
-// however large, sees the coarser two-term query.
+// separate int32 accumulator: 128 (K.Q) + K.lo2 can exceed int32), however small its key
+// scales.
 template <int D>
 struct QkOperand<D, kInt8> {
   int4_t hi[D / 64], lo[D / 64], lo2[D / 64];
@@ -675,7 +652,7 @@ __device__ __forceinline__ float qk_operand(const QueryRaw<D>& q, bool gvalid, f
       col.w[h][0] = q.w[h][0];
       col.w[h][1] = q.w[h][1];
     }
-    return query_column_i8<QT, D, 3>(col, gvalid, qk_scale_log2, op.hi, op.lo, op.lo2);
+    return query_column_i8<QT, D>(col, gvalid, qk_scale_log2, op.hi, op.lo, op.lo2);
   } else {
     return query_operand<QT, D>(q, gvalid, qk_scale_log2, op.op) * code_scale<KF>();
   }
@@ -688,7 +665,7 @@ template <typename QT, int D, int KF>
 __device__ __forceinline__ float qk_operand_column(const QueryColumn<QT, D>& col, bool gvalid,
                                                    float qk_scale_log2, QkOperand<D, KF>& op) {
   if constexpr (KF == kInt8) {
-    return query_column_i8<QT, D, 3>(col, gvalid, qk_scale_log2, op.hi, op.lo, op.lo2);
+    return query_column_i8<QT, D>(col, gvalid, qk_scale_log2, op.hi, op.lo, op.lo2);
   } else {
     static_assert(sizeof(QT) == 2, "FP8 codes take 16-bit queries on the MFMA path");
     return query_operand<QT, D>(reinterpret_cast<const QueryRaw<D>&>(col), gvalid,
