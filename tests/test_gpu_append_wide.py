@@ -9,6 +9,7 @@ import torch
 
 from aster_amd import KVQuantization, PagedKVCache
 from oracle import reference_cpu as ref
+from tests.division_pairs import dangerous_pairs
 from tests.gpu_util import arena_numpy
 
 pytestmark = pytest.mark.gpu
@@ -91,3 +92,59 @@ def test_wide_append_keeps_non_finite_rows_out(device, dim, bad):
                 else:
                     assert ks[t // 16, h, t % 16] == 1
         assert kc[2 // 16, 0, 2].any() and vc.any()  # in the flagging row's own workgroup
+
+
+def _append_rows(device, rows, fmt):
+    """Codes and scales of ``[T, D]`` rows through the append, as [T, D] bytes and [T]."""
+    tokens, dim = rows.shape
+    cache = PagedKVCache(num_blocks=-(-tokens // 16), num_layers=1, num_kv_heads=1, head_dim=dim,
+                         device=device, quantization=KVQuantization(fmt))
+    key = rows.to(device)[:, None]
+    cache.append(0, key, key, torch.arange(tokens, device=device), check=True)
+    kc, ks, vc, vs = arena_numpy(cache)
+    np.testing.assert_array_equal(kc, vc)
+    return kc.reshape(-1, dim)[:tokens].view(np.int8), ks.reshape(-1)[:tokens]
+
+
+@pytest.mark.parametrize("fmt,offsets", [("int8", range(-1, 9)), ("fp8_e4m3fn", (-1, 0, 14, 15, 16, 17, 18)),
+                                         ("fp8_e5m2", (-1, 0))])
+def test_every_f16_quotient(device, fmt, offsets):
+    """Row maxima of every f16 significand over elements of every f16 significand and the
+    exponents at which their codes differ: up to powers of two all quotients of 16-bit input."""
+    sig = torch.arange(1024, dtype=torch.int16)
+    for top in range(0, 1024, 128):
+        amax = (sig[top:top + 128] | (29 << 10)).view(torch.float16)
+        x = torch.cat([(sig | ((28 - e) << 10)).view(torch.float16) for e in offsets])
+        x = torch.cat([x, x.new_zeros(-len(x) % 511)]).reshape(-1, 511)
+        x = torch.minimum(x.expand(len(amax), -1, -1), amax[:, None, None])
+        rows = torch.cat([amax[:, None, None].expand(-1, x.shape[1], 1), x], 2).reshape(-1, 512)
+        rows[:, 2::2] *= -1
+        codes, scales = _append_rows(device, rows, fmt)
+        want_codes, want_scales = _oracle(rows.float().numpy()[:, None], fmt)
+        np.testing.assert_array_equal(scales, want_scales[:, 0])
+        np.testing.assert_array_equal(codes, want_codes[:, 0])
+
+
+@pytest.mark.parametrize("fmt,odd", [("int8", range(1, 255, 2)), ("fp8_e4m3fn", range(17, 32, 2)),
+                                     ("fp8_e5m2", range(9, 16, 2))])
+def test_float32_quotients_beside_ties(device, fmt, odd):
+    """float32 rows whose quotients lie where the corrected product could round to the other
+    side of a tie (division_pairs)."""
+    most = np.float32({"int8": 127.0, "fp8_e4m3fn": 448.0, "fp8_e5m2": 57344.0}[fmt])
+    rows = []
+    for t, x, b in dangerous_pairs(odd):
+        x, b = np.float32(x), np.float32(b)
+        amax = np.float32(most * b)
+        if amax / most != b:
+            continue  # no row has this scale
+        tie = t / 2 if fmt == "int8" else t
+        x = np.ldexp(x, int(np.round(np.log2(tie * b / x))))
+        row = np.zeros(64, np.float32)
+        row[:3] = amax, x, -x
+        rows.append(row)
+    assert len(rows) > 20
+    rows = np.stack(rows)
+    codes, scales = _append_rows(device, torch.from_numpy(rows), fmt)
+    want_codes, want_scales = _oracle(rows[:, None], fmt)
+    np.testing.assert_array_equal(scales, want_scales[:, 0])
+    np.testing.assert_array_equal(codes, want_codes[:, 0])
