@@ -81,15 +81,20 @@ def hipcc():
 # registers ran at 313 and one wave per SIMD after a change that went unnoticed).
 # The exact fp32 VALU decode kernels (fp32 queries) are known to spill this way. The
 # prefill kernels at head dim 256 run one wave per SIMD by design (their operand buffers
-# fill the LDS), so the second half of the register file is theirs.
-AGPR_SPILL_ALLOWED = ("decode_valu_kernel", "prefill_mfma_kernelIfLi256", "prefill_mfma_kernelIDF16_Li256",
-                      "prefill_mfma_kernelINS_6bf16_tELi256", "prefix_tiles_kernelIfLi256",
-                      "prefix_tiles_kernelIDF16_Li256", "prefix_tiles_kernelINS_6bf16_tELi256")
+# fill the LDS), so the second half of the register file is theirs. What each may hold there
+# is bounded a little above what it does, so that growth is noticed.
+AGPR_LIMITS = ((r"decode_valu_kernelI", 240),
+               (r"(prefill_mfma|prefix_tiles)_kernelIfLi256E", 136),
+               (r"(prefill_mfma|prefix_tiles)_kernelI(DF16_|NS_6bf16_tE)Li256E", 184))
+
+
+def _agpr_limit(name):
+    return max((most for pattern, most in AGPR_LIMITS if re.search(pattern, name)), default=0)
 
 
 def _scratch_kernels(remarks):
     """Kernels whose resource-usage remark reports a non-zero scratch size, or AGPRs
-    (spilled VGPRs) outside AGPR_SPILL_ALLOWED."""
+    (spilled VGPRs) past AGPR_LIMITS."""
     bad, name = [], None
     for line in remarks.splitlines():
         m = re.search(r"Function Name: (\S+)", line)
@@ -100,7 +105,7 @@ def _scratch_kernels(remarks):
         if m and int(m.group(1)) > 0:
             bad.append(f"{name} ({m.group(1)} bytes/lane of scratch)")
         m = re.search(r"AGPRs: (\d+)", line)
-        if m and int(m.group(1)) > 0 and not any(k in (name or "") for k in AGPR_SPILL_ALLOWED):
+        if m and int(m.group(1)) > _agpr_limit(name or ""):
             bad.append(f"{name} ({m.group(1)} AGPRs: VGPRs spilled)")
     return bad
 

@@ -1,7 +1,7 @@
 """The build rejects kernels that spill registers: per-lane scratch (stack) memory, or
-AGPRs used as spill space (every MFMA accumulator is meant to live in VGPRs), outside
-the exact fp32 VALU decode kernels known to spill that way: parsing of the compiler's
-kernel-resource-usage remarks."""
+AGPRs used as spill space (every MFMA accumulator is meant to live in VGPRs) past what the
+kernels known to spill that way may hold: parsing of the compiler's kernel-resource-usage
+remarks."""
 
 from aster_amd import build
 
@@ -30,6 +30,16 @@ def test_register_spills_are_reported():
     assert build._scratch_kernels(remarks) == ["kern_b (544 bytes/lane of scratch)",
                                                "kern_c (41 AGPRs: VGPRs spilled)"]
     assert build._scratch_kernels("") == []
+
+
+def test_spills_of_the_one_wave_kernels_are_bounded():
+    name = "_ZN4astr4attn12_GLOBAL__N_1{}ILi256ELi4ELi1EEEvNS0_9ChunkArgsE"
+    half, single = "19prefill_mfma_kernelINS_6bf16_tELi256ELi4E", "19prefix_tiles_kernelIfLi256ELi4E"
+    for kernel, agprs, bad in ((half, 168, False), (half, 200, True), (single, 129, False),
+                               (single, 160, True), (half.replace("256", "128"), 1, True)):
+        remarks = "\n".join([_remark(1, "Function Name: " + name.replace("{}I", kernel + "I")),
+                             _remark(1, f"    AGPRs: {agprs}")])
+        assert bool(build._scratch_kernels(remarks)) == bad, (kernel, agprs)
 
 
 def test_build_flags_request_resource_remarks():
