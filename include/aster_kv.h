@@ -249,14 +249,18 @@ int astr_paged_attention_i8_noalloc(const astr_paged_kv* cache, const void* quer
  *              n query tokens sits at position ctx-n+i and sees key k iff
  *              k <= position (causal != 0; else k < ctx) and, when window > 0,
  *              k > position - window. ctx < n raises ASTR_FLAG_BAD_INDEX.
- *   Other arguments as astr_paged_attention_i8 (workspace sized by
- *   astr_paged_attention_i8_workspace_bytes for num_seqs rows; chunk rows need none).
+ *   Other arguments as astr_paged_attention_i8; workspace sized by
+ *   astr_paged_attention_i8_workspace_bytes for num_seqs rows. All of it is scratch,
+ *   also in calls of chunk rows alone: long histories of few chunk rows are cut into
+ *   key ranges, as many as their partials find room there.
  * Sequences with one query token take the decode kernels (the query sees every
- * key, as for astr_paged_attention_i8), longer ones the MFMA prefill kernel
- * (bf16/fp16/fp32 queries; with int8 codes a query column enters the int8 QK
- * MFMAs as integers within 1/2 of q * 16256 / max|q|, with FP8 codes it is
- * rounded to f16 after an exact power-of-two rescale), launched after the
- * decode kernels on the same stream.
+ * key, as for astr_paged_attention_i8), longer ones the MFMA prefill kernel, launched
+ * after them on the same stream. 16-bit calls of num_seqs * max_query_len tokens, or
+ * with max_context_len <= 512 and a compute unit for every (sequence, KV head), skip
+ * the decode kernels: the prefill kernel takes every row. It multiplies in f16, the
+ * codes exactly; a 16-bit query enters as one f16 term, an fp32 one as two (22 bits),
+ * its (token, head) column scaled by a power of two where the largest element is 2^15
+ * or more or (bf16, fp32) below 2^-3.
  */
 int astr_paged_attention_varlen_i8(const astr_paged_kv* cache, const void* query,
                                    int32_t q_dtype, int64_t q_token_stride,

@@ -190,11 +190,10 @@ def test_key_scale_outliers_past_the_group_tokens(device, part, dim):
 
 
 @pytest.mark.parametrize("dim", [64, 128, 256])
-def test_scores_near_the_chunk_third_term_threshold(device, dim):
-    """Keys x 3 and queries x 3: the chunk rows' steps sit around the key scale at
-    which the prefill kernel adds its third query term (some take it, most not), and
-    both kinds of step are held to the float64 oracle at the plain tolerance plus fp32
-    rounding."""
+def test_scores_nine_times_the_ordinary(device, dim):
+    """Keys x 3 and queries x 3: scores nine times the ordinary ones, where 15 bits of a
+    query element would no longer do, held to the float64 oracle at the plain tolerance
+    plus fp32 rounding (decode rows: three int8 terms; chunk rows: f16 operands)."""
     w = _workload(MIXED_Q, MIXED_CTX, hq=16, hkv=4, dim=dim, seed=dim + 29)
     cache, tables, lens = _build(w, device, "int8")
     cache.scales[:, 0, 0] *= 3.0

@@ -173,8 +173,8 @@ def test_shared_prefix_tiles_formats_and_padding(device, fmt):
 
 
 def test_shared_prefix_tiles_extreme_scores(device):
-    """q x100 and K scales x100: the tiles' scores take the third query term on every
-    step, and every output stays within the fp32 rounding of the exact result."""
+    """q x100 and K scales x100: every output of the tiles stays within the fp32 rounding of
+    the exact result."""
     from tests.test_gpu_hardening import _assert_within_fp32_rounding
 
     w = _shared_workload(128, 32, 8, torch.bfloat16, seed=9)

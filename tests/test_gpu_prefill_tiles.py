@@ -84,8 +84,9 @@ def test_scaled_columns(device, dtype, power):
 
 @pytest.mark.parametrize("fmt", ["int8", "fp8_e4m3fn", "fp8_e5m2"])
 def test_large_scales(device, fmt):
-    """V scales up to 2^20 larger in some blocks, alone and beside ordinary ones: the
-    tolerance scales with the largest values (the weights' f16 rounding)."""
+    """V scales up to 2^20 larger in some blocks, beside ordinary ones: no product or sum
+    leaves its range. The tolerance is of the largest values (the weights' f16 rounding), so
+    that only these blocks are checked here; test_exponents_of_padded_blocks has the others'."""
     lens, counts = [300, 90], [70, 33]
     cache, tables, gen = _cache(device, lens, 128, 2, fmt, 11)
     cache.scales[::3, :, 1] *= 2.0 ** 20
@@ -132,7 +133,7 @@ def test_smallest_key_scales(device, dtype):
 
 
 def test_long_history(device):
-    """More than 64 key steps (the block ids are fetched 64 steps at a time)."""
+    """A unit of 130 key steps, its ids read one step ahead of its blocks, in a window too."""
     lens, counts = [64 * 64 * 2 + 77], [9]
     cache, tables, gen = _cache(device, lens, 64, 1, "int8", 5)
     query = torch.randn((9, 2, 64), generator=gen, device=device).half()
@@ -251,6 +252,20 @@ def test_small_bf16_columns(device, power, fmt):
     _check(cache, tables, [n], [9], query, atol=0)
 
 
+@pytest.mark.parametrize("nats", [10, 12, 14])
+def test_mass_in_weights_below_f16s_normal_range(device, nats):
+    """Thousands of keys ``nats`` below the first: each weight is subnormal in f16, and the
+    sum has to count them as the numerator does. Tolerance: half of f16's step of 2^-24 on
+    each weight, and its output."""
+    n, dim = 6000, 128
+    unit = (dim - 1) * 2 * 96 * dim ** -0.5
+    cache, tables = _two_groups(device, dim, "int8", n, 1, (96, -96), (nats / unit, nats / unit),
+                                (0.0, 1.0))
+    query = torch.ones((9, 1, dim), device=device)
+    _check(cache, tables, [n], [9], query.half(), atol=0,
+           rtol=2.0 ** -25 / np.exp(-nats) + 2.0 ** -10)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("fmt", ["int8", "fp8_e4m3fn"])
 @pytest.mark.parametrize("counts,priors", [([16], [700]), ([33, 2], [250, 40]), ([250], [0]),
@@ -266,6 +281,26 @@ def test_key_halves_at_head_dim_256(device, group, counts, priors, fmt, dtype):
     _check(cache, tables, lens, counts, query, window=45)
     mark_padding(cache, tables, lens, 0.3, seed=3)
     _check(cache, tables, lens, counts, query)
+
+
+@pytest.mark.parametrize("fmt", ["int8", "fp8_e4m3fn", "fp8_e5m2"])
+@pytest.mark.parametrize("lens,counts", [([300, 90], [70, 33]), ([3000], [20])])
+def test_exponents_of_padded_blocks(device, lens, counts, fmt):
+    """Blocks whose V scales need exponents of 1 to 5 hold padding keys alone: they change the
+    unit of the accumulators (four of them within one key step, in one piece of a split unit),
+    and the result is the other blocks', of ordinary size and tolerance."""
+    cache, tables, gen = _cache(device, lens, 128, 2, fmt, 17)
+    large = {5: 15, 8: 18, 9: 16, 10: 17, 14: 14}  # block of a sequence: power of its scales
+    for row, n in enumerate(lens):
+        for block, power in large.items():
+            if 16 * (block + 1) > n - counts[row]:
+                continue
+            cache.scales[int(tables[row, block]), :, 1] *= 2.0 ** power
+            slots = int(tables[row, block]) * 16 + torch.arange(16, device=device)
+            cache.write_key_valid(slots, torch.zeros(16, dtype=torch.bool, device=device))
+    query = torch.randn((sum(counts), 8, 128), generator=gen, device=device)
+    for dtype in (torch.float32, torch.bfloat16):
+        _check(cache, tables, lens, counts, query.to(dtype))
 
 
 @pytest.mark.parametrize("fmt", ["int8", "fp8_e4m3fn"])
