@@ -218,6 +218,8 @@ __device__ int scan_tiles(const ChunkArgs& a, int tq, int unit, int* s_wsum, int
 // factor below this keeps every score finite (max code 127; 448 2^-8 for E4M3FN; 57344).
 constexpr float safe_factor() { return KF == kInt8 ? 1.0e29f : KF == kE4M3 ? 1.0e31f : 5.0e26f; }
 
+constexpr uint32_t kScaledBit = 4, kLargeBit = 8;  // beside a half step's block bits
+
 // A scaled column's factor 2^ex in [kBackLeast, 1] keeps its scores (before the key factor)
 // in range on either side; any other takes the edge path.
 constexpr float kBackLeast = 0x1p-64f;
@@ -506,12 +508,13 @@ struct WaveBounds {
 // the layout that P^T enters the second product in. t = s * ks - m is the base-2 score
 // over the running maximum, p = exp2(t). Bit w of `use` (wave-uniform): block w holds keys
 // some column of the wave sees; of `bounded`: the column bounds [lo, hi] cut into block w.
-// `scaled`: a column is scaled; `large`: a key factor is. Keys that are all used, not bounded,
-// not padded and not large take no per-score condition (no score can overflow) unless a column
-// is scaled beyond kBackLeast, only the scaled columns' factors; otherwise scores are masked to
-// -inf outside the bounds, for padding keys and for unused blocks (which repeat the range's
-// last one) and checked for non-finite values. vf: the blocks' exponent factors 2^(e_w - ve)
-// on the weights of the numerator only, where `vmix`.
+// Further bits of `use`: kScaledBit, a column is scaled; kLargeBit, a key factor is large (and
+// kScaledBit). Keys that are all used, not bounded, not padded and not large take no per-score
+// condition (no score can overflow) unless a column is scaled beyond kBackLeast, only the
+// scaled columns' factors; otherwise scores are masked to -inf outside the bounds, for padding
+// keys and for unused blocks (which repeat the range's last one) and checked for non-finite
+// values. vf: the blocks' exponent factors 2^(e_w - ve) on the weights of the numerator only,
+// where `vmix`.
 //
 // The operands come from LDS well ahead of their MFMAs (a read takes over 100 cycles, and a
 // wave that waits for each pair of them spends more time there than on the arithmetic): the
@@ -527,9 +530,8 @@ __device__ __forceinline__ void load_k_operands(const PrefillLds<D>& L, int buf,
 
 template <typename QT, int D, int NT, typename Between>
 __device__ __forceinline__ void prefill_half(const PrefillLds<D>& L, int buf, int kt, uint32_t use,
-                                             uint32_t bounded, bool masks, bool scaled,
-                                             bool large, int kb0, half8_t (&kop)[D / 16],
-                                             Between between,
+                                             uint32_t bounded, bool masks, int kb0,
+                                             half8_t (&kop)[D / 16], Between between,
                                              const QOp<QT, D> (&qop)[NT], const float (&back)[NT],
                                              const int (&lo)[NT], const int (&hi)[NT], int lane,
                                              bool vmix, half2_t vf,
@@ -584,13 +586,15 @@ __device__ __forceinline__ void prefill_half(const PrefillLds<D>& L, int buf, in
   for (int x = 0; x < 4; ++x)
     ks[x] = *reinterpret_cast<const float4_t*>(&L.ks[buf][32 * kt + 8 * x + 4 * h]);
   if constexpr (QOp<QT, D>::kAhead) __builtin_amdgcn_sched_barrier(0);
-  if (use != 3u || bounded != 0 || scaled || large || padded) {
+  if (use != 3u || bounded != 0 || padded) {
     asm volatile("");  // keeps this a branch: if-converted, the interior steps would pay for it
-    bool far = false;
+    bool factors = use == (3u | kScaledBit) && bounded == 0 && !padded;  // those alone?
+    if (factors) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
-      far |= __ballot(!(back[t] <= 1.f && back[t] >= kBackLeast)) != 0;
-    if (use == 3u && bounded == 0 && !far && !large && !padded) {  // scaled columns alone
+      for (int t = 0; t < NT; ++t)
+        factors = factors && __ballot(!(back[t] <= 1.f && back[t] >= kBackLeast)) == 0;
+    }
+    if (factors) {
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -599,10 +603,15 @@ __device__ __forceinline__ void prefill_half(const PrefillLds<D>& L, int buf, in
       // Per-score masks as all-ones/zero words in VGPRs (sign bits of differences, bit
       // selects): lane masks of unrolled compares would stay live in SGPRs and spill.
       uint32_t nonfinite = 0;
+      uint32_t pads[4] = {0x01010101u, 0x01010101u, 0x01010101u, 0x01010101u};
+      if (masks) {
+#pragma unroll
+        for (int x = 0; x < 4; ++x) pads[x] = L.pad[buf][8 * kt + 2 * x + h];
+      }
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
         const int w = x / 2;
-        const uint32_t pad = masks ? L.pad[buf][8 * kt + 2 * x + h] : 0x01010101u;
+        const uint32_t pad = pads[x];
         const bool used = (use >> w) & 1u, bnd = (bounded >> w) & 1u;  // wave-uniform
 #pragma unroll
         for (int y = 0; y < 4; ++y) {
@@ -850,10 +859,11 @@ __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L
     const int4_t fv = *reinterpret_cast<const int4_t*>(L.flags[buf]);
     const int f0 = __builtin_amdgcn_readfirstlane(fv[0]), f1 = __builtin_amdgcn_readfirstlane(fv[1]);
     const int f2 = __builtin_amdgcn_readfirstlane(fv[2]), f3 = __builtin_amdgcn_readfirstlane(fv[3]);
-    bool vmix = false, large = false;
+    bool vmix = false;
+    uint32_t slow = scaled ? kScaledBit : 0u;
     half4_t vf = {(_Float16)1.f, (_Float16)1.f, (_Float16)1.f, (_Float16)1.f};
     if (__builtin_expect((f0 | f1 | f2 | f3 | ve) != 0, 0)) {
-      large = ((f0 | f1 | f2 | f3) & kLargeFlag) != 0;
+      if (((f0 | f1 | f2 | f3) & kLargeFlag) != 0) slow = kScaledBit | kLargeBit;
       const int e4[kWaves] = {f0 & (kLargeFlag - 1), f1 & (kLargeFlag - 1), f2 & (kLargeFlag - 1),
                               f3 & (kLargeFlag - 1)};
       const int emax = max(max(e4[0], e4[1]), max(e4[2], e4[3]));
@@ -889,20 +899,20 @@ __device__ __forceinline__ void prefill_unit(const AttnArgs& a, PrefillLds<D>& L
     if constexpr (KS == 2) {
       const uint32_t mine = use >> (2 * half) & 3u;
       if (mine != 0)
-        prefill_half<QT, D, NT>(L, buf, half, mine, bounded >> (2 * half) & 3u, masks, scaled,
-                                large, kb0 + 32 * half, kop, []() {}, qop, back, lo, hi, lane, vmix,
+        prefill_half<QT, D, NT>(L, buf, half, mine | slow, bounded >> (2 * half) & 3u, masks,
+                                kb0 + 32 * half, kop, []() {}, qop, back, lo, hi, lane, vmix,
                                 half != 0 ? half2_t{vf[2], vf[3]} : half2_t{vf[0], vf[1]}, acc, m,
                                 l, bad_score);
     } else if (use != 0) {
-      prefill_half<QT, D, NT>(L, buf, 0, use & 3u, bounded & 3u, masks, scaled, large, kb0, kop,
+      prefill_half<QT, D, NT>(L, buf, 0, (use & 3u) | slow, bounded & 3u, masks, kb0, kop,
                               [&]() __attribute__((always_inline)) {
                                 load_k_operands<D>(L, buf, 1, lane, kop);
                               },
                               qop, back, lo, hi, lane, vmix, half2_t{vf[0], vf[1]}, acc, m, l,
                               bad_score);
-      prefill_half<QT, D, NT>(L, buf, 1, use >> 2, bounded >> 2, masks, scaled, large,
-                              kb0 + 32, kop, []() {}, qop, back, lo, hi, lane, vmix,
-                              half2_t{vf[2], vf[3]}, acc, m, l, bad_score);
+      prefill_half<QT, D, NT>(L, buf, 1, use >> 2 | slow, bounded >> 2, masks, kb0 + 32, kop,
+                              []() {}, qop, back, lo, hi, lane, vmix, half2_t{vf[2], vf[3]}, acc,
+                              m, l, bad_score);
     }
     if (i + 1 < nsteps) {
       // the other buffer was last read in step i - 1, before the barrier that ended it
