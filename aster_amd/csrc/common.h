@@ -182,14 +182,14 @@ __device__ __forceinline__ int8_t quant_code(float x, float scale) {
 }
 
 // x / scale clamped to the format's range, with the code of the correctly rounded quotient,
-// from inv = 1 / scale (correctly rounded): the product's residual, exact in one fma, corrects
-// it (Markstein's division step). The product is within 1.5 steps of the quotient, so that the
-// corrected one is rounded from within 2.5 * 2^-24 of a step of it: it can differ from the
-// division only where the quotient lies that near a rounding boundary, and a code only where
-// this is a boundary beside a tie of two codes. All float32 pairs there (up to scaling by
-// powers of two) give the division's result, and so do all f16 rows, a tenth of whose
-// quotients are exact or near ties (both tests enumerate them). scale >= kMinFastScale keeps
-// the residual of every quotient that can round to a code above the denormals.
+// from inv = 1 / scale (correctly rounded): the product's residual, in one fma, corrects it
+// (Markstein's division step). The product is within 1.5 steps of the quotient, its residual
+// and inv within 2^-24 of themselves, so that the corrected one is rounded from within 3 2^-24
+// of a step: it can differ from the division only where the quotient lies that near a rounding
+// boundary, and its code only where this boundary is beside a tie of two codes. All float32
+// pairs there (up to scaling by powers of two) give the division's result, and so does every
+// pair of f16 significands (the tests list them). scale >= kMinFastScale keeps the residual of
+// every quotient that can round to a code above the denormals.
 constexpr float kMinFastScale = 0x1p-64f;
 template <int KF>
 __device__ __forceinline__ float quant_unit(float x, float scale, float inv) {

@@ -1,20 +1,21 @@
 """Quotients where the append's corrected product could miss the division's code.
 
 With inv = RN(1 / b), q = RN(x inv), r = RN(x - q b), the corrected q' = RN(q + r inv) rounds
-a value within 2.5 * 2^-24 steps of x / b, so that it can differ from RN(x / b) only where x / b
-lies that near a rounding boundary of float32. Its code can then differ only where the boundary
-is the one above or below a tie t 2^e of two codes (t odd). With 24-bit integers X 2^j = B M + d,
-M the boundary as an integer of 25 bits, that is |d| <= 5: for every t, side and d the pairs
-(X, B) follow from B = -d / M mod 2^j."""
+a value within 3 * 2^-24 steps of x / b (q is within 1.5 steps; inv and r within 2^-24 of
+themselves), so that it can differ from RN(x / b) only where x / b lies that near a rounding
+boundary of float32. Its code can then differ only where the boundary is the one above or below
+a tie t 2^e of two codes (t odd). With 24-bit integers X 2^j = B M + d, M the boundary in half
+steps (25 bits), that is |d| <= 6: for every t, side and d the pairs (X, B) follow from
+B = -d / M mod 2^j."""
 
 from fractions import Fraction
 
 import numpy as np
 
 
-def dangerous_pairs(odd, reach=6):
-    """(t, x, b) as floats, x / b within ``reach`` steps of 2^-24 of the boundary beside a tie
-    with significand t, for the odd numbers ``odd``; x and b in [1, 2)."""
+def dangerous_pairs(odd, reach=8):
+    """(t, x, b) as floats, x / b within ``reach`` (|d|) of the boundary beside a tie with
+    significand t, for the odd numbers ``odd``; x and b in [1, 2)."""
     out = []
     for t in odd:
         for side in (-1, 1):
